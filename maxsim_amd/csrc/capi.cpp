@@ -436,8 +436,8 @@ void select_quantized(msim_int4_docs* h, int64_t batch, int64_t query_tokens, fl
   }
   score_quantized(h, batch, query_tokens, d_scores, stream);
   if (k > 0)
-    check_hip(launch_topk(d_scores, batch, h->num_docs, h->num_docs, k, nullptr, d_top_s, d_top_i, stream),
-              "launch int8q topk selection kernel");
+    run_topk(h->ws, d_scores, batch, h->num_docs, k, nullptr, d_top_s, d_top_i, stream,
+             "launch int8q topk selection kernel");
 }
 
 void run_int8q(msim_int4_docs* h, const float* d_query, int64_t batch, int64_t query_tokens,

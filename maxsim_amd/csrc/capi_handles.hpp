@@ -21,13 +21,14 @@ struct ScoreWorkspace {
   DeviceBuffer cand_ids, cand_info, cand_tiles;
   // cascade: coarse scores, top-M candidates (scores / ids), fine scores
   DeviceBuffer coarse, top_m_scores, top_m_ids, fine;
+  DeviceBuffer topk_scratch;  // chunk candidates of the top-k of long rows
   // Synchronous calls: the fp32 query and the top-k results, in pinned host
   // memory that the kernels read and write directly.
   HostBuffer host_query, host_out;
   uint64_t bytes() const {
     return qpack.cap + qpack_alt.cap + colmul.cap + qsum.cap + weights.cap + pooled.cap + qbits.cap + full_info.cap +
            full_tiles.cap + cand_ids.cap + cand_info.cap + cand_tiles.cap + coarse.cap + top_m_scores.cap +
-           top_m_ids.cap + fine.cap;
+           top_m_ids.cap + fine.cap + topk_scratch.cap;
   }
 };
 
@@ -87,6 +88,10 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& host_offs
                        const DocStreams& s, const QueryInput& q, int reducer, float temperature,
                        int64_t batch, int64_t query_tokens, const float* h_row_weights, const Targets& t,
                        float* d_out, int64_t out_stride, int32_t* d_iout, hipStream_t stream);
+
+// launch_topk with the workspace's scratch memory.
+void run_topk(ScoreWorkspace& ws, const float* d_scores, int64_t batch, int64_t n, int64_t k, const int64_t* d_id_map,
+              float* d_out_scores, int64_t* d_out_ids, hipStream_t stream, const char* what);
 
 }  // namespace msim
 

@@ -41,6 +41,15 @@ T* upload_vec(DeviceBuffer& buf, const std::vector<T>& v, const char* what, hipS
 
 }  // namespace
 
+void run_topk(ScoreWorkspace& ws, const float* d_scores, int64_t batch, int64_t n, int64_t k, const int64_t* d_id_map,
+              float* d_out_scores, int64_t* d_out_ids, hipStream_t stream, const char* what) {
+  const size_t bytes = topk_scratch_bytes(batch, n, k);
+  if (bytes) ws.topk_scratch.ensure(bytes, "hipMalloc top-k scratch");
+  check_hip(launch_topk(d_scores, batch, n, n, k, d_id_map, d_out_scores, d_out_ids, stream,
+                        bytes ? ws.topk_scratch.ptr : nullptr),
+            what);
+}
+
 CandidateLayout candidate_layout(int64_t batch, int64_t query_tokens, int limbs, int64_t per_target,
                                  int64_t max_doc_tiles, int chunks) {
   const int64_t rpp = score_rows_per_pass(limbs, query_tokens, chunks);
@@ -440,8 +449,7 @@ extern "C" int msim_int4_topk_batch(msim_int4_docs* h, const float* query, int64
     select_device(h->device);
     float* d = int4_score_device(h, query, batch, query_tokens, dim, kRedMax, {}, 1.0f, nullptr, 0, false, nullptr);
     const HostTopk out(h->ws, batch, k);
-    check_hip(launch_topk(d, batch, h->num_docs, h->num_docs, k, nullptr, out.s, out.i, nullptr),
-              "launch topk selection kernel");
+    run_topk(h->ws, d, batch, h->num_docs, k, nullptr, out.s, out.i, nullptr, "launch topk selection kernel");
     out.finish(out_scores, out_indices, nullptr);
   });
 }
@@ -516,8 +524,7 @@ float* binary_score_device(msim_binary_docs* h, const float* query, int64_t batc
 void copy_topk_out(msim_binary_docs* h, const float* d_scores, int64_t batch, int64_t k, float* out_scores,
                    int64_t* out_indices, hipStream_t stream) {
   const HostTopk out(h->ws, batch, k);
-  check_hip(launch_topk(d_scores, batch, h->num_docs, h->num_docs, k, nullptr, out.s, out.i, stream),
-            "launch topk selection kernel");
+  run_topk(h->ws, d_scores, batch, h->num_docs, k, nullptr, out.s, out.i, stream, "launch topk selection kernel");
   out.finish(out_scores, out_indices, stream);
 }
 
@@ -783,9 +790,8 @@ extern "C" int msim_binary_topk_hamming_async(msim_binary_docs* h, const uint8_t
     select_device(h->device);
     h->scores.ensure(sizeof(float) * batch * h->num_docs, "hipMalloc score cache");
     hamming_device(h, d_qbits, batch, query_tokens, h->scores.as<float>(), nullptr, as_stream(stream));
-    check_hip(launch_topk(h->scores.as<float>(), batch, h->num_docs, h->num_docs, k, nullptr, d_scores, d_indices,
-                          as_stream(stream)),
-              "launch topk selection kernel");
+    run_topk(h->ws, h->scores.as<float>(), batch, h->num_docs, k, nullptr, d_scores, d_indices, as_stream(stream),
+             "launch topk selection kernel");
   });
 }
 
@@ -837,15 +843,14 @@ void cascade_device(ScoreWorkspace& ws, int64_t batch, int64_t num_docs, int64_t
     tables_ready = tables;
   } else {
     ws.top_m_scores.ensure(sizeof(float) * batch * m, "hipMalloc cascade candidate scores");
-    check_hip(launch_topk(ws.coarse.as<float>(), batch, num_docs, num_docs, m, nullptr, ws.top_m_scores.as<float>(),
-                          ws.top_m_ids.as<int64_t>(), stream),
-              "launch cascade candidate selection");
+    run_topk(ws, ws.coarse.as<float>(), batch, num_docs, m, nullptr, ws.top_m_scores.as<float>(),
+             ws.top_m_ids.as<int64_t>(), stream, "launch cascade candidate selection");
     check_hip(launch_sort_rows(ws.top_m_ids.as<int64_t>(), batch, m, stream), "launch candidate sort");
   }
   ws.fine.ensure(sizeof(float) * batch * m, "hipMalloc cascade fine scores");
   fine(ws.top_m_ids.as<int64_t>(), ws.fine.as<float>(), tables_ready);
-  check_hip(launch_topk(ws.fine.as<float>(), batch, m, m, k, ws.top_m_ids.as<int64_t>(), d_top_s, d_top_i, stream),
-            "launch cascade final selection");
+  run_topk(ws, ws.fine.as<float>(), batch, m, k, ws.top_m_ids.as<int64_t>(), d_top_s, d_top_i, stream,
+           "launch cascade final selection");
 }
 
 }  // namespace
@@ -879,9 +884,8 @@ extern "C" int msim_int4_cascade_topk(msim_int4_docs* h, const float* query, int
       h->scores.ensure(sizeof(float) * batch * h->num_docs, "hipMalloc score cache");
       run_generic_score(h->ws, h->host_offsets, h->num_tokens, fused, qi, red, (float)temperature, batch,
                         query_tokens, wp, Targets{}, h->scores.as<float>(), h->num_docs, nullptr, nullptr);
-      check_hip(launch_topk(h->scores.as<float>(), batch, h->num_docs, h->num_docs, k, nullptr, out.s, out.i,
-                            nullptr),
-                "launch topk selection kernel");
+      run_topk(h->ws, h->scores.as<float>(), batch, h->num_docs, k, nullptr, out.s, out.i, nullptr,
+               "launch topk selection kernel");
     } else {
       cascade_device(
           h->ws, batch, h->num_docs, k, candidates,
@@ -1003,9 +1007,8 @@ void binres_cascade(msim_binary_docs* h, const float* d_query, int64_t batch, in
     h->scores.ensure(sizeof(float) * batch * h->num_docs, "hipMalloc score cache");
     run_generic_score(h->ws, h->host_offsets, h->num_tokens, fused, qi, kRedMax, 1.0f, batch, query_tokens, nullptr,
                       Targets{}, h->scores.as<float>(), h->num_docs, nullptr, stream);
-    check_hip(launch_topk(h->scores.as<float>(), batch, h->num_docs, h->num_docs, k, nullptr, d_top_s, d_top_i,
-                          stream),
-              "launch topk selection kernel");
+    run_topk(h->ws, h->scores.as<float>(), batch, h->num_docs, k, nullptr, d_top_s, d_top_i, stream,
+             "launch topk selection kernel");
     return;
   }
   // With the int8 query, one quantisation serves both passes: the prefix
@@ -1137,8 +1140,8 @@ extern "C" int msim_binary_binres_topk(msim_binary_docs* h, const float* query, 
     run_generic_score(h->ws, h->host_offsets, h->num_tokens, s, qi, kRedMax, 1.0f, batch, query_tokens, nullptr,
                       Targets{}, h->scores.as<float>(), h->num_docs, nullptr, nullptr);
     const HostTopk out(h->ws, batch, k);
-    check_hip(launch_topk(h->scores.as<float>(), batch, h->num_docs, h->num_docs, k, nullptr, out.s, out.i, nullptr),
-              "launch topk selection kernel");
+    run_topk(h->ws, h->scores.as<float>(), batch, h->num_docs, k, nullptr, out.s, out.i, nullptr,
+             "launch topk selection kernel");
     out.finish(out_scores, out_indices, nullptr);
   });
 }
@@ -1221,8 +1224,7 @@ extern "C" int msim_int4_topk_score(msim_int4_docs* h, const float* query, int64
     float* d = int4_score_device(h, query, batch, query_tokens, dim, red, w, (float)temperature, nullptr, 0,
                                  residual != 0, nullptr);
     const HostTopk out(h->ws, batch, k);
-    check_hip(launch_topk(d, batch, h->num_docs, h->num_docs, k, nullptr, out.s, out.i, nullptr),
-              "launch topk selection kernel");
+    run_topk(h->ws, d, batch, h->num_docs, k, nullptr, out.s, out.i, nullptr, "launch topk selection kernel");
     out.finish(out_scores, out_indices, nullptr);
   });
 }

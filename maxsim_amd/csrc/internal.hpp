@@ -302,10 +302,13 @@ hipError_t launch_select_topm(const float* d_scores, int64_t batch, int64_t n, i
 
 // Block top-k (topk.hip): per row b of scores[b * row_stride + i], i < n, the k
 // largest by (score desc, position asc).  id_map (nullable, [batch, n]) maps a
-// position to the reported id.
+// position to the reported id.  `scratch` (nullable, 8-byte aligned): device
+// memory of topk_scratch_bytes, with which rows longer than a workgroup's
+// registers are selected chunk by chunk.
 constexpr int kTopkMaxK = 4096;
+size_t topk_scratch_bytes(int64_t batch, int64_t n, int64_t k);
 hipError_t launch_topk(const float* d_scores, int64_t batch, int64_t n, int64_t row_stride,
                        int64_t k, const int64_t* d_id_map, float* d_out_scores,
-                       int64_t* d_out_ids, hipStream_t stream);
+                       int64_t* d_out_ids, hipStream_t stream, void* scratch = nullptr);
 
 }  // namespace msim

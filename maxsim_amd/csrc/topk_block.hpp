@@ -1,5 +1,5 @@
-// topk_block.hpp -- top-k of one score row by a workgroup or by one wave,
-// shared by the stand-alone top-k kernel and the fused search kernels' tail.
+// topk_block.hpp -- top-k of one score row by a workgroup (radix form), shared
+// by the stand-alone top-k kernels, and the fused search kernels' tail.
 //
 // Order restated from the reference: score descending, then position
 // ascending (cu:1629-1692 selection order; _api.py:732-735 lexsort).
@@ -303,110 +303,6 @@ __device__ void block_topk(const float* __restrict__ row, int64_t n, int k,
   __syncthreads();
   rank_and_write<kCoherent>(sm.key, sm.pos, k, tid, THREADS, row, n, id_map, out_scores, out_ids);
   __syncthreads();
-}
-
-// ----------------------------------------------------------------- wave form
-// One wave selects the top-k of a row of n <= 64 * EPT scores.  Survivors go
-// to skey/spos (k entries, wave-private LDS).  1 <= k <= n.
-template <int EPT>
-__device__ void wave_topk(const float* __restrict__ row, int64_t n, int k,
-                          const int64_t* __restrict__ id_map, float* __restrict__ out_scores,
-                          int64_t* __restrict__ out_ids, uint32_t* hist, uint32_t* skey,
-                          int32_t* spos) {
-  const int lane = lane_id();
-  const int64_t per = (n + kWave - 1) / kWave;
-  const int64_t lo = min((int64_t)lane * per, n);
-  const int cnt = (int)(min(lo + per, n) - lo);
-  uint32_t keys[EPT];
-  uint32_t kmin = 0xFFFFFFFFu, kmax = 0u;
-#pragma unroll
-  for (int e = 0; e < EPT; ++e) {
-    keys[e] = e < cnt ? score_key(load_score<false>(row + lo + e)) : 0u;
-    if (e < cnt) {
-      kmin = min(kmin, keys[e]);
-      kmax = max(kmax, keys[e]);
-    }
-  }
-  kmin = wave_min_u32(kmin);
-  kmax = wave_max_u32(kmax);
-  const int shift0 = first_shift(kmin, kmax);
-  uint32_t mask = shift0 < 0 ? 0xFFFFFFFFu : (shift0 + 8 >= 32 ? 0u : ~((2u << (shift0 + 7)) - 1u));
-  uint32_t prefix = kmax & mask;
-  uint32_t kk = (uint32_t)k;
-  for (int shift = shift0; shift >= 0;) {
-    for (int i = lane; i < 256; i += kWave) hist[i] = 0;
-    wave_sync_lds();
-#pragma unroll
-    for (int e = 0; e < EPT; ++e)
-      if (e < cnt && (keys[e] & mask) == prefix) atomicAdd(&hist[(keys[e] >> shift) & 255u], 1u);
-    wave_sync_lds();
-    uint32_t c[4];
-    uint32_t local = 0;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      c[x] = hist[255 - 4 * lane - x];
-      local += c[x];
-    }
-    const uint32_t incl = wave_inclusive_scan(local);
-    uint32_t above = incl - local;
-    uint32_t found = 0, d = 0, r = 0;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      if (above < kk && kk <= above + c[x]) {
-        found = 1;
-        d = (uint32_t)(255 - 4 * lane - x);
-        r = kk - above;
-      }
-      above += c[x];
-    }
-    // Exactly one lane holds the digit: broadcast it.
-    const unsigned long long who = __ballot(found);
-    const int src = who ? __ffsll(who) - 1 : 0;
-    prefix |= (uint32_t)__shfl((int)d, src) << shift;
-    mask |= 255u << shift;
-    kk = (uint32_t)__shfl((int)r, src);
-    wave_sync_lds();
-    if (shift == 0) break;
-    shift = shift > 8 ? shift - 8 : 0;
-  }
-
-  // Survivors: keys above the threshold, then the first kk ties by position.
-  uint32_t my_ties = 0;
-#pragma unroll
-  for (int e = 0; e < EPT; ++e) my_ties += (e < cnt && keys[e] == prefix) ? 1u : 0u;
-  const uint32_t tie_base = wave_inclusive_scan(my_ties) - my_ties;
-  uint32_t tr = tie_base, mine = 0;
-#pragma unroll
-  for (int e = 0; e < EPT; ++e) {
-    if (e < cnt) {
-      if (keys[e] > prefix) {
-        ++mine;
-      } else if (keys[e] == prefix) {
-        if (tr < kk) ++mine;
-        ++tr;
-      }
-    }
-  }
-  uint32_t slot = wave_inclusive_scan(mine) - mine;
-  tr = tie_base;
-#pragma unroll
-  for (int e = 0; e < EPT; ++e) {
-    if (e < cnt) {
-      bool keep = keys[e] > prefix;
-      if (keys[e] == prefix) {
-        keep = tr < kk;
-        ++tr;
-      }
-      if (keep && slot < (uint32_t)k) {
-        skey[slot] = keys[e];
-        spos[slot] = (int32_t)(lo + e);
-        ++slot;
-      }
-    }
-  }
-  wave_sync_lds();
-  rank_and_write<false>(skey, spos, k, lane, kWave, row, n, id_map, out_scores, out_ids);
-  wave_sync_lds();
 }
 
 // ----------------------------------------------------------------- tail form
