@@ -55,14 +55,14 @@ MFMA_FP4_PEAK_TOPS = 10100.0  # MI355X dense fp4 MFMA
 MIX_NS_PER_MFMA = 11.43
 RAMP_US = 2.1
 TAIL_US = 4.8
-# Config 3's MaxSim score launch, the same way: its loop issues 24 MFMAs per
-# 16-token tile and pass (three limbs, four row blocks) with about five other
-# VALU instructions each (profiles/score_kernel_config3_sq_counters.md: 4.95),
-# a mix the rate tests put between mfma_fma4 (12.79 ns per MFMA) and
-# mfma_fma6 (15.61 ns): 14.2 ns.  The first tile lands at 2.0 us (median
-# wave, per-wave stamps) and the last wave ends its loop about 1 us before
-# the launch ends.
-MIX3_NS_PER_MFMA = 14.2
+# Config 3's MaxSim score launch: its loop issues 20 fp6 MFMAs
+# (v_mfma_scale_f32_16x16x128_f8f6f4) per 16-token tile and pass (five digits,
+# four row blocks) with about two other VALU instructions each, which a rate
+# test of that mix on random operands puts at 12.3 ns per MFMA and SIMD (11.2 ns
+# without the VALU).  Ramp and tail: the first tile's latency and the last
+# waves' end, about 2 us and 1 us.
+MIX3_NS_PER_MFMA = 12.3
+MFMA_FP6_PEAK_TOPS = 10066.0  # 1024 SIMDs x 2 x 16 x 16 x 128 per 16 cycles at 2.4 GHz
 RAMP3_US = 2.0
 TAIL3_US = 1.0
 
@@ -641,10 +641,10 @@ def bench_config3(args):
         e1.record(stream)
         torch.cuda.synchronize()
         kernel_ms = e0.elapsed_time(e1) / (SCAN_BLOCK * 4)
-        int8_ops = 3 * 2.0 * b * q * t * 128
+        digit_ops = 5 * 2.0 * b * q * t * 128
         per[red] = {"ms_per_step": wall, "p50_ms": float(np.percentile(ev, 50)), "docs_per_s": b * n / (wall * 1e-3),
                     "score_kernel_ms": kernel_ms,
-                    "mfma_frac": int8_ops / (kernel_ms * 1e-3) / 1e12 / MFMA_INT8_PEAK_TOPS}
+                    "mfma_frac": digit_ops / (kernel_ms * 1e-3) / 1e12 / MFMA_FP6_PEAK_TOPS}
     # weighted MaxSim with new weights every step (two arrays alternating, so
     # the handle's unchanged-weights check never skips the upload)
     other = np.ascontiguousarray(weights[::-1])
@@ -663,21 +663,21 @@ def bench_config3(args):
                      "on the stream each step)"}
     ms = float(np.mean([v["ms_per_step"] for v in per.values()]))
     ops = 2.0 * b * q * t * 128  # multiply-adds x 2 of the fp32 contraction
-    roof = {"kernel": "score_kernel (3 int8 limbs)", "bound": "mfma", "unit": "TOP/s",
-            "achieved": 3 * ops / (ms * 1e-3) / 1e12, "peak": MFMA_INT8_PEAK_TOPS,
+    roof = {"kernel": "digit_score_kernel (5 fp6 digits)", "bound": "mfma", "unit": "TOP/s",
+            "achieved": 5 * ops / (ms * 1e-3) / 1e12, "peak": MFMA_FP6_PEAK_TOPS,
             "fp32_equivalent_TFLOPs": ops / (ms * 1e-3) / 1e12, "fp32_vector_peak_TFLOPs": FP32_PEAK_TFLOPS,
-            "note": "step time (scan + top-10); int8 ops = 3 limbs x 2 B Q T 128"}
+            "note": "step time (scan + top-10); fp6 ops = 5 digits x 2 B Q T 128"}
     roof["frac"] = roof["achieved"] / roof["peak"]
     # The MaxSim launch's issue bound (see MIX3_NS_PER_MFMA): two 64-row passes
     # over every tile, spread over the chip's SIMDs.
     simds = torch.cuda.get_device_properties(0).multi_processor_count * 4
     passes = (b * q + 63) // 64
     tiles_per_simd = passes * scan_tiles(packed.doc_offsets) / simds
-    bound_us = RAMP3_US + tiles_per_simd * 24 * MIX3_NS_PER_MFMA * 1e-3 + TAIL3_US
+    bound_us = RAMP3_US + tiles_per_simd * 20 * MIX3_NS_PER_MFMA * 1e-3 + TAIL3_US
     roof["maxsim_achievable_bound"] = {
-        "kernel_us": bound_us, "frac": 3 * ops / (bound_us * 1e-6) / 1e12 / MFMA_INT8_PEAK_TOPS,
+        "kernel_us": bound_us, "frac": 5 * ops / (bound_us * 1e-6) / 1e12 / MFMA_FP6_PEAK_TOPS,
         "tiles_per_simd": tiles_per_simd,
-        "basis": "ramp %.1f us + tiles per SIMD x 24 MFMAs x %.1f ns (an MFMA and about five VALU instructions, "
+        "basis": "ramp %.1f us + tiles per SIMD x 20 MFMAs x %.1f ns (an MFMA and about two VALU instructions, "
                  "two waves per SIMD, rate tests) + tail %.1f us; against the MaxSim launch's measured "
                  "score_kernel_ms" % (RAMP3_US, MIX3_NS_PER_MFMA, TAIL3_US)}
     cpu = None

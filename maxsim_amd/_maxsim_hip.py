@@ -431,8 +431,8 @@ class CudaInt4PackedDocs:
 class CudaPackedDocs:
     """Resident sign-bit corpus (reference: CudaPackedDocs, cu:1872-2675).
 
-    Every scoring method runs the MFMA kernels of score.hip: fp32 queries are
-    split into three int8 limbs, int8 queries (``*_int8q``) use one, and
+    Every scoring method runs MFMA kernels: fp32 queries as five base-32 digits
+    (digit_kernel.hpp), int8 queries (``*_int8q``) as one limb (score.hip), and
     sign-bit queries (``hamming_batch`` / ``topk_hamming``) are exact +-1
     dot products, i.e. dim - 2 popcount(q ^ d)."""
 
@@ -627,7 +627,7 @@ class CudaPackedDocs:
 
     def set_rescore_limbs(self, limbs):
         """Query limbs of fused scoring and cascade rescoring: 1 = int8 query,
-        3 = fp32 query (three int8 limbs)."""
+        3 = fp32 query."""
         check(self._lib.msim_binary_set_rescore_limbs(self._h, int(limbs)))
 
     def get_rescore_limbs(self) -> int:

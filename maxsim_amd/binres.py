@@ -13,7 +13,7 @@ residual, cascade.py:60-93); this module defines it:
 
 Queries are quantised to int8 per row (sigma = max|q| / 127, as the int4
 int8-query path); the fused scores (and a cascade's rescoring) can instead
-take the fp32 query as three int8 limbs (query_precision="fp32").  Coarse
+take the fp32 query (query_precision="fp32").  Coarse
 similarity a_t (q . sign_t); fused similarity a_t (q . sign_t) +
 s^r_t (q . v^r_t), i.e. q . x'_t with x'_t = a_t sign_t + s^r_t v^r_t the
 reconstructed token; both reduced with MaxSim.  The cascade takes the
@@ -126,7 +126,7 @@ def binres_score(query_tokens, packed: BinaryResidualPackedDocs, *, fused: bool 
     """Coarse (fused=False) or fused scores; candidate_indices None or i64 [B, M].
 
     query_precision: the query of the fused scores, "int8" (one int8 limb) or
-    "fp32" (three int8 limbs); the coarse scores always use the int8 query."""
+    "fp32" (the whole query); the coarse scores always use the int8 query."""
     q, squeeze = _query(query_tokens, packed.dim)
     resident = binres_to_device(packed)
     cand = None if candidate_indices is None else np.asarray(candidate_indices, dtype=np.int64)

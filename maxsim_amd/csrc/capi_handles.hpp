@@ -15,7 +15,7 @@ struct ScoreWorkspace {
   DeviceBuffer qpack_alt;  // the query also in the int4 layout (QueryInput::alt_int4)
   std::vector<float> weights_host;  // what `weights` holds (a repeated weight vector is not copied again)
   DeviceBuffer full_info, full_tiles;  // cached whole-corpus tables
-  int64_t full_key = -1;               // wave count the cached tables were built for (units: -2 - workgroups)
+  int64_t full_key = -1;               // waves the cached tables were built for (work units: -2 - workgroups)
   int64_t full_waves = 0;              // records in the cached table
   int64_t full_units = 0;              // records per workgroup (work-unit tables), else 0
   DeviceBuffer cand_ids, cand_info, cand_tiles;
@@ -24,7 +24,7 @@ struct ScoreWorkspace {
   DeviceBuffer topk_scratch;  // chunk candidates of the top-k of long rows
   // Synchronous calls: the fp32 query and the top-k results, in pinned host
   // memory that the kernels read and write directly.
-  HostBuffer host_query, host_out;
+  HostBuffer host_query, host_out, host_ids;
   uint64_t bytes() const {
     return qpack.cap + qpack_alt.cap + colmul.cap + qsum.cap + weights.cap + pooled.cap + qbits.cap + full_info.cap +
            full_tiles.cap + cand_ids.cap + cand_info.cap + cand_tiles.cap + coarse.cap + top_m_scores.cap +
@@ -36,14 +36,15 @@ struct ScoreWorkspace {
 struct QueryInput {
   const float* d_query = nullptr;    // fp32 [rows, 128 chunks] (device or pinned host memory), or
   const uint8_t* d_qbits = nullptr;  // sign bits [rows, 16] (pack_signs order)
-  int limbs = 3;                     // 3: fp32 split into int8 limbs, 1: int8
+  int limbs = 3;                     // 3: the fp32 query (as digits), 1: int8
   bool recip = false;                // int8 rounding q * (1 / sigma) (binary int8q)
   bool quantized = false;            // the workspace already holds this query in this layout
   bool alt_int4 = false;             // also quantise into qpack_alt in the int4 layout
   bool from_alt = false;             // score the rows an earlier alt_int4 call left in qpack_alt
 };
 
-// The document streams and scales of one scoring call.
+// The document streams and scales of one scoring call (int4 codes as fp6 rows
+// where the query is fp32).
 struct DocStreams {
   int doc = kDocInt4;
   bool residual = false;
@@ -60,13 +61,15 @@ struct DocStreams {
 };
 
 // Candidate targets: none (every document), one list shared by all batch
-// rows, or one list of `count` per batch row.
+// rows, or one list of `count` per batch row.  Lists in host memory are staged
+// by the (synchronous) call.
 struct Targets {
   const int64_t* host = nullptr;
   int64_t count = 0;
   bool per_row = false;
-  // Candidate lists already on the device ([batch][count], per_row): tables
-  // are written on the device; documents have at most max_doc_tiles tiles.
+  // Candidate lists already on the device ([batch][count], per_row); tables,
+  // where needed, are written on the device: documents have at most
+  // max_doc_tiles tiles.
   const int64_t* device = nullptr;
   const int64_t* d_offsets = nullptr;
   int64_t max_doc_tiles = 1;
@@ -80,7 +83,10 @@ struct CandidateLayout {
   int64_t waves = 0, per_wave = 0, cap = 0;
 };
 CandidateLayout candidate_layout(int64_t batch, int64_t query_tokens, int limbs, int64_t per_target,
-                                 int64_t max_doc_tiles, int chunks = 1);
+                                 int64_t max_doc_tiles);
+
+// Bytes of the fp32 query's digits (launch_quantize_digits).
+size_t digit_bytes(int64_t rows_padded, int chunks);
 
 // Scores of `batch` x `query_tokens` query rows against the targets into
 // d_out[b * out_stride + t] (and d_iout[b * targets + t] as int32 if set).
@@ -117,10 +123,10 @@ struct msim_int4_docs {
   int64_t block_pos_off = 0;      // index of the workgroup start positions in wave_info
   msim::DeviceBuffer wave_info, tile_table;
   msim::DeviceBuffer packed, offsets, token_scales, token_scales16, residual_packed, residual_token_scales16;
-  // Generalized path: codes widened to whole 128-dim chunks (64 bytes each)
-  // when dim is not a multiple of 128, per-token 1/16 when the corpus has no
-  // token scales.
-  msim::DeviceBuffer codes_wide, residual_wide, ones16;
+  // fp32 queries: the codes as fp6 rows (96 bytes per token and 128-dim
+  // chunk), made on the device at the first such call, and per-token 1/16 when
+  // the corpus has no token scales.
+  msim::DeviceBuffer codes6, residual6, ones16;
   // workspaces (grow monotonically, freed with the handle; cu:3057-3067)
   msim::DeviceBuffer qpack, qscale, qbias, scores, rowmax;
   msim::HostBuffer host_io;  // synchronous calls: query in, results out (pinned)
@@ -131,7 +137,7 @@ struct msim_int4_docs {
 
   uint64_t resident_bytes() const {
     return packed_size + offsets_size * 8 + token_scales.cap + token_scales16.cap + residual_packed.cap +
-           residual_token_scales16.cap + codes_wide.cap + residual_wide.cap + ones16.cap;
+           residual_token_scales16.cap + codes6.cap + residual6.cap + ones16.cap;
   }
   uint64_t workspace_bytes() const {
     return qpack.cap + qscale.cap + qbias.cap + scores.cap +
@@ -155,8 +161,9 @@ struct msim_binary_docs {
   double residual_scale = 1.0;
   int64_t max_doc_tiles = 1;  // 16-token tiles of the longest document
   msim::DeviceBuffer residual_packed, residual_token_scales16;
-  // Query limbs of the fused (prefix + residual) scoring and of a cascade's
-  // rescoring pass: 1 = the int8 query, 3 = the fp32 query (three int8 limbs).
+  msim::DeviceBuffer residual6;  // the residual codes as fp6 rows (fp32 rescoring)
+  // Query of the fused (prefix + residual) scoring and of a cascade's
+  // rescoring pass: 1 = the int8 query, 3 = the fp32 query.
   int rescore_limbs = 1;
   // The int8-query scan over the sign stream (a cascade's prefix pass): its
   // tables (cached by wave count) and whether every token scale suits its
@@ -169,7 +176,7 @@ struct msim_binary_docs {
 
   uint64_t resident_bytes() const {
     return packed.cap + offsets.cap + scale_vector.cap + token_scales.cap + ones.cap + residual_packed.cap +
-           residual_token_scales16.cap;
+           residual_token_scales16.cap + residual6.cap;
   }
   uint64_t workspace_bytes() const {
     return scores.cap + iscores.cap + scale_override.cap + scan_wave_info.cap +

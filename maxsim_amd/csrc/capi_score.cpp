@@ -51,17 +51,142 @@ void run_topk(ScoreWorkspace& ws, const float* d_scores, int64_t batch, int64_t 
 }
 
 CandidateLayout candidate_layout(int64_t batch, int64_t query_tokens, int limbs, int64_t per_target,
-                                 int64_t max_doc_tiles, int chunks) {
-  const int64_t rpp = score_rows_per_pass(limbs, query_tokens, chunks);
+                                 int64_t max_doc_tiles) {
+  CandidateLayout cl;
+  if (limbs == 3) {  // one candidate per wave, no tables
+    cl.per_wave = 1;
+    cl.waves = per_target;
+    cl.cap = 0;
+    return cl;
+  }
+  const int64_t rpp = score_rows_per_pass(query_tokens);
   const int64_t subs = ceil_div(query_tokens, rpp);
   int64_t waves = ceil_div((int64_t)device_cu_count() * 8, batch * subs);
   waves = std::max<int64_t>(1, std::min(waves, per_target));
-  CandidateLayout cl;
   cl.per_wave = ceil_div(per_target, waves);
   cl.waves = ceil_div(ceil_div(per_target, cl.per_wave), 4) * 4;
   cl.cap = cl.per_wave * std::max<int64_t>(1, max_doc_tiles) + 1;
   return cl;
 }
+
+namespace {
+
+// Candidate lists of a synchronous call in the workspace's pinned host
+// memory (the previous call has finished: the caller waits for its stream).
+const int64_t* stage_ids(ScoreWorkspace& ws, const int64_t* ids, int64_t count) {
+  ws.host_ids.ensure(sizeof(int64_t) * std::max<int64_t>(count, 1), "hipHostMalloc candidate staging");
+  std::memcpy(ws.host_ids.ptr, ids, sizeof(int64_t) * (size_t)count);
+  return ws.host_ids.as<int64_t>();
+}
+
+// Reducer weights, one per query row (padding rows 0), on the device.
+const float* row_weights_device(ScoreWorkspace& ws, const float* h_row_weights, int64_t rows, int64_t rows_padded,
+                                hipStream_t stream) {
+  if (h_row_weights == nullptr) return nullptr;
+  std::vector<float> w((size_t)rows_padded, 0.0f);
+  std::memcpy(w.data(), h_row_weights, sizeof(float) * rows);
+  if (ws.weights.ptr == nullptr || w.size() != ws.weights_host.size() ||
+      std::memcmp(w.data(), ws.weights_host.data(), sizeof(float) * w.size()) != 0) {
+    upload_vec(ws.weights, w, "copy reducer query weights to device", stream);
+    ws.weights_host = std::move(w);
+  }
+  return ws.weights.as<float>();
+}
+
+void set_streams(ScoreArgs& a, const DocStreams& s) {
+  a.codes = s.codes;
+  a.tscale = s.tscale;
+  a.tmul = s.tmul;
+  a.rcodes = s.rcodes;
+  a.rtscale = s.rtscale;
+  a.rmul = s.rmul;
+  a.doc_scale = s.doc_scale;
+  a.scale = s.scale;
+  a.unit_tscale = s.unit_tscale;
+}
+
+// fp32 queries: digits, then one launch over every document (work units) or
+// over candidate documents (one per wave).
+void run_digit_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, const DocStreams& s, const QueryInput& q,
+                     int reducer, float temperature, int64_t batch, int64_t query_tokens, const float* h_row_weights,
+                     const Targets& t, float* d_out, int64_t out_stride, hipStream_t stream) {
+  const int64_t num_docs = (int64_t)off.size() - 1;
+  const int64_t targets = (t.host || t.device) ? t.count : num_docs;
+  const int64_t rows = batch * query_tokens, rows_padded = ceil_div(rows, 16) * 16 + 128;
+  const int64_t groups = t.per_row ? batch : 1;
+  const DigitPlan plan = digit_plan(t.per_row ? 1 : batch, query_tokens, s.chunks);
+
+  ws.qpack.ensure(digit_bytes(rows_padded, s.chunks), "hipMalloc query digits");
+  ws.colmul.ensure(sizeof(float) * rows_padded, "hipMalloc query scales");
+  const int64_t ids = t.host ? groups * t.count : 0;
+  const int64_t* staged = nullptr;
+  if (t.host) {
+    staged = stage_ids(ws, t.host, ids);
+    ws.cand_ids.ensure(sizeof(int64_t) * std::max<int64_t>(ids, 1), "hipMalloc candidates");
+  }
+  if (!q.quantized)
+    check_hip(launch_quantize_digits(q.d_query, rows, rows_padded, ws.qpack.as<uint8_t>(), ws.colmul.as<float>(),
+                                     s.chunks, staged, ws.cand_ids.as<int64_t>(), ids, stream),
+              "launch query digit kernel");
+
+  ScoreArgs a{};
+  set_streams(a, s);
+  a.weights = row_weights_device(ws, h_row_weights, rows, rows_padded, stream);
+  if (t.host || t.device || num_docs >= kScoreMaxUnitTargets) {
+    // (Tile entries hold 24 bits of target index: more documents go one per
+    // wave.)
+    if (t.d_offsets == nullptr) throw InvalidArgument("candidate lists need the token offsets");
+    a.targets = t.device ? t.device : t.host ? ws.cand_ids.as<int64_t>() : nullptr;
+    a.targets_grp_stride = t.per_row ? t.count : 0;
+    a.direct_offsets = t.d_offsets;
+    a.direct_count = targets;
+  } else {
+    // A list of work units per CU and pass; few documents are spread over as
+    // many CUs.
+    const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(device_cu_count() / plan.subs, num_docs));
+    if (ws.full_key != -2 - wgs) {
+      std::vector<int64_t> info;
+      std::vector<uint64_t> tiles;
+      ws.full_units = build_score_units(off.data(), nullptr, num_docs, wgs, info, tiles,
+                                        s.doc == kDocSign ? kDigitUnitSign : kDigitUnitInt4);
+      upload_vec(ws.full_info, info, "copy score wave table to device");
+      upload_vec(ws.full_tiles, tiles, "copy score tile table to device");
+      ws.full_key = -2 - wgs;
+      ws.full_waves = (int64_t)info.size() / kScoreInfoWords;
+    }
+    a.wave_info = ws.full_info.as<int64_t>();
+    a.tiles = ws.full_tiles.as<uint64_t>();
+    a.num_waves = ws.full_waves;
+    a.group_units = (int32_t)ws.full_units;
+  }
+  a.qpack = ws.qpack.as<int8_t>();
+  a.rows_padded = rows_padded;
+  a.colmul = ws.colmul.as<float>();
+  a.subs = (int32_t)plan.subs;
+  a.pass_rows = (int32_t)plan.pass_rows;
+  a.grp_rows = (int32_t)(t.per_row ? query_tokens : rows);
+  a.temperature = temperature;
+  a.query_tokens = (int32_t)query_tokens;
+  a.chunks = s.chunks;
+  if (plan.whole) {  // the kernel sums each batch row's tokens
+    a.out = d_out;
+    a.out_stride = out_stride;
+    check_hip(launch_digit_score(a, s.doc, s.residual, plan.nt, reducer, groups, stream), "launch score kernel");
+    return;
+  }
+  ws.pooled.ensure(sizeof(float) * std::max<int64_t>(1, groups * targets * a.grp_rows), "hipMalloc pooled rows");
+  a.pooled = ws.pooled.as<float>();
+  a.pooled_grp_stride = targets * a.grp_rows;
+  check_hip(launch_digit_score(a, s.doc, s.residual, plan.nt, reducer, groups, stream), "launch score kernel");
+  check_hip(launch_pool_sum(ws.pooled.as<float>(), batch, query_tokens, targets,
+                            t.per_row ? targets * query_tokens : query_tokens, t.per_row ? query_tokens : rows, d_out,
+                            out_stride, nullptr, stream),
+            "launch pooled sum kernel");
+}
+
+}  // namespace
+
+size_t digit_bytes(int64_t rows_padded, int chunks) { return (size_t)(kScoreDigits * rows_padded * 96 * chunks); }
 
 void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int64_t num_tokens,
                        const DocStreams& s, const QueryInput& q, int reducer, float temperature,
@@ -79,22 +204,26 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
     if (d_iout) check_hip(launch_fill_f32(reinterpret_cast<float*>(d_iout), batch * targets, 0.0f, stream), "zero scores");
     return;
   }
-  const int limbs = q.limbs;
+  if (q.limbs == 3) {
+    run_digit_score(ws, off, s, q, reducer, temperature, batch, query_tokens, h_row_weights, t, d_out, out_stride,
+                    stream);
+    return;
+  }
+  // int8 and sign-bit queries: sign documents (with or without the residual
+  // stream), MaxSim.
+  if (s.doc != kDocSign || s.chunks != 1) throw NotSupported("int8 and sign-bit queries are scored at dims up to 128");
+  if (reducer != kRedMax || h_row_weights) throw NotSupported("int8 and sign-bit queries are scored with MaxSim");
   const int64_t rows_padded = ceil_div(rows, 16) * 16 + 128;
-  const int chunks = s.chunks;
-  if (chunks != 1 && (limbs != 3 || q.d_qbits || q.alt_int4 || q.from_alt || (s.doc == kDocSign && s.residual)))
-    throw NotSupported("dims above 128 are scored for fp32 queries against int4 or sign documents only");
 
   // Sign-bit queries against sign documents over every document, MaxSim on
   // unit token scales: the fp4 Hamming kernel reads the query bits itself.
-  const bool fp4 = g_hamming_fp4 != 0 && q.d_qbits && s.doc == kDocSign && !s.residual && reducer == kRedMax &&
-                   s.unit_tscale && chunks == 1 && !t.host && !t.device && h_row_weights == nullptr;
+  const bool fp4 = g_hamming_fp4 != 0 && q.d_qbits && !s.residual && s.unit_tscale && !t.host && !t.device;
 
   // 1. Quantise the query rows.
-  ws.qpack.ensure((size_t)limbs * rows_padded * 128 * chunks, "hipMalloc query limbs");
+  ws.qpack.ensure((size_t)rows_padded * 128, "hipMalloc query codes");
   ws.colmul.ensure(sizeof(float) * rows_padded, "hipMalloc query scales");
-  ws.qsum.ensure(sizeof(int32_t) * limbs * rows_padded, "hipMalloc query limb sums");
-  if (q.alt_int4) ws.qpack_alt.ensure((size_t)limbs * rows_padded * 128, "hipMalloc query limbs (int4 layout)");
+  ws.qsum.ensure(sizeof(int32_t) * rows_padded, "hipMalloc query code sums");
+  if (q.alt_int4) ws.qpack_alt.ensure((size_t)rows_padded * 128, "hipMalloc query codes (int4 layout)");
   if (q.quantized || q.from_alt || fp4) {
     // reuse the workspace's quantised rows (the fp4 kernel reads the bits)
   } else if (q.d_qbits)
@@ -104,29 +233,15 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
   else
     // A sign stream paired with an int4 residual is unpacked in the int4
     // lane order, so both share the int4 query layout.
-    check_hip(launch_quantize_limbs(q.d_query, rows, rows_padded, limbs, s.residual ? kDocInt4 : s.doc, q.recip,
+    check_hip(launch_quantize_limbs(q.d_query, rows, rows_padded, s.residual ? kDocInt4 : s.doc, q.recip,
                                     ws.qpack.as<int8_t>(), ws.colmul.as<float>(), ws.qsum.as<int32_t>(), stream,
-                                    kDocInt4, q.alt_int4 ? ws.qpack_alt.as<int8_t>() : nullptr, chunks),
+                                    kDocInt4, q.alt_int4 ? ws.qpack_alt.as<int8_t>() : nullptr),
               "launch query quantize kernel");
 
-  // 2. Reducer weights, one per query row (padding rows 0).
-  const float* d_weights = nullptr;
-  if (h_row_weights) {
-    std::vector<float> w((size_t)rows_padded, 0.0f);
-    std::memcpy(w.data(), h_row_weights, sizeof(float) * rows);
-    if (ws.weights.ptr != nullptr && w.size() == ws.weights_host.size() &&
-        std::memcmp(w.data(), ws.weights_host.data(), sizeof(float) * w.size()) == 0) {
-      d_weights = ws.weights.as<float>();
-    } else {
-      d_weights = upload_vec(ws.weights, w, "copy reducer query weights to device", stream);
-      ws.weights_host = std::move(w);
-    }
-  }
-
-  // 3. Work split.
+  // 2. Work split.
   const int64_t groups = t.per_row ? batch : 1;
   const int64_t grp_rows = t.per_row ? query_tokens : rows;
-  const int64_t rpp = fp4 ? kHammingRowsPerPass : score_rows_per_pass(limbs, grp_rows, chunks);
+  const int64_t rpp = fp4 ? kHammingRowsPerPass : score_rows_per_pass(grp_rows);
   const int64_t subs = ceil_div(grp_rows, rpp);
   const int64_t per_target = t.per_row ? t.count : targets;
   int64_t waves = ceil_div((int64_t)device_cu_count() * 8, groups * subs);
@@ -134,18 +249,26 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
 
   ScoreArgs a{};
   const int64_t* d_targets = nullptr;
-  if (t.device) {
-    // Candidate lists on the device: fixed-size target ranges per wave; with
-    // more than one per wave, tables written by candidate_tables_kernel (or
-    // already by the selector).
-    if (!t.per_row) throw InvalidArgument("device candidate lists must be per batch row");
-    const CandidateLayout cl = candidate_layout(batch, query_tokens, limbs, per_target, t.max_doc_tiles, chunks);
+  if (t.host || t.device) {
+    // Candidate lists: fixed-size target ranges per wave; with more than one
+    // per wave, tables written by candidate_tables_kernel (or already by the
+    // selector).
+    if (!t.per_row) throw InvalidArgument("candidate lists must be per batch row");
+    if (t.d_offsets == nullptr) throw InvalidArgument("candidate lists need the token offsets");
+    const CandidateLayout cl = candidate_layout(batch, query_tokens, q.limbs, per_target, t.max_doc_tiles);
     const int64_t w4 = cl.waves;
     d_targets = t.device;
+    if (t.host) {
+      const int64_t count = groups * t.count;
+      ws.cand_ids.ensure(sizeof(int64_t) * count, "hipMalloc candidates");
+      check_hip(hipMemcpyAsync(ws.cand_ids.ptr, stage_ids(ws, t.host, count), sizeof(int64_t) * (size_t)count,
+                               hipMemcpyHostToDevice, stream),
+                "copy candidates to device");
+      d_targets = ws.cand_ids.as<int64_t>();
+    }
     if (cl.per_wave == 1) {
       // One candidate per wave: the kernel takes its tiles from the
       // document's token range (no tables).
-      if (t.d_offsets == nullptr) throw InvalidArgument("device candidate lists need the token offsets");
       a.direct_offsets = t.d_offsets;
       a.direct_count = per_target;
       a.num_waves = w4;
@@ -153,7 +276,7 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
       ws.cand_info.ensure(sizeof(int64_t) * groups * w4 * kScoreInfoWords, "hipMalloc candidate wave table");
       ws.cand_tiles.ensure(sizeof(uint64_t) * groups * w4 * cl.cap, "hipMalloc candidate tile table");
       if (!t.tables_ready)
-        check_hip(launch_candidate_tables(t.device, per_target, groups, t.d_offsets, w4, cl.per_wave, cl.cap,
+        check_hip(launch_candidate_tables(d_targets, per_target, groups, t.d_offsets, w4, cl.per_wave, cl.cap,
                                           ws.cand_info.as<int64_t>(), ws.cand_tiles.as<uint64_t>(), stream),
                   "launch candidate table kernel");
       a.wave_info = ws.cand_info.as<int64_t>();
@@ -161,104 +284,56 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
       a.num_waves = w4;
       a.info_grp_stride = w4 * kScoreInfoWords;
     }
-  } else if (!t.host) {
-    // The row-block pipeline kernels (three limbs, four 16-row blocks per
-    // pass, one 128-dim chunk, no residual) take work units: a list per
-    // workgroup of eight waves, about `waves` waves in all.
-    const bool unit_tables = !fp4 && limbs == 3 && rpp == 64 && chunks == 1 && !s.rcodes &&
-                             num_docs < kScoreMaxUnitTargets;
-    const int64_t key = unit_tables ? -2 - ceil_div(waves, 8) : waves;
-    if (ws.full_key != key) {
+  } else {
+    if (ws.full_key != waves) {
       std::vector<int64_t> info;
       std::vector<uint64_t> tiles;
+      build_score_tables(off.data(), nullptr, num_docs, waves, info, tiles);
+      upload_vec(ws.full_info, info, "copy score wave table to device");
+      upload_vec(ws.full_tiles, tiles, "copy score tile table to device");
+      ws.full_key = waves;
       ws.full_units = 0;
-      if (unit_tables)
-        ws.full_units = build_score_units(off.data(), nullptr, num_docs, ceil_div(waves, 8), info, tiles);
-      else
-        build_score_tables(off.data(), nullptr, num_docs, waves, info, tiles);
-      upload_vec(ws.full_info, info, "copy score wave table to device", stream);
-      upload_vec(ws.full_tiles, tiles, "copy score tile table to device", stream);
-      ws.full_key = key;
       ws.full_waves = (int64_t)info.size() / kScoreInfoWords;
     }
     a.wave_info = ws.full_info.as<int64_t>();
     a.tiles = ws.full_tiles.as<uint64_t>();
     a.num_waves = ws.full_waves;
-    a.group_units = (int32_t)ws.full_units;
     a.info_grp_stride = 0;
-  } else {
-    // Per group: its own table, all padded to the same wave count.
-    std::vector<std::vector<int64_t>> infos((size_t)groups);
-    std::vector<uint64_t> tiles;
-    int64_t max_waves = 0;
-    for (int64_t gi = 0; gi < groups; ++gi) {
-      std::vector<uint64_t> gt;
-      build_score_tables(off.data(), t.host + gi * (t.per_row ? t.count : 0), per_target, waves, infos[gi], gt);
-      for (size_t w = 0; w < infos[gi].size(); w += kScoreInfoWords) infos[gi][w + 3] += (int64_t)tiles.size();
-      tiles.insert(tiles.end(), gt.begin(), gt.end());
-      max_waves = std::max<int64_t>(max_waves, (int64_t)infos[gi].size() / kScoreInfoWords);
-    }
-    std::vector<int64_t> info;
-    for (int64_t gi = 0; gi < groups; ++gi) {
-      auto& gi_info = infos[gi];
-      while ((int64_t)gi_info.size() / kScoreInfoWords < max_waves) {
-        const int64_t pad[kScoreInfoWords] = {per_target, 0, 0, 0};
-        gi_info.insert(gi_info.end(), pad, pad + kScoreInfoWords);
-      }
-      info.insert(info.end(), gi_info.begin(), gi_info.end());
-    }
-    a.wave_info = upload_vec(ws.cand_info, info, "copy candidate wave table to device", stream);
-    a.tiles = upload_vec(ws.cand_tiles, tiles, "copy candidate tile table to device", stream);
-    a.num_waves = max_waves;
-    a.info_grp_stride = max_waves * kScoreInfoWords;
-    std::vector<int64_t> ids(t.host, t.host + groups * per_target);
-    d_targets = upload_vec(ws.cand_ids, ids, "copy candidates to device", stream);
   }
 
-  // 4. Score; the batch-row sums over query tokens are taken in the kernel
+  // 3. Score; the batch-row sums over query tokens are taken in the kernel
   // or by pool_sum_kernel over pooled[target][row].
-  a.codes = s.codes;
-  a.tscale = s.tscale;
-  a.tmul = s.tmul;
-  a.rcodes = s.rcodes;
-  a.rtscale = s.rtscale;
-  a.rmul = s.rmul;
+  set_streams(a, s);
   a.targets = d_targets;
   a.targets_grp_stride = t.per_row ? t.count : 0;
   a.qpack = q.from_alt ? ws.qpack_alt.as<int8_t>() : ws.qpack.as<int8_t>();
   a.rows_padded = rows_padded;
   a.colmul = ws.colmul.as<float>();
   a.qsum = ws.qsum.as<int32_t>();
-  a.weights = d_weights;
   a.subs = (int32_t)subs;
   a.grp_rows = (int32_t)grp_rows;
-  a.doc_scale = s.doc_scale;
-  a.scale = s.scale;
   a.temperature = temperature;
-  a.unit_tscale = s.unit_tscale;
   a.query_tokens = (int32_t)query_tokens;
-  a.chunks = chunks;
+  a.chunks = 1;
   a.qbits = fp4 ? q.d_qbits : nullptr;
   // Passes that hold whole batch rows let the kernel sum them itself.
   const bool in_kernel_sum = t.per_row ? subs == 1 : rpp % query_tokens == 0;
+  auto launch = [&] {
+    if (fp4) check_hip(launch_hamming(a, stream), "launch fp4 hamming kernel");
+    else check_hip(launch_score(a, s.residual, groups, stream), "launch score kernel");
+  };
   if (in_kernel_sum) {
     a.out = d_out;
     a.out_stride = out_stride;
     a.iout = d_iout;
     a.iout_stride = per_target;
-    if (fp4)
-      check_hip(launch_hamming(a, stream), "launch fp4 hamming kernel");
-    else
-      check_hip(launch_score(a, s.doc, s.residual, limbs, reducer, groups, stream), "launch score kernel");
+    launch();
     return;
   }
   ws.pooled.ensure(sizeof(float) * std::max<int64_t>(1, groups * per_target * grp_rows), "hipMalloc pooled rows");
   a.pooled = ws.pooled.as<float>();
   a.pooled_grp_stride = per_target * grp_rows;
-  if (fp4)
-    check_hip(launch_hamming(a, stream), "launch fp4 hamming kernel");
-  else
-    check_hip(launch_score(a, s.doc, s.residual, limbs, reducer, groups, stream), "launch score kernel");
+  launch();
   const int64_t bs = t.per_row ? per_target * query_tokens : query_tokens;
   const int64_t ts = t.per_row ? query_tokens : rows;
   check_hip(launch_pool_sum(ws.pooled.as<float>(), batch, query_tokens, per_target, bs, ts, d_out, out_stride, d_iout,
@@ -376,17 +451,38 @@ void copy_scores_out(ScoreWorkspace& ws, void* out, const void* d, size_t bytes)
 
 // ------------------------------------------------------------------ int4
 
+// int4 codes as fp6 rows, made at the first fp32 query of the handle (about
+// 30 us per half million tokens) and waited for, so that a later call may come
+// on any stream.
+const uint8_t* fp6_rows(DeviceBuffer& rows, const uint8_t* codes, int64_t num_tokens, int64_t dim) {
+  if (rows.ptr == nullptr && num_tokens > 0) {
+    const int chunks = score_chunks(dim);
+    DeviceBuffer made;
+    // (and the kScanPadTokens zero rows a tile may read past the last token)
+    const int64_t words = 24 * chunks;  // floats per row
+    made.ensure((size_t)((num_tokens + kScanPadTokens) * words * 4), "hipMalloc fp6 document rows");
+    check_hip(launch_encode_fp6(codes, num_tokens, dim / 2, chunks, made.as<uint8_t>(), nullptr),
+              "launch fp6 document kernel");
+    check_hip(launch_fill_f32(made.as<float>() + num_tokens * words, kScanPadTokens * words, 0.0f, nullptr),
+              "zero fp6 document padding");
+    check_hip(hipStreamSynchronize(nullptr), "synchronize fp6 document kernel");
+    std::swap(rows.ptr, made.ptr);
+    std::swap(rows.cap, made.cap);
+  }
+  return rows.as<uint8_t>();
+}
+
 DocStreams int4_streams(msim_int4_docs* h, bool residual) {
   if (h->dim > kScoreMaxDim) throw NotSupported("fp32-query int4 scoring currently supports dim <= 512");
   if (h->num_tokens > 0 && !h->has_token_scale && h->ones16.cap < (size_t)h->num_tokens * 4) {
-    std::vector<float> ones((size_t)h->num_tokens, 0.0625f);
+    std::vector<float> ones((size_t)(h->num_tokens + kScanPadTokens), 0.0625f);
     h->ones16.ensure(ones.size() * 4, "hipMalloc int4 unit token scales");
     check_hip(hipMemcpy(h->ones16.ptr, ones.data(), ones.size() * 4, hipMemcpyHostToDevice), "copy unit token scales");
   }
   DocStreams s;
   s.doc = kDocInt4;
   s.chunks = score_chunks(h->dim);
-  s.codes = h->codes_wide.ptr ? h->codes_wide.as<uint8_t>() : h->packed.as<uint8_t>();
+  s.codes = fp6_rows(h->codes6, h->packed.as<uint8_t>(), h->num_tokens, h->dim);
   s.tscale = h->has_token_scale ? h->token_scales16.as<float>() : h->ones16.as<float>();
   s.tmul = (float)h->scale;
   s.scale = 1.0f;
@@ -394,7 +490,7 @@ DocStreams int4_streams(msim_int4_docs* h, bool residual) {
     if (!h->has_residual)
       throw InvalidArgument("residual int4 data was requested but is not loaded on this CUDA handle");
     s.residual = true;
-    s.rcodes = h->residual_wide.ptr ? h->residual_wide.as<uint8_t>() : h->residual_packed.as<uint8_t>();
+    s.rcodes = fp6_rows(h->residual6, h->residual_packed.as<uint8_t>(), h->num_tokens, h->dim);
     s.rtscale = h->residual_token_scales16.as<float>();
     s.rmul = (float)h->residual_scale;
   }
@@ -418,6 +514,7 @@ float* int4_score_device(msim_int4_docs* h, const float* query, int64_t batch, i
   qi.d_query = d_query;
   qi.limbs = 3;
   Targets t{cand, m, false};
+  t.d_offsets = h->offsets.as<int64_t>();
   run_generic_score(h->ws, h->host_offsets, h->num_tokens, s, qi, reducer, temperature, batch, query_tokens,
                     w.empty() ? nullptr : w.data(), t, h->scores.as<float>(), targets, nullptr, stream);
   return h->scores.as<float>();
@@ -489,7 +586,7 @@ DocStreams binary_streams(msim_binary_docs* h, double scale, bool use_scale_vect
   if (use_token_scale && !h->has_token_scale)
     throw InvalidArgument("token scale vector was requested but is not loaded on this CUDA handle");
   if (h->num_tokens > 0 && !(use_token_scale) && h->ones.cap < (size_t)h->num_tokens * 4) {
-    std::vector<float> ones((size_t)h->num_tokens, 1.0f);
+    std::vector<float> ones((size_t)(h->num_tokens + kScanPadTokens), 1.0f);
     h->ones.ensure(ones.size() * 4, "hipMalloc binary unit token scales");
     check_hip(hipMemcpy(h->ones.ptr, ones.data(), ones.size() * 4, hipMemcpyHostToDevice), "copy unit token scales");
   }
@@ -516,6 +613,7 @@ float* binary_score_device(msim_binary_docs* h, const float* query, int64_t batc
   qi.limbs = limbs;
   qi.recip = recip;
   Targets t{cand, m, false};
+  t.d_offsets = h->offsets.as<int64_t>();
   run_generic_score(h->ws, h->host_offsets, h->num_tokens, s, qi, reducer, temperature, batch, query_tokens,
                     w.empty() ? nullptr : w.data(), t, h->scores.as<float>(), targets, nullptr, nullptr);
   return h->scores.as<float>();
@@ -907,7 +1005,7 @@ extern "C" int msim_int4_cascade_topk(msim_int4_docs* h, const float* query, int
                               query_tokens, wp, t, d, candidates, nullptr, nullptr);
           },
           out.s, out.i, nullptr,
-          candidate_layout(batch, query_tokens, qi.limbs, candidates, h->max_doc_tiles, fused.chunks),
+          candidate_layout(batch, query_tokens, qi.limbs, candidates, h->max_doc_tiles),
           h->offsets.as<int64_t>());
     }
     out.finish(out_scores, out_indices, nullptr);
@@ -918,7 +1016,8 @@ extern "C" int msim_int4_cascade_topk(msim_int4_docs* h, const float* query, int
 
 namespace {
 
-DocStreams binres_streams(msim_binary_docs* h, bool fused) {
+// limbs 3: the residual codes as fp6 rows (the fp32 query's form).
+DocStreams binres_streams(msim_binary_docs* h, bool fused, int limbs) {
   if (h->dim != 128) throw InvalidArgument("binary residual scoring currently requires dim=128");
   if (!h->has_token_scale)
     throw InvalidArgument("binary residual scoring needs the prefix scales: call set_token_scale_vector first");
@@ -931,7 +1030,8 @@ DocStreams binres_streams(msim_binary_docs* h, bool fused) {
   s.tmul = 1.0f;
   if (fused) {
     s.residual = true;
-    s.rcodes = h->residual_packed.as<uint8_t>();
+    s.rcodes = limbs == 3 ? fp6_rows(h->residual6, h->residual_packed.as<uint8_t>(), h->num_tokens, h->dim)
+                          : h->residual_packed.as<uint8_t>();
     s.rtscale = h->residual_token_scales16.as<float>();
     s.rmul = (float)h->residual_scale;
   }
@@ -966,7 +1066,7 @@ bool binres_scan_prefix(msim_binary_docs* h, const float* d_query, int64_t batch
   ws.qpack_alt.ensure((size_t)rows_padded * 128, "hipMalloc query limbs (int4 layout)");
   ws.colmul.ensure(sizeof(float) * rows_padded, "hipMalloc query scales");
   ws.qsum.ensure(sizeof(int32_t) * rows_padded, "hipMalloc query limb sums");
-  check_hip(launch_quantize_limbs(d_query, rows, rows_padded, 1, kDocSign, false, ws.qpack.as<int8_t>(),
+  check_hip(launch_quantize_limbs(d_query, rows, rows_padded, kDocSign, false, ws.qpack.as<int8_t>(),
                                   ws.colmul.as<float>(), ws.qsum.as<int32_t>(), stream, kDocInt4,
                                   ws.qpack_alt.as<int8_t>()),
             "launch query quantize kernel");
@@ -999,7 +1099,7 @@ bool binres_scan_prefix(msim_binary_docs* h, const float* d_query, int64_t batch
 
 void binres_cascade(msim_binary_docs* h, const float* d_query, int64_t batch, int64_t query_tokens, int64_t k,
                     int64_t m, float* d_top_s, int64_t* d_top_i, hipStream_t stream) {
-  const DocStreams prefix = binres_streams(h, false), fused = binres_streams(h, true);
+  const DocStreams prefix = binres_streams(h, false, 1), fused = binres_streams(h, true, h->rescore_limbs);
   QueryInput qi;
   qi.d_query = d_query;
   qi.limbs = h->rescore_limbs;
@@ -1014,7 +1114,7 @@ void binres_cascade(msim_binary_docs* h, const float* d_query, int64_t batch, in
   // With the int8 query, one quantisation serves both passes: the prefix
   // pass's sign layout, and the int4 layout the fused pass reads (its sign
   // stream is unpacked in the int4 lane order).  With the fp32 query, the
-  // rescoring pass quantises its three limbs itself (its buffers sized first,
+  // rescoring pass quantises its digits itself (its buffers sized first,
   // so that no buffer the prefix pass reads is reallocated while in flight).
   QueryInput coarse_q = qi;
   coarse_q.limbs = 1;
@@ -1024,8 +1124,7 @@ void binres_cascade(msim_binary_docs* h, const float* d_query, int64_t batch, in
     fine_q.from_alt = true;
   } else {
     const int64_t rows_padded = ceil_div(batch * query_tokens, 16) * 16 + 128;
-    h->ws.qpack.ensure((size_t)qi.limbs * rows_padded * 128, "hipMalloc query limbs");
-    h->ws.qsum.ensure(sizeof(int32_t) * qi.limbs * rows_padded, "hipMalloc query limb sums");
+    h->ws.qpack.ensure(digit_bytes(rows_padded, 1), "hipMalloc query digits");
   }
   cascade_device(
       h->ws, batch, h->num_docs, k, m,
@@ -1064,8 +1163,10 @@ extern "C" int msim_binary_set_residual(msim_binary_docs* h, const uint8_t* pack
     select_device(h->device);
     std::vector<uint8_t> codes(packed, packed + (size_t)num_tokens * (size_t)row_bytes);
     upload_vec(h->residual_packed, codes, "copy binary residual data to device");
+    h->residual6.reset();
     std::vector<float> s16(token_scales, token_scales + count);
     for (float& v : s16) v *= 0.0625f;
+    s16.resize((size_t)(count + kScanPadTokens), 0.0f);  // rows the fp32-query scorer may read past the end
     upload_vec(h->residual_token_scales16, s16, "copy binary residual token scales to device");
     h->residual_scale = scale;
     h->has_residual = true;
@@ -1101,7 +1202,7 @@ extern "C" int msim_binary_binres_score(msim_binary_docs* h, const float* query,
   return guarded([&] {
     require_handle(h);
     check_binary_query(h, batch, query_tokens, dim);
-    const DocStreams s = binres_streams(h, fused != 0);
+    const DocStreams s = binres_streams(h, fused != 0, h->rescore_limbs);
     if (candidates) {
       if (num_candidates < 0) throw InvalidArgument("candidate_indices must have shape [batch, candidates]");
       check_candidates(candidates, batch * num_candidates, h->num_docs);
@@ -1113,6 +1214,8 @@ extern "C" int msim_binary_binres_score(msim_binary_docs* h, const float* query,
     qi.d_query = stage_query(h->ws, query, batch * query_tokens, dim);
     qi.limbs = fused ? h->rescore_limbs : 1;
     Targets t{candidates, num_candidates, candidates != nullptr};
+    t.d_offsets = h->offsets.as<int64_t>();
+    t.max_doc_tiles = h->max_doc_tiles;
     h->scores.ensure(sizeof(float) * batch * targets, "hipMalloc score cache");
     // Prefix scores of every document: the scan a cascade's prefix pass uses.
     const bool scanned = !fused && !candidates && g_scan_prefix &&
@@ -1130,7 +1233,7 @@ extern "C" int msim_binary_binres_topk(msim_binary_docs* h, const float* query, 
     require_handle(h);
     check_binary_query(h, batch, query_tokens, dim);
     check_k(k, h->num_docs);
-    const DocStreams s = binres_streams(h, true);
+    const DocStreams s = binres_streams(h, true, h->rescore_limbs);
     if (batch == 0) return;
     select_device(h->device);
     QueryInput qi;
@@ -1153,7 +1256,7 @@ extern "C" int msim_binary_cascade_topk(msim_binary_docs* h, const float* query,
     require_handle(h);
     check_binary_query(h, batch, query_tokens, dim);
     check_cascade(k, candidates, h->num_docs);
-    binres_streams(h, true);
+    binres_streams(h, true, 1);
     if (batch == 0) return;
     select_device(h->device);
     const float* d_query = stage_query(h->ws, query, batch * query_tokens, dim);
@@ -1170,7 +1273,7 @@ extern "C" int msim_binary_cascade_topk_async(msim_binary_docs* h, const float* 
     require_handle(h);
     require_shape(batch, query_tokens);
     check_cascade(k, candidates, h->num_docs);
-    binres_streams(h, true);
+    binres_streams(h, true, 1);
     if (batch == 0) return;
     select_device(h->device);
     binres_cascade(h, d_query, batch, query_tokens, k, candidates, d_scores, d_indices, as_stream(stream));

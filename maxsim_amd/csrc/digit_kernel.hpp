@@ -1,0 +1,558 @@
+// digit_kernel.hpp -- MaxSim scoring of fp32 queries on gfx950's fp6/fp4 MFMA:
+// int4 or sign-bit documents (optionally with an int4 residual stream), the
+// reference's five reducers, every document or given candidates.  Semantics:
+// score.hip's header (the same restated lines of the reference).
+//
+// Query rows as digits.  A row q is fixed-point on a power-of-two grid: with
+// colmul = 2^(E-1), max|q| <= 2^E, each q / colmul in [-2, 2] is rounded to a
+// multiple of 2^-23 and written as five balanced digits of base 32,
+//   q = colmul * sum_i d_i 2^-3 32^-i,  i = 0..4,  |d_0| <= 16, -16 <= d_i <= 15,
+// every digit exact as fp6 (e2m3 holds the integers to 16 in units of 1/8).
+// The grid keeps every bit of the row's largest elements and resolves the
+// row to 2^-25..2^-24 of max|q|.
+//
+// Documents.  int4 codes are integers up to 8, exact in e2m3 too: a handle
+// keeps a copy of its codes as fp6 rows (96 bytes per token and 128 dims,
+// encode_fp6_kernel), because unpacking nibbles to 6-bit fields in registers
+// costs about a hundred VALU instructions per tile.  Sign documents become
+// fp4 +-1 with two instructions per dword (fp4_signs).  The MFMA's E8M0 scales
+// hold the digits' weights 32^-i, so one v_mfma_scale_f32_16x16x128_f8f6f4
+// per digit and 128 dims adds all digits into one fp32 accumulator, lowest
+// digit first (measured: each MFMA's 128 products are summed exactly and
+// rounded once with the accumulator, so the smaller digits keep their bits
+// until the last steps; dots against float64: 3.1e-8 rms, a plain fp32 dot
+// 5.6e-8).  A similarity is then one fma (times the token scale, the row mask
+// as addend), or nothing for sign documents without token scales.
+//
+// Why digits rather than int8 limbs: three exact int8 limb dots need six MFMAs
+// of 64 dims per 16 x 16 block and 4.5 VALU instructions per similarity to
+// recombine (9 for sign documents); five MFMAs of 128 dims and one (or no)
+// VALU instruction do the same.  Rates measured per MFMA and SIMD, two waves,
+// random operands: i8 16x16x64 7.9 ns, fp6 x fp6 16x16x128 11.2 ns, fp4 x fp6
+// 9.5 ns.  MaxSim launches before (three limbs) and now, 32 query tokens:
+//   int4, 16,384 documents of 64..192 tokens, 4 queries   117.6 -> 93.0 us
+//   int4,  4,096 of the same, 2 queries                    20.8 -> 19.7 us
+//   signs, 10,240 documents of 256..1,024 tokens, 1 / 2    125 / 206 -> 76 / 117 us
+// (80 ns per 16 x 16 block of int4 at four blocks, 73 of signs, against 56 and 48
+// of the MFMAs alone; one int4 query is bound by memory, 6.4 TB/s of fp6 rows.)
+//
+// Work split: the eight waves (two per SIMD) of a workgroup share one pass of
+// query rows; its digits are staged once in LDS and held in registers (NT
+// blocks of 16 rows, 30 VGPRs each per 128 dims).  A wave walks 16-token tiles
+// (the MFMA's A operand), held in a ring of registers filled by buffer loads
+// (an address is a descriptor in SGPRs and a constant offset: 64-bit VGPR
+// addresses would share registers with pending loads and make the compiler wait
+// for them, 101 us where this takes 93; filling the ring in LDS by DMA took
+// 120), from work units its workgroup's waves take from a
+// counter in LDS (every document), or of one candidate document per wave.
+// Step j of a tile issues row block j's MFMAs; the epilogue of the block one
+// step back (the previous tile's last block for j = 0) is spread between them
+// from the third MFMA on, so that its accumulators are at least two further
+// MFMAs (32 cycles) old: no MFMA-result fence, and the matrix core and the
+// VALU work at once.
+#pragma once
+
+#include "common.hpp"
+#include "internal.hpp"
+#include "score_reduce.hpp"
+
+namespace msim {
+namespace digit {
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+typedef int v8i __attribute__((ext_vector_type(8)));
+
+constexpr int kDigits = kScoreDigits;
+// Waves per workgroup: two per SIMD, one where four chunks of two streams
+// take more than half of a SIMD's registers.
+constexpr int group_waves(bool res, int kc) { return res && kc == 4 ? 4 : 8; }
+constexpr int kFormatFp6 = 2, kFormatFp4 = 4;  // cbsz / blgp: e2m3, e2m1
+
+// E8M0 scale bytes: 2^-5i of digit i, and of the document operand (int4 codes
+// are held as code / 8: 2^3).
+constexpr int kDigitScales = 127 | (122 << 8) | (117 << 16) | (112 << 24);
+constexpr int kDigitScale4 = 107;
+
+// Six dwords of a lane: 16 bytes at 16 g of a 96-byte row, 8 at 64 + 8 g.
+struct Six {
+  int w[6];
+};
+__device__ __forceinline__ Six load_six(const void* row, uint32_t byte_lo, uint32_t byte_hi) {
+  const v4i lo = *reinterpret_cast<const v4i*>(static_cast<const char*>(row) + byte_lo);
+  const v2i hi = *reinterpret_cast<const v2i*>(static_cast<const char*>(row) + byte_hi);
+  return {{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1]}};
+}
+__device__ __forceinline__ Six load_six(__amdgpu_buffer_rsrc_t r, int byte_lo, int byte_hi) {
+  const v4u lo = load_b128(r, byte_lo);
+  const uint64_t hi = load_b64(r, byte_hi);
+  return {{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3], (int)(uint32_t)hi, (int)(uint32_t)(hi >> 32)}};
+}
+__device__ __forceinline__ v8i operand(const Six& x) {
+  return (v8i){x.w[0], x.w[1], x.w[2], x.w[3], x.w[4], x.w[5], 0, 0};
+}
+__device__ __forceinline__ v8i operand(const v4i& x) { return (v8i){x[0], x[1], x[2], x[3], 0, 0, 0, 0}; }
+
+// acc + documents (A) x digit D of the query (B).
+template <int DOC, int D>
+__device__ __forceinline__ v4f mfma_digit(const v8i& a, const v8i& b, const v4f& c, int sa, int s03, int s4) {
+  constexpr int kA = DOC == kDocInt4 ? kFormatFp6 : kFormatFp4;
+  if constexpr (D < 4) return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, kA, kFormatFp6, 0, sa, D, s03);
+  else return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b, c, kA, kFormatFp6, 0, sa, 0, s4);
+}
+
+// Tiles held per wave (one computed, the rest in flight): what the registers
+// left by the query digits take.  Signs are small (256 bytes per tile), so
+// only many of them in flight cover the memory latency.
+constexpr int ring_size(int doc, bool res, int nt, int kc, bool unit) {
+  if (doc == kDocSign && !res && kc == 1) return unit ? 8 : nt == 4 ? 4 : 8;
+  if (res) return nt * kc >= 4 ? 2 : 4;
+  return kc == 1 ? 4 : nt * kc >= 4 ? 2 : 4;
+}
+
+// State of row block a in lanes 0 .. 31 and of b in lanes 32 .. 63, each merged
+// over the wave's two halves (row 0 / 1 or 2 / 3 of 16 lanes for swap16).
+template <int RED, typename Swap>
+__device__ __forceinline__ ReducerState<RED> swap_merge(const ReducerState<RED>& a, const ReducerState<RED>& b, Swap swap) {
+  ReducerState<RED> x = a, y = b;
+  auto sw = [&](float& u, float& v) __attribute__((always_inline)) {
+    const auto r = swap(__float_as_uint(u), __float_as_uint(v));
+    u = __uint_as_float(r[0]);
+    v = __uint_as_float(r[1]);
+  };
+  if constexpr (RED == kRedMax) {
+    sw(x.m, y.m);
+    x.m = fmaxf(x.m, y.m);
+  } else if constexpr (RED == kRedLse) {
+    sw(x.m, y.m);
+    sw(x.s, y.s);
+    x.merge(y.m, y.s);
+  } else {
+    constexpr int K = RED == kRedTop2 ? 2 : 4;
+#pragma unroll
+    for (int i = 0; i < K; ++i) sw(x.t[i], y.t[i]);
+#pragma unroll
+    for (int i = 0; i < K; ++i) x.insert(y.t[i]);
+  }
+  return x;
+}
+
+// UNIT: sign documents without token scales, MaxSim: the similarity is the
+// accumulator itself.  DIRECT: one target per wave, its document's token range
+// from p.direct_offsets; else work units.
+template <int DOC, bool RES, int NT, int RED, int KC, bool UNIT, bool DIRECT>
+__global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) / 4) void digit_score_kernel(
+    ScoreArgs p) {
+  constexpr int kWavesPerGroup = group_waves(RES, KC), kThreads = kWavesPerGroup * kWave;
+  static_assert(!UNIT || (DOC == kDocSign && !RES && RED == kRedMax), "accumulators as similarities");
+  static_assert(!(DOC == kDocSign && RES) || KC == 1, "sign prefix + residual: 128 dims");
+  constexpr int kRing = ring_size(DOC, RES, NT, KC, UNIT);
+  static_assert(kRing < (DOC == kDocSign ? kDigitUnitSign : kDigitUnitInt4), "work units cover the tiles loaded ahead");
+  static_assert(kRing % 2 == 0, "accumulator sets alternate over an even ring");
+  constexpr int kSets = NT == 1 ? 2 : NT;  // accumulators of a step and of the step before it
+  constexpr int kCodeBytes = (DOC == kDocInt4 ? 96 : 16) * KC, kResBytes = 96 * KC, kRowBytes = 96 * KC;
+  constexpr float kStart = UNIT ? kNegInf : 0.0f;  // accumulators before the first tile
+  constexpr int kChain = kDigits * KC, kSteps = RES ? 2 * kChain : kChain;  // MFMAs of a step
+
+  // The pass's query digits: [row][digit][96 KC], rows 16 j + c.
+  constexpr int kVecs = kDigits * 16 * NT * kRowBytes / 16;
+  __shared__ __attribute__((aligned(16))) v4i s_q[kVecs];
+  __shared__ float s_pool[kWavesPerGroup][16 * NT];
+  __shared__ int s_next;
+  const int lane = lane_id();
+  const int wave = wave_uniform(threadIdx.x / kWave);
+  const int g = lane >> 4, c = lane & 15;
+  const int grp = (int)blockIdx.y / p.subs, sub = (int)blockIdx.y % p.subs;
+  const int lr0 = sub * p.pass_rows;                      // first local row of the pass
+  const int64_t grow0 = (int64_t)grp * p.grp_rows + lr0;  // its global query row
+
+  // The tile stream.  Work units: a wave starts with units `wave` and wave + 8
+  // of its workgroup's list and takes the following ones from a counter; unit
+  // A holds the current tile, unit B the next one, taken as A starts.  Every
+  // unit but a list's last has more than kRing tiles, so the tiles loaded ahead
+  // (and the entry after them) lie in A or B; past the list's end they are the
+  // table's padding entry (token 0).  The two waves of a SIMD do not share it
+  // evenly (the older wave issues first); taking units as they go, both finish
+  // with the workgroup's list.
+  using TilePtr = const __attribute__((address_space(4))) uint64_t*;
+  const int64_t gw = (int64_t)wave * gridDim.x + blockIdx.x;  // DIRECT: the target
+  int64_t ds = 0, doc0 = 0;
+  int ntok = 0, na = 0, nb = 0;
+  const TilePtr pad = as_constant(p.tiles);
+  TilePtr ta = pad, tb = pad;
+  const auto unit_info = as_constant(p.wave_info) + (int64_t)blockIdx.x * p.group_units * kScoreInfoWords;
+  auto unit = [&](int k, TilePtr& tp, int& n) __attribute__((always_inline)) {
+    n = 0;
+    if (k < p.group_units) {
+      const auto rec = unit_info + (int64_t)k * kScoreInfoWords;
+      n = (int)rec[2];
+      tp = pad + rec[3];
+    }
+  };
+  if constexpr (DIRECT) {
+    if (gw < p.direct_count) {
+      doc0 = p.targets ? as_constant(p.targets)[grp * p.targets_grp_stride + gw] : gw;
+      ds = as_constant(p.direct_offsets)[doc0];
+      ntok = (int)(as_constant(p.direct_offsets)[doc0 + 1] - ds);
+      na = ntok == 0 ? 1 : (ntok + 15) / 16;  // an empty document: one tile, not scored
+    }
+  } else {
+    unit(wave, ta, na);
+    unit(wave + kWavesPerGroup, tb, nb);
+  }
+  // Entry of the tile at position q of unit A (and on into B).
+  auto entry = [&](int q) __attribute__((always_inline)) -> uint64_t {
+    if constexpr (DIRECT) {
+      const int left = ntok - 16 * q;
+      const bool in = left > 0;
+      return score_tile_entry(in ? ds + 16 * (int64_t)q : 0, in ? min(16, left) : 1, q + 1 == na, ntok == 0, 0);
+    } else {
+      return *(q < na ? ta + q : q - na < nb ? tb + (q - na) : pad);
+    }
+  };
+
+  // The query digits: global loads first, the first tiles behind them, then
+  // to LDS.
+  constexpr int kStage = (kVecs + kThreads - 1) / kThreads;
+  v4i stage[kStage];
+#pragma unroll
+  for (int x = 0; x < kStage; ++x)
+    stage[x] = reinterpret_cast<const v4i*>(p.qpack + grow0 * (kDigits * kRowBytes))[min((int)threadIdx.x + x * kThreads, kVecs - 1)];
+  // At a target's end lane group g holds row block (g >> 1) + 2 (g & 1).
+  const int blk = (g >> 1) | ((g & 1) << 1);
+  const int64_t my_row = grow0 + 16 * min(blk, NT - 1) + c;
+  const float colmul_row = p.colmul[my_row], weight = p.weights ? p.weights[my_row] : 1.0f;
+  float lse_mul[RED == kRedLse ? NT : 1];
+  if constexpr (RED == kRedLse) {
+#pragma unroll
+    for (int j = 0; j < NT; ++j) lse_mul[j] = p.colmul[grow0 + 16 * j + c];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  struct Tile {
+    uint64_t e;
+    Six code[DOC == kDocInt4 ? KC : 1];
+    unsigned sign[DOC == kDocSign ? KC : 1];
+    Six res[RES ? KC : 1];
+    float s[UNIT ? 1 : 4], sr[RES ? 4 : 1];
+  };
+  // A tile's loads: one buffer per stream at the tile's first token, the lane's
+  // part a constant offset.  Rows past a short document are the next tokens
+  // (or the kScanPadTokens zero tokens after the last one), masked below.
+  const int va = DOC == kDocInt4 ? c * kCodeBytes + 16 * g : c * kCodeBytes + 4 * g;
+  const int vr = c * kResBytes + 16 * g, vs = 16 * g;
+  auto load = [&](uint64_t e, Tile& t) __attribute__((always_inline)) {
+    t.e = e;
+    const int64_t start = (int64_t)(e & kTileStartMask);
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.codes + start * kCodeBytes, 16 * kCodeBytes);
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc) {
+      if constexpr (DOC == kDocInt4) t.code[kc] = load_six(ra, va + 96 * kc, va + 96 * kc + 64 - 8 * g);
+      else t.sign[kc] = load_b32(ra, va + 16 * kc);
+    }
+    if constexpr (RES) {
+      const __amdgpu_buffer_rsrc_t rr = make_rsrc(p.rcodes + start * kResBytes, 16 * kResBytes);
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) t.res[kc] = load_six(rr, vr + 96 * kc, vr + 96 * kc + 64 - 8 * g);
+    }
+    if constexpr (!UNIT) {
+      const v4u sv = load_b128(make_rsrc(p.tscale + start, 64u), vs);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) t.s[k] = __uint_as_float(sv[k]);
+      if constexpr (RES) {
+        const v4u rv = load_b128(make_rsrc(p.rtscale + start, 64u), vs);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) t.sr[k] = __uint_as_float(rv[k]);
+      }
+    }
+  };
+  Tile ring[kRing];
+#pragma unroll
+  for (int u = 0; u < kRing - 1; ++u) load(entry(u), ring[u]);
+  uint64_t next = entry(kRing - 1);  // the entry of the tile loaded next
+  int q = 0;                         // position (in A) of the current tile
+  __builtin_amdgcn_sched_barrier(0);
+
+  if (threadIdx.x == 0) s_next = 2 * kWavesPerGroup;
+#pragma unroll
+  for (int x = 0; x < kStage; ++x) s_q[min((int)threadIdx.x + x * kThreads, kVecs - 1)] = stage[x];
+  __syncthreads();
+  if (na == 0) return;  // no barriers below
+  Six bq[NT][kDigits][KC];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+#pragma unroll
+    for (int d = 0; d < kDigits; ++d)
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc)
+        bq[j][d][kc] = load_six(reinterpret_cast<const char*>(s_q) + ((16 * j + c) * kDigits + d) * kRowBytes + 96 * kc,
+                                16u * g, 64u + 8u * g);
+  }
+  // Factors of a similarity before (int4 token scales are stored / 16) and
+  // after the reduction; one stream takes its constant factor after it.
+  const float mul = DOC == kDocInt4 ? 16.0f * p.tmul : p.tmul;
+  const float after_mul = RES ? 1.0f : mul;
+  const float colmul = colmul_row * after_mul;
+  const float k2 = kLog2e / p.temperature;
+  int sa = DOC == kDocInt4 ? 130 : 127, sr = 130, s03 = kDigitScales, s4 = kDigitScale4;
+  asm volatile("" : "+v"(sa), "+v"(sr), "+v"(s03), "+v"(s4));  // kept in VGPRs
+  const auto doc_scale = p.doc_scale ? as_constant(p.doc_scale) : nullptr;
+
+  ReducerState<RED> st[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) st[j].init();
+  v4f acc[kSets], accr[RES ? kSets : 1];
+  int len = 0;  // tokens of the current target so far
+  auto rows_of = [](uint64_t e) -> int { return (int)((e >> kTileRowsShift) & 15) + 1; };
+  auto target_of = [&](uint64_t e) -> int64_t { return DIRECT ? gw : (int64_t)(e >> kTileLocalShift); };
+  auto scale_of = [&](int64_t target) -> float { return doc_scale ? doc_scale[DIRECT ? doc0 : target] : p.scale; };
+  auto begin_target = [&](uint64_t e) __attribute__((always_inline)) {
+    if constexpr (RED == kRedLse) {
+      const float f = scale_of(target_of(e)) * k2;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) st[j].k = lse_mul[j] * after_mul * f;
+    }
+  };
+  const int pass_rows = min(p.pass_rows, p.grp_rows - lr0);
+  const bool sum_regs = NT > 1 && p.out && p.query_tokens == 32;
+  // End of the target whose last tile is e.
+  auto finish_target = [&](uint64_t e) __attribute__((always_inline)) {
+    const int64_t tg = target_of(e);
+    auto sw32 = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_permlane32_swap(a, b, false, false); };
+    auto sw16 = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_permlane16_swap(a, b, false, false); };
+    ReducerState<RED> none;
+    none.init();
+    const ReducerState<RED> x = swap_merge<RED>(st[0], NT > 1 ? st[NT > 1 ? 1 : 0] : none, sw32);
+    const ReducerState<RED> y = NT > 2 ? swap_merge<RED>(st[NT > 2 ? 2 : 0], st[NT > 3 ? 3 : 0], sw32) : none;
+    const ReducerState<RED> all = swap_merge<RED>(x, y, sw16);
+    const bool empty = ((e >> kTileEmptyShift) & 1) != 0;
+    const float v = all.finish(empty ? 0 : len, colmul, p.temperature, weight, scale_of(tg));
+#pragma unroll
+    for (int j = 0; j < NT; ++j) st[j].init();
+    len = 0;
+    const int64_t b0 = grow0 / p.query_tokens;
+    if (sum_regs) {
+      // 32-token queries: a batch row's token l and l + 16 are 32 lanes apart
+      // (lane groups g and g + 2), summed in token_sum16's order.
+      float w = v, o = 0.0f;
+      const auto r = sw32(__float_as_uint(w), __float_as_uint(o));  // upper half of w over the lower of o
+      w = row_butterfly16(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+      if (c == 0 && 32 * g < pass_rows && g < NT / 2) p.out[(b0 + g) * p.out_stride + tg] = w;
+    } else if (p.out) {
+      // Whole batch rows in this pass: their query tokens summed here.
+      if (blk < NT) s_pool[wave][16 * blk + c] = v;
+      wave_sync_lds();
+      sum_batch_rows(s_pool[wave], pass_rows / p.query_tokens, p.query_tokens,
+                     [&](int b, float s) { p.out[(b0 + b) * p.out_stride + tg] = s; });
+      wave_sync_lds();
+    } else {
+      float* out = p.pooled + grp * p.pooled_grp_stride + tg * p.grp_rows + lr0;
+      if (blk < NT && 16 * blk + c < pass_rows) out[16 * blk + c] = v;
+    }
+  };
+
+  // What the epilogue of a tile needs once its ring slot is reused.  mask: -inf
+  // for rows past the tile's, else -0 (x + -0 = x for every x), which joins
+  // the similarity's fma.
+  struct Pend {
+    float s[UNIT ? 1 : 4], sr[RES ? 4 : 1], mask[UNIT ? 1 : 4];
+    uint64_t e;
+  };
+  // Row k of an accumulator set as similarities, and a row block's four into
+  // its reducer.
+  auto zval = [&](const Pend& P, const v4f& x, const v4f& y, int k) __attribute__((always_inline)) -> float {
+    if constexpr (UNIT) return x[k];
+    const float z = fmaf(x[k], P.s[k], P.mask[k]);
+    if constexpr (RES) return fmaf(y[k], P.sr[k], z);
+    return z;
+  };
+  auto fold = [&](const Pend& P, float (&z)[4], int j) __attribute__((always_inline)) {
+    if constexpr (UNIT) {
+      const int rows = rows_of(P.e);
+      if (rows < 16) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) z[k] = 4 * g + k >= rows ? kNegInf : z[k];
+      }
+    }
+    st[j].add4(z, k2);
+  };
+  // One step: the MFMAs of row block j of tile t into accumulator set `set`.
+  // Between them, from the third MFMA on, the epilogue of the step before
+  // (tile P, its block jp and set), and what extra(m) puts after MFMA m.
+  auto step = [&](const Tile& t, int j, int set, const Pend& P, int jp, int setp, auto extra)
+                  __attribute__((always_inline)) {
+    constexpr int kWait = 2, kSpan = kSteps - kWait;  // >= 3 slots
+    const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    float z[4];
+    int m = 0;
+    auto after = [&](int m) __attribute__((always_inline)) {
+      extra(m);
+      if (m >= kWait) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (kWait + k * kSpan / 4 == m) z[k] = zval(P, acc[setp], accr[RES ? setp : 0], k);
+        if (m == kSteps - 1) fold(P, z, jp);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    v8i a[KC];
+#pragma unroll
+    for (int kc = 0; kc < KC; ++kc) {
+      if constexpr (DOC == kDocInt4) a[kc] = operand(t.code[kc]);
+      else a[kc] = operand(fp4_signs(t.sign[kc]));
+    }
+    auto digits = [&](auto digit_c, v4f& dst, const v8i (&ops)[KC], auto doc_c, int scale)
+                      __attribute__((always_inline)) {
+      constexpr int d = decltype(digit_c)::value;
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) {
+        const v4f& from = d == kDigits - 1 && kc == 0 ? zero : dst;
+        dst = mfma_digit<decltype(doc_c)::value, d>(ops[kc], operand(bq[j][d][kc]), from, scale, s03, s4);
+        after(m++);
+      }
+    };
+    auto chain = [&](v4f& dst, const v8i (&ops)[KC], auto doc_c, int scale) __attribute__((always_inline)) {
+      digits(std::integral_constant<int, 4>{}, dst, ops, doc_c, scale);
+      digits(std::integral_constant<int, 3>{}, dst, ops, doc_c, scale);
+      digits(std::integral_constant<int, 2>{}, dst, ops, doc_c, scale);
+      digits(std::integral_constant<int, 1>{}, dst, ops, doc_c, scale);
+      digits(std::integral_constant<int, 0>{}, dst, ops, doc_c, scale);
+    };
+    chain(acc[set], a, std::integral_constant<int, DOC>{}, sa);
+    if constexpr (RES) {
+      v8i r[KC];
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) r[kc] = operand(t.res[kc]);
+      chain(accr[set], r, std::integral_constant<int, kDocInt4>{}, sr);
+    }
+  };
+
+  // All steps of the tile in slot U, the previous tile's last epilogue in its
+  // first step.  The loads of the tile kRing - 1 ahead go to the previous
+  // tile's slot; their address arithmetic and the entry after them lie between
+  // the MFMAs.
+  Pend P;
+  bool masked = true;  // P.mask has rows past its tile
+  int last_set = 0;    // accumulator set of the last tile (one row block)
+  auto set_masks = [&](int rows) __attribute__((always_inline)) {
+    if constexpr (!UNIT) {
+      if (rows < 16 || masked) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) P.mask[k] = 4 * g + k >= rows ? kNegInf : -0.0f;
+        masked = rows < 16;
+      }
+    }
+  };
+  auto tile_steps = [&](auto u_c) __attribute__((always_inline)) {
+    constexpr int U = decltype(u_c)::value, kPrev = (U + kRing - 1) % kRing;
+    const Tile& t = ring[U];
+    auto fetch = [&](int m) __attribute__((always_inline)) {
+      if (m == 0) load(next, ring[kPrev]);
+      if (m == 1) {
+        next = entry(q + kRing);
+        ++q;
+      }
+    };
+    auto none = [](int) {};
+    step(t, 0, NT == 1 ? U & 1 : 0, P, NT - 1, NT == 1 ? (U + 1) & 1 : NT - 1, fetch);
+    const bool fresh = ((P.e >> kTileLastShift) & 1) != 0;
+    len += rows_of(P.e);
+    if (fresh) finish_target(P.e);
+    P.e = t.e;
+    last_set = U & 1;
+    if constexpr (!UNIT) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        P.s[k] = RES ? t.s[k] * mul : t.s[k];
+        if constexpr (RES) P.sr[k] = t.sr[k] * (16.0f * p.rmul);
+      }
+      set_masks(rows_of(P.e));
+    }
+    if (fresh) begin_target(P.e);
+#pragma unroll
+    for (int j = 1; j < NT; ++j) step(t, j, j, P, j - 1, j - 1, none);
+  };
+  // Before the first tile: zero accumulators and every row masked, whose
+  // epilogue changes nothing (no copy of the loop's body for the first tile:
+  // the compiler would wait for every load in flight to move it into the
+  // loop's registers).
+  P.e = score_tile_entry(0, 1, false, false, 0);
+#pragma unroll
+  for (int k = 0; k < (UNIT ? 1 : 4); ++k) {
+    P.s[k] = 0.0f;
+    P.mask[k] = kNegInf;
+  }
+#pragma unroll
+  for (int k = 0; k < (RES ? 4 : 1); ++k) P.sr[k] = 0.0f;
+#pragma unroll
+  for (int x = 0; x < kSets; ++x) acc[x] = (v4f){kStart, kStart, kStart, kStart};
+#pragma unroll
+  for (int x = 0; x < (RES ? kSets : 1); ++x) accr[x] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+  len = -1;  // that tile's row count
+  begin_target(ring[0].e);
+  // The tiles of slots k .. kRing - 1; false at the stream's end.
+  auto round = [&](auto self, auto u_c) __attribute__((always_inline)) -> bool {
+    constexpr int k = decltype(u_c)::value;
+    if constexpr (k == kRing) {
+      return true;
+    } else {
+      if (q == na) {
+        if (DIRECT || nb == 0) return false;
+        q = 0;  // unit A done: B follows
+        ta = tb;
+        na = nb;
+        int n = 0;
+        if (lane == 0) n = atomicAdd(&s_next, 1);
+        n = __builtin_amdgcn_readfirstlane(n);
+        unit(n, tb, nb);
+      }
+      tile_steps(u_c);
+      return self(self, std::integral_constant<int, k + 1>{});
+    }
+  };
+  while (round(round, std::integral_constant<int, 0>{})) {
+  }
+  // The last block of the last tile, right after its MFMAs.
+  mfma_results_fence();
+  {
+    float z[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      v4f x = acc[NT == 1 ? 0 : NT - 1], y = accr[RES && NT > 1 ? NT - 1 : 0];
+      if constexpr (NT == 1) {
+        x[k] = last_set ? acc[kSets - 1][k] : acc[0][k];
+        if constexpr (RES) y[k] = last_set ? accr[kSets - 1][k] : accr[0][k];
+      }
+      z[k] = zval(P, x, y, k);
+    }
+    fold(P, z, NT - 1);
+  }
+  len += rows_of(P.e);
+  finish_target(P.e);
+}
+
+template <int DOC, bool RES, int NT, int RED, int KC, bool UNIT = false>
+hipError_t launch_mode(const ScoreArgs& a, dim3 grid, hipStream_t s) {
+  constexpr int kThreads = kWave * group_waves(RES, KC);
+  if (a.direct_offsets) digit_score_kernel<DOC, RES, NT, RED, KC, UNIT, true><<<grid, kThreads, 0, s>>>(a);
+  else digit_score_kernel<DOC, RES, NT, RED, KC, UNIT, false><<<grid, kThreads, 0, s>>>(a);
+  return hipGetLastError();
+}
+template <int DOC, bool RES, int NT, int KC>
+hipError_t launch_reducer(const ScoreArgs& a, int reducer, dim3 grid, hipStream_t s) {
+  switch (reducer) {
+    case kRedMax: return launch_mode<DOC, RES, NT, kRedMax, KC>(a, grid, s);
+    case kRedTop2: return launch_mode<DOC, RES, NT, kRedTop2, KC>(a, grid, s);
+    case kRedTop4: return launch_mode<DOC, RES, NT, kRedTop4, KC>(a, grid, s);
+    case kRedLse: return launch_mode<DOC, RES, NT, kRedLse, KC>(a, grid, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+// The instantiations by document format (one source file each).
+hipError_t launch_int4(const ScoreArgs& a, bool residual, int nt, int reducer, dim3 grid, hipStream_t s);
+hipError_t launch_sign(const ScoreArgs& a, bool residual, int nt, int reducer, dim3 grid, hipStream_t s);
+hipError_t launch_wide(const ScoreArgs& a, int doc, bool residual, int nt, int reducer, dim3 grid, hipStream_t s);
+
+}  // namespace digit
+}  // namespace msim

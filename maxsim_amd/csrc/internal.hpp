@@ -171,9 +171,10 @@ void build_scan_tables(const int64_t* offsets, int64_t num_docs, int64_t waves, 
                        std::vector<int64_t>& wave_info, std::vector<uint64_t>& tile_table, int64_t& tile_stride,
                        int64_t& num_waves);
 
-// Generalized scoring (score.hip): int4 or sign-bit documents, optional int4
-// residual stream, 1 (int8) or 3 (fp32 split into int8 limbs) query limbs,
-// reducers.  Targets are documents or candidate positions, walked from a
+// Generalized scoring: fp32 queries as base-32 digits on fp6 / fp4 MFMA
+// (digit_score.hip: int4 or sign-bit documents, optional int4 residual stream,
+// reducers), int8 and sign-bit queries against sign documents (score.hip).
+// Targets are documents or candidate positions, walked from a
 // host-built table (build_score_tables): per wave kScoreInfoWords int64
 // words {target base, targets, tiles, first tile-table entry}, padded to
 // whole workgroups; per tile one entry: bits 0..33 first token, 34..37
@@ -192,22 +193,22 @@ constexpr int kScoreInfoWords = 4;
 enum : int { kDocInt4 = 0, kDocSign = 1 };
 enum : int { kRedMax = 0, kRedTop2 = 1, kRedTop4 = 2, kRedLse = 3 };
 struct ScoreArgs {
-  const uint8_t* codes;        // int4 [T, 64 chunks] or sign bits [T, 16 chunks]
+  const uint8_t* codes;        // sign bits [T, 16 chunks]; fp32 queries: or int4 as fp6 [T, 96 chunks]
   const float* tscale;         // [T] per-token scale of `codes` (never null)
   float tmul;                  // constant factor of the `codes` similarity
-  const uint8_t* rcodes;       // residual int4 codes [T, 64 chunks] (residual kernels)
+  const uint8_t* rcodes;       // residual int4 codes [T, 64], fp32 queries: as fp6 [T, 96 chunks]
   const float* rtscale;        // [T] residual per-token scale
   float rmul;
   const int64_t* wave_info;    // [groups][num_waves][kScoreInfoWords]
   const uint64_t* tiles;
-  // Work units (row-block pipeline kernels, eight waves per workgroup): 0 =
-  // wave w of a group takes record w of wave_info; n > 0 = workgroup x of a
-  // group owns records [n x, n x + n) (num_waves = n x workgroups), taken by
-  // its waves one after another from a counter in LDS; a record with no
-  // tiles ends the workgroup's list.
+  // Work units (fp32 queries over every document, eight waves per
+  // workgroup): workgroup x owns records [n x, n x + n) of wave_info
+  // (num_waves = n x workgroups), taken by its waves one after another from
+  // a counter in LDS; a record with no tiles ends the workgroup's list.
+  // (score.hip: wave w of a group takes record w.)
   int32_t group_units;
-  // Direct mode (wave_info / tiles unused): wave w of a group scores target w
-  // (w < direct_count), the document targets[w] whose tokens are
+  // Direct mode (wave_info / tiles unused): a wave scores one target t
+  // (t < direct_count), the document targets[t] whose tokens are
   // [direct_offsets[doc], direct_offsets[doc + 1]).
   const int64_t* direct_offsets;
   int64_t direct_count;
@@ -215,12 +216,13 @@ struct ScoreArgs {
   int64_t info_grp_stride;     // int64 words between groups' wave tables (0 = shared)
   const int64_t* targets;      // document of each target, or nullptr (target = document)
   int64_t targets_grp_stride;  // entries between groups' target lists
-  const int8_t* qpack;         // [limbs][rows_padded][128 chunks] B-operand order per 128-dim chunk
+  const int8_t* qpack;         // [rows_padded][128] B-operand order; fp32 queries: digits [rows_padded][5][96 chunks]
   int64_t rows_padded;
   const float* colmul;         // [rows_padded] per query row factor (sigma)
-  const int32_t* qsum;         // [limbs][rows_padded] limb sums (sign documents)
+  const int32_t* qsum;         // [rows_padded] code sums (int8 queries)
   const float* weights;        // [rows_padded] weighted MaxSim factors or nullptr
   int32_t subs;                // passes per group (query rows / rows per pass)
+  int32_t pass_rows;           // query rows per pass (fp32 queries)
   int32_t grp_rows;            // query rows per group
   const float* doc_scale;      // [num_docs] per-document scale or nullptr
   float scale;                 // document scale when doc_scale is null
@@ -245,19 +247,42 @@ struct ScoreArgs {
 // Query rows per pass of the fp4 Hamming kernel (sixteen 16-row blocks).
 constexpr int kHammingRowsPerPass = 256;
 hipError_t launch_hamming(const ScoreArgs& a, hipStream_t stream);
-// Dims above 128 are scored in 128-dim chunks whose MFMA dots accumulate in
-// one int32 accumulator: 2 chunks up to 256 dims, 4 up to 512 (0: above).
-// 512 is the limit of the three-limb combination 254 a1 + a2 in int32
-// (|a| <= 128 * 127 * 512 < 2^23).
+// Dims above 128 (fp32 queries) are scored in 128-dim chunks whose MFMA dots
+// accumulate in one accumulator: 2 chunks up to 256 dims, 4 up to 512 (0:
+// above; a 16-row pass of 512 dims takes 120 VGPRs of query digits).
 constexpr int64_t kScoreMaxDim = 512;
 inline int score_chunks(int64_t dim) { return dim <= 128 ? 1 : dim <= 256 ? 2 : dim <= 512 ? 4 : 0; }
-int score_rows_per_pass(int limbs, int64_t rows, int chunks = 1);
-hipError_t launch_score(const ScoreArgs& a, int doc, bool residual, int limbs, int reducer, int64_t groups,
-                        hipStream_t stream);
-// Query rows of 128 * chunks floats (dims past the query's own zero).
-hipError_t launch_quantize_limbs(const float* d_query, int64_t rows, int64_t rows_padded, int limbs, int layout,
-                                 bool recip, int8_t* qpack, float* colmul, int32_t* qsum, hipStream_t stream,
-                                 int layout2 = 0, int8_t* qpack2 = nullptr, int chunks = 1);
+int score_rows_per_pass(int64_t rows);
+hipError_t launch_score(const ScoreArgs& a, bool residual, int64_t groups, hipStream_t stream);
+
+// fp32 queries (digit_score.hip): digits per query element, the passes over a
+// group's batch rows, the digits [rows_padded][kScoreDigits][96 chunks] of
+// rows x 128 chunks floats, the fp6 rows of int4 codes (row_bytes bytes of
+// nibbles per token, the rest of its chunks zero), and the scorer itself.
+// launch_quantize_digits also copies `count` int64 values from src (pinned host
+// memory) to dst: candidate ids of the same call.
+constexpr int kScoreDigits = 5;
+// The work units' least tiles, by document format: more than a wave has in
+// flight.
+constexpr int kDigitUnitInt4 = 6, kDigitUnitSign = 10;
+struct DigitPlan {
+  int64_t pass_rows, subs;
+  int nt;      // 16-row blocks per pass: 1, 2 or 4
+  bool whole;  // passes hold whole batch rows
+};
+DigitPlan digit_plan(int64_t batch, int64_t query_tokens, int chunks);
+hipError_t launch_encode_fp6(const uint8_t* codes, int64_t tokens, int64_t row_bytes, int chunks, uint8_t* out,
+                             hipStream_t stream);
+hipError_t launch_quantize_digits(const float* d_query, int64_t rows, int64_t rows_padded, uint8_t* qpack,
+                                  float* colmul, int chunks, const int64_t* src, int64_t* dst, int64_t count,
+                                  hipStream_t stream);
+hipError_t launch_digit_score(const ScoreArgs& a, int doc, bool residual, int nt, int reducer, int64_t groups,
+                              hipStream_t stream);
+
+// int8 query rows of 128 floats.
+hipError_t launch_quantize_limbs(const float* d_query, int64_t rows, int64_t rows_padded, int layout, bool recip,
+                                 int8_t* qpack, float* colmul, int32_t* qsum, hipStream_t stream, int layout2 = 0,
+                                 int8_t* qpack2 = nullptr);
 hipError_t launch_quantize_bits(const uint8_t* d_qbits, int64_t rows, int64_t rows_padded, int8_t* qpack,
                                 float* colmul, int32_t* qsum, hipStream_t stream);
 hipError_t launch_pool_sum(const float* pooled, int64_t batch, int64_t query_tokens, int64_t targets, int64_t bs,
@@ -266,17 +291,18 @@ hipError_t launch_pool_sum(const float* pooled, int64_t batch, int64_t query_tok
 // over about `waves` waves, balanced by tiles + 1 per target.
 void build_score_tables(const int64_t* offsets, const int64_t* targets, int64_t num_targets, int64_t waves,
                         std::vector<int64_t>& info, std::vector<uint64_t>& tiles);
-// Work units of the row-block pipeline kernels (ScoreArgs::group_units): the
+// Work units of the fp32-query scorer (ScoreArgs::group_units): the
 // targets balanced over `workgroups` lists (tiles + 1 per target, longest
 // first onto the least-loaded list), each list cut into units of whole
 // targets, longest first, every unit but the list's last of at least
-// kScoreUnitMinTiles tiles; lists padded with empty records to the same
+// min_tiles tiles (what a wave loads ahead); lists padded with empty records to the same
 // count, which is returned.  Tile entries hold absolute target indices, so
 // num_targets must be below 2^24 (kScoreMaxUnitTargets).
 constexpr int64_t kScoreUnitMinTiles = 4;
 constexpr int64_t kScoreMaxUnitTargets = int64_t(1) << 24;
 int64_t build_score_units(const int64_t* offsets, const int64_t* targets, int64_t num_targets, int64_t workgroups,
-                          std::vector<int64_t>& info, std::vector<uint64_t>& tiles);
+                          std::vector<int64_t>& info, std::vector<uint64_t>& tiles,
+                          int64_t min_tiles = kScoreUnitMinTiles);
 
 // Cascade helpers (cascade.hip): tile tables of per-group candidate lists
 // written on the device (groups x waves waves of at most per_wave

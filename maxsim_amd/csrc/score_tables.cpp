@@ -86,7 +86,7 @@ void build_score_tables(const int64_t* off, const int64_t* targets, int64_t n, i
 }
 
 int64_t build_score_units(const int64_t* off, const int64_t* targets, int64_t n, int64_t workgroups,
-                          std::vector<int64_t>& info, std::vector<uint64_t>& tiles) {
+                          std::vector<int64_t>& info, std::vector<uint64_t>& tiles, int64_t min_tiles) {
   info.clear();
   tiles.clear();
   workgroups = std::max<int64_t>(1, std::min(workgroups, std::max<int64_t>(1, n)));
@@ -108,6 +108,7 @@ int64_t build_score_units(const int64_t* off, const int64_t* targets, int64_t n,
     mine[(size_t)l.second].push_back(t);
     heap.push({l.first + tiles_of(t) + 1, l.second});
   }
+  tiles.push_back(score_tile_entry(0, 1, false, true, 0));  // padding: what a wave loads past its list's end
   std::vector<std::vector<int64_t>> units((size_t)workgroups);  // records, kScoreInfoWords each
   int64_t most = 1;
   for (int64_t w = 0; w < workgroups; ++w) {
@@ -126,7 +127,7 @@ int64_t build_score_units(const int64_t* off, const int64_t* targets, int64_t n,
       for (int64_t x = s; x < e; x += 16)
         tiles.push_back(score_tile_entry(x, std::min<int64_t>(16, e - x), x + 16 >= e, false, t));
       ++count;
-      if ((int64_t)tiles.size() - tab0 >= kScoreUnitMinTiles) close();
+      if ((int64_t)tiles.size() - tab0 >= min_tiles) close();
     }
     if (count > 0) close();
     most = std::max<int64_t>(most, (int64_t)rec.size() / kScoreInfoWords);
@@ -138,7 +139,6 @@ int64_t build_score_units(const int64_t* off, const int64_t* targets, int64_t n,
     }
     info.insert(info.end(), rec.begin(), rec.end());
   }
-  if (tiles.empty()) tiles.push_back(score_tile_entry(0, 1, false, false, 0));
   return most;
 }
 

@@ -1,0 +1,111 @@
+"""fp32 queries as five base-32 digits against the C oracle, at the tile, chunk and pass edges.
+
+The documents are exact in fp32 (scales are powers of two), so with
+e = 2^-24 the scores differ from exact ones by, per query token and at
+its documents' largest sum |doc||q|: the row's fixed point (half a unit of
+2^(E-24), 2^E <= 2 max|q|), one fp32 rounding per MFMA of the chain (five digits
+per 128 dims, a residual's as many) and up to eight in the epilogue, weights
+and the oracle; then one per addition of the query tokens.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = (1, 15, 16, 17, 0, 31, 32, 33, 100, 0, 129, 1)
+
+
+def _codes(rng, tokens, dim):
+    v = rng.integers(-8, 8, (tokens, dim)).astype(np.int8)
+    v[0] = -8
+    return v, ((v[:, 0::2] & 15) | ((v[:, 1::2] & 15) << 4)).astype(np.uint8)
+
+
+def _bound(query, sims_abs, row_abs, streams, chunks, temperature):
+    """[batch, docs]: the error of the module's docstring, both sides together."""
+    e = 2.0**-24
+    per_row = sims_abs * (streams * 5 * chunks + 8) * e + row_abs * 2 * e + temperature * 16 * e + 2.0**-146
+    return per_row.sum(1) + sims_abs.sum(1) * query.shape[1] * e
+
+
+def _doc_max(x, offsets):
+    """Largest of each document's tokens: x [tokens, rows] -> [docs, rows]."""
+    return np.stack([x[s:e].max(0) if e > s else np.zeros(x.shape[1]) for s, e in zip(offsets[:-1], offsets[1:])])
+
+
+@pytest.mark.parametrize("kind", ["int4", "residual", "sign", "sign_scaled"])
+@pytest.mark.parametrize("dim", [8, 128, 136, 256, 264, 512])
+@pytest.mark.parametrize("shape", [(1, 1), (1, 16), (3, 17), (2, 32), (5, 32), (2, 65)])
+def test_digit_scores_at_the_edges(gpu, oracle, kind, dim, shape):
+    from maxsim_amd._maxsim_hip import CudaInt4PackedDocs, CudaPackedDocs
+
+    rng = np.random.default_rng(dim * 100 + shape[0] * shape[1])
+    lengths = np.array(LENGTHS * 3, np.int64)
+    offsets = np.concatenate(([0], np.cumsum(lengths))).astype(np.int64)
+    tokens = int(offsets[-1])
+    scale = np.exp2(rng.integers(-2, 3, tokens)).astype(np.float32)
+    values, packed = _codes(rng, tokens, dim)
+    streams = 1
+    if kind in ("int4", "residual"):
+        h = CudaInt4PackedDocs(packed, offsets, dim, 1.0)
+        h.set_token_scale_vector(scale)
+        docs = values * scale[:, None]
+        score, cand_score, kw = h.score_batch, h.score_candidates_batch, {}
+        if kind == "residual":
+            values2, packed2 = _codes(rng, tokens, dim)
+            scale2 = scale / 16
+            h.set_residual_int4(packed2, 1.0, scale2)
+            docs = docs + values2 * scale2[:, None]
+            score, cand_score, streams = h.score_residual_batch, h.score_residual_candidates_batch, 2
+    else:
+        bits = rng.integers(0, 2, (tokens, dim))
+        h = CudaPackedDocs(np.packbits(bits, axis=1, bitorder="little"), offsets, dim)
+        docs = (2 * bits - 1).astype(np.float32)
+        score, cand_score, kw = h.score_batch, h.score_candidates_batch, {}
+        if kind == "sign_scaled":
+            h.set_token_scale_vector(scale)
+            docs = docs * scale[:, None]
+            kw = {"use_token_scale": True}
+    query = rng.standard_normal((*shape, dim)).astype(np.float32)
+    flat = query.reshape(-1, dim)
+    flat[0] = 0.0
+    flat[-1, 0] = 64.0  # one element far above the rest of its row
+    if shape[0] > 1:  # whole batch rows far from the others
+        query[1] *= np.float32(1e30)
+        query[-1] *= np.float32(1e-41) if shape[0] > 2 else np.float32(1)
+    ids = rng.integers(0, lengths.size, 37)
+    chunks = {8: 1, 128: 1, 136: 2, 256: 2}.get(dim, 4)
+    mag = np.abs(docs).astype(np.float64)
+    if kind == "residual":
+        mag = np.abs(values * scale[:, None]).astype(np.float64) + np.abs(values2 * scale2[:, None])
+    q64 = np.abs(flat).astype(np.float64)
+    sims = _doc_max(mag @ q64.T, offsets).T.reshape(*shape, lengths.size)
+    rows = (_doc_max(mag.sum(1)[:, None], offsets).T * q64.max(1)[:, None]).reshape(*shape, lengths.size)
+    for reducer, temperature in (("maxsim", 0.0), ("topk2", 0.0), ("topk4", 0.0), ("smoothsim", 0.5)):
+        if reducer == "smoothsim" and shape[0] > 1:
+            continue  # exponents of rows of 1e30
+        args = {"temperature": temperature} if reducer == "smoothsim" else {}
+        got = score(query, reducer, None, **args, **kw)
+        exp = oracle.dense_scores(query, docs, offsets, reducer=reducer, **args)
+        err = np.abs(got.astype(np.float64) - exp)
+        # (a log-sum of up to 129 terms rounds each of them)
+        bound = _bound(query, sims, rows, streams, chunks, 129 * temperature)
+        assert (err <= bound).all(), (reducer, float((err / np.maximum(bound, 1e-300)).max()))
+        np.testing.assert_array_equal(cand_score(query, ids, reducer, None, **args, **kw), got[:, ids])
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_rows_that_are_not_finite_leave_the_others_alone(gpu, bad):
+    from maxsim_amd._maxsim_hip import CudaInt4PackedDocs
+
+    rng = np.random.default_rng(5)
+    offsets = np.arange(0, 40 * 33, 33, dtype=np.int64)
+    _, packed = _codes(rng, int(offsets[-1]), 128)
+    h = CudaInt4PackedDocs(packed, offsets, 128, 0.1)
+    query = rng.standard_normal((4, 8, 128)).astype(np.float32)
+    clean = h.score_batch(query, "maxsim")
+    query[2, 3, 7] = bad
+    got = h.score_batch(query, "maxsim")
+    np.testing.assert_array_equal(got[[0, 1, 3]], clean[[0, 1, 3]])
+    if np.isinf(bad):
+        assert np.isnan(got[2]).all()
