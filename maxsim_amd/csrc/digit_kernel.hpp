@@ -376,6 +376,12 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
     }
     st[j].add4(z, k2);
   };
+  // MFMAs stay before the pins of their result, and its reads behind the next
+  // one: the compiler otherwise sinks a chain to its epilogue in a later
+  // step, or hoists the row mask up to the chain, and the epilogue stands
+  // right behind the MFMAs (too early for max3_op, whose inline asm operands
+  // get no wait states, and with nothing to overlap).
+  auto pin = [](v4f& x) __attribute__((always_inline)) { asm volatile("" : "+v"(x)); };
   // One step: the MFMAs of row block j of tile t into accumulator set `set`.
   // Between them, from the third MFMA on, the epilogue of the step before
   // (tile P, its block jp and set), and what extra(m) puts after MFMA m.
@@ -388,6 +394,10 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
     auto after = [&](int m) __attribute__((always_inline)) {
       extra(m);
       if (m >= kWait) {
+        if (m == kWait) {
+          pin(acc[setp]);
+          if constexpr (RES) pin(accr[setp]);
+        }
 #pragma unroll
         for (int k = 0; k < 4; ++k)
           if (kWait + k * kSpan / 4 == m) z[k] = zval(P, acc[setp], accr[RES ? setp : 0], k);
@@ -408,6 +418,7 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
       for (int kc = 0; kc < KC; ++kc) {
         const v4f& from = d == kDigits - 1 && kc == 0 ? zero : dst;
         dst = mfma_digit<decltype(doc_c)::value, d>(ops[kc], operand(bq[j][d][kc]), from, scale, s03, s4);
+        if (m == kWait) pin(dst);
         after(m++);
       }
     };
@@ -417,6 +428,7 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
       digits(std::integral_constant<int, 2>{}, dst, ops, doc_c, scale);
       digits(std::integral_constant<int, 1>{}, dst, ops, doc_c, scale);
       digits(std::integral_constant<int, 0>{}, dst, ops, doc_c, scale);
+      pin(dst);
     };
     chain(acc[set], a, std::integral_constant<int, DOC>{}, sa);
     if constexpr (RES) {
