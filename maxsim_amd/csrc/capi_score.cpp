@@ -105,6 +105,58 @@ void set_streams(ScoreArgs& a, const DocStreams& s) {
   a.unit_tscale = s.unit_tscale;
 }
 
+// Every document as work units for `workgroups` workgroups at once: a list per
+// workgroup and pass; few documents are spread over as many workgroups.
+void set_units(ScoreWorkspace& ws, const std::vector<int64_t>& off, int64_t workgroups, int64_t subs, int64_t min_tiles,
+               ScoreArgs& a) {
+  const int64_t num_docs = (int64_t)off.size() - 1;
+  const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(workgroups / subs, num_docs));
+  if (ws.full_key != -2 - wgs) {
+    std::vector<int64_t> info;
+    std::vector<uint64_t> tiles;
+    ws.full_units = build_score_units(off.data(), nullptr, num_docs, wgs, info, tiles, min_tiles);
+    upload_vec(ws.full_info, info, "copy score wave table to device");
+    upload_vec(ws.full_tiles, tiles, "copy score tile table to device");
+    ws.full_key = -2 - wgs;
+    ws.full_waves = (int64_t)info.size() / kScoreInfoWords;
+  }
+  a.wave_info = ws.full_info.as<int64_t>();
+  a.tiles = ws.full_tiles.as<uint64_t>();
+  a.num_waves = ws.full_waves;
+  a.group_units = (int32_t)ws.full_units;
+}
+
+// Sign-bit queries against every sign document (MaxSim, unit token scales).
+void run_hamming_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, const DocStreams& s, const uint8_t* d_qbits,
+                       int64_t batch, int64_t query_tokens, float* d_out, int64_t out_stride, int32_t* d_iout,
+                       hipStream_t stream) {
+  const int64_t num_docs = (int64_t)off.size() - 1, rows = batch * query_tokens;
+  const HammingPlan plan = hamming_plan(batch, query_tokens);
+  ScoreArgs a{};
+  set_streams(a, s);
+  set_units(ws, off, 2 * device_cu_count(), plan.subs, kDigitUnitSign, a);
+  a.qbits = d_qbits;
+  a.subs = (int32_t)plan.subs;
+  a.pass_rows = (int32_t)plan.pass_rows;
+  a.grp_rows = (int32_t)rows;
+  a.query_tokens = (int32_t)query_tokens;
+  a.chunks = 1;
+  if (plan.whole) {
+    a.out = d_out;
+    a.out_stride = out_stride;
+    a.iout = d_iout;
+    a.iout_stride = num_docs;
+    check_hip(launch_hamming(a, stream), "launch fp4 hamming kernel");
+    return;
+  }
+  ws.pooled.ensure(sizeof(float) * num_docs * rows, "hipMalloc pooled rows");
+  a.pooled = ws.pooled.as<float>();
+  check_hip(launch_hamming(a, stream), "launch fp4 hamming kernel");
+  check_hip(launch_pool_sum(ws.pooled.as<float>(), batch, query_tokens, num_docs, query_tokens, rows, d_out, out_stride,
+                            d_iout, stream),
+            "launch pooled sum kernel");
+}
+
 // fp32 queries: digits, then one launch over every document (work units) or
 // over candidate documents (one per wave).
 void run_digit_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, const DocStreams& s, const QueryInput& q,
@@ -141,23 +193,7 @@ void run_digit_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, const 
     a.direct_offsets = t.d_offsets;
     a.direct_count = targets;
   } else {
-    // A list of work units per CU and pass; few documents are spread over as
-    // many CUs.
-    const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(device_cu_count() / plan.subs, num_docs));
-    if (ws.full_key != -2 - wgs) {
-      std::vector<int64_t> info;
-      std::vector<uint64_t> tiles;
-      ws.full_units = build_score_units(off.data(), nullptr, num_docs, wgs, info, tiles,
-                                        s.doc == kDocSign ? kDigitUnitSign : kDigitUnitInt4);
-      upload_vec(ws.full_info, info, "copy score wave table to device");
-      upload_vec(ws.full_tiles, tiles, "copy score tile table to device");
-      ws.full_key = -2 - wgs;
-      ws.full_waves = (int64_t)info.size() / kScoreInfoWords;
-    }
-    a.wave_info = ws.full_info.as<int64_t>();
-    a.tiles = ws.full_tiles.as<uint64_t>();
-    a.num_waves = ws.full_waves;
-    a.group_units = (int32_t)ws.full_units;
+    set_units(ws, off, device_cu_count(), plan.subs, s.doc == kDocSign ? kDigitUnitSign : kDigitUnitInt4, a);
   }
   a.qpack = ws.qpack.as<int8_t>();
   a.rows_padded = rows_padded;
@@ -215,17 +251,21 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
   if (reducer != kRedMax || h_row_weights) throw NotSupported("int8 and sign-bit queries are scored with MaxSim");
   const int64_t rows_padded = ceil_div(rows, 16) * 16 + 128;
 
-  // Sign-bit queries against sign documents over every document, MaxSim on
-  // unit token scales: the fp4 Hamming kernel reads the query bits itself.
-  const bool fp4 = g_hamming_fp4 != 0 && q.d_qbits && !s.residual && s.unit_tscale && !t.host && !t.device;
+  // Sign-bit queries over every document on unit token scales: the fp4
+  // Hamming kernel reads the query bits itself.
+  if (g_hamming_fp4 != 0 && q.d_qbits && !s.residual && s.unit_tscale && !t.host && !t.device && !s.doc_scale &&
+      num_docs < kScoreMaxUnitTargets) {
+    run_hamming_score(ws, off, s, q.d_qbits, batch, query_tokens, d_out, out_stride, d_iout, stream);
+    return;
+  }
 
   // 1. Quantise the query rows.
   ws.qpack.ensure((size_t)rows_padded * 128, "hipMalloc query codes");
   ws.colmul.ensure(sizeof(float) * rows_padded, "hipMalloc query scales");
   ws.qsum.ensure(sizeof(int32_t) * rows_padded, "hipMalloc query code sums");
   if (q.alt_int4) ws.qpack_alt.ensure((size_t)rows_padded * 128, "hipMalloc query codes (int4 layout)");
-  if (q.quantized || q.from_alt || fp4) {
-    // reuse the workspace's quantised rows (the fp4 kernel reads the bits)
+  if (q.quantized || q.from_alt) {
+    // reuse the workspace's quantised rows
   } else if (q.d_qbits)
     check_hip(launch_quantize_bits(q.d_qbits, rows, rows_padded, ws.qpack.as<int8_t>(), ws.colmul.as<float>(),
                                    ws.qsum.as<int32_t>(), stream),
@@ -241,7 +281,7 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
   // 2. Work split.
   const int64_t groups = t.per_row ? batch : 1;
   const int64_t grp_rows = t.per_row ? query_tokens : rows;
-  const int64_t rpp = fp4 ? kHammingRowsPerPass : score_rows_per_pass(grp_rows);
+  const int64_t rpp = score_rows_per_pass(grp_rows);
   const int64_t subs = ceil_div(grp_rows, rpp);
   const int64_t per_target = t.per_row ? t.count : targets;
   int64_t waves = ceil_div((int64_t)device_cu_count() * 8, groups * subs);
@@ -315,13 +355,9 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
   a.temperature = temperature;
   a.query_tokens = (int32_t)query_tokens;
   a.chunks = 1;
-  a.qbits = fp4 ? q.d_qbits : nullptr;
   // Passes that hold whole batch rows let the kernel sum them itself.
   const bool in_kernel_sum = t.per_row ? subs == 1 : rpp % query_tokens == 0;
-  auto launch = [&] {
-    if (fp4) check_hip(launch_hamming(a, stream), "launch fp4 hamming kernel");
-    else check_hip(launch_score(a, s.residual, groups, stream), "launch score kernel");
-  };
+  auto launch = [&] { check_hip(launch_score(a, s.residual, groups, stream), "launch score kernel"); };
   if (in_kernel_sum) {
     a.out = d_out;
     a.out_stride = out_stride;

@@ -204,6 +204,12 @@ __device__ __forceinline__ float max3_op(float a, float b, float c) {
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
+// The maximum of m and four values in two v_max3_f32 (one asm: the compiler puts
+// a wait state between two of max3_op).
+__device__ __forceinline__ float max5_op(float m, float a, float b, float c, float d) {
+  asm("v_max3_f32 %0, %0, %1, %2\n\tv_max3_f32 %0, %0, %3, %4" : "+v"(m) : "v"(a), "v"(b), "v"(c), "v"(d));
+  return m;
+}
 
 // numpy's pairwise float64 reduction order over a[0..n) for 8 < n <= 128 is
 // eight strided accumulators, combined ((r0+r1)+(r2+r3))+((r4+r5)+(r6+r7)),

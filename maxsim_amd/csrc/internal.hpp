@@ -201,7 +201,7 @@ struct ScoreArgs {
   float rmul;
   const int64_t* wave_info;    // [groups][num_waves][kScoreInfoWords]
   const uint64_t* tiles;
-  // Work units (fp32 queries over every document, eight waves per
+  // Work units (fp32 and sign-bit queries over every document, eight waves per
   // workgroup): workgroup x owns records [n x, n x + n) of wave_info
   // (num_waves = n x workgroups), taken by its waves one after another from
   // a counter in LDS; a record with no tiles ends the workgroup's list.
@@ -222,7 +222,7 @@ struct ScoreArgs {
   const int32_t* qsum;         // [rows_padded] code sums (int8 queries)
   const float* weights;        // [rows_padded] weighted MaxSim factors or nullptr
   int32_t subs;                // passes per group (query rows / rows per pass)
-  int32_t pass_rows;           // query rows per pass (fp32 queries)
+  int32_t pass_rows;           // query rows per pass (fp32 and sign-bit queries)
   int32_t grp_rows;            // query rows per group
   const float* doc_scale;      // [num_docs] per-document scale or nullptr
   float scale;                 // document scale when doc_scale is null
@@ -241,11 +241,16 @@ struct ScoreArgs {
   bool unit_tscale;            // tscale is all ones (sign documents): integer maximum
   int32_t chunks;              // 128-dim chunks per token and query row (1, 2 or 4)
   // Sign-bit queries [rows][16] (pack_signs order) scored against sign
-  // documents by the fp4 Hamming kernel (launch_hamming); null otherwise.
+  // documents by the fp4 Hamming kernel (launch_hamming: work units, pass_rows, chunks 1).
   const uint8_t* qbits;
 };
-// Query rows per pass of the fp4 Hamming kernel (sixteen 16-row blocks).
+// Query rows per pass of the fp4 Hamming kernel at most (sixteen 16-row blocks).
 constexpr int kHammingRowsPerPass = 256;
+struct HammingPlan {
+  int64_t pass_rows, subs;
+  bool whole;  // passes hold whole batch rows
+};
+HammingPlan hamming_plan(int64_t batch, int64_t query_tokens);
 hipError_t launch_hamming(const ScoreArgs& a, hipStream_t stream);
 // Dims above 128 (fp32 queries) are scored in 128-dim chunks whose MFMA dots
 // accumulate in one accumulator: 2 chunks up to 256 dims, 4 up to 512 (0:

@@ -21,7 +21,7 @@ struct ReducerState<kRedMax> {
   float m;
   __device__ void init() { m = kNegInf; }
   // Two three-way maxima (v_max3_f32) for four values: exact, any order.
-  __device__ void add4(const float (&z)[4], float) { m = max3_op(max3_op(m, z[0], z[1]), z[2], z[3]); }
+  __device__ void add4(const float (&z)[4], float) { m = max5_op(m, z[0], z[1], z[2], z[3]); }
   __device__ float finish(int len, float colmul, float, float weight, float doc_scale) const {
     return len == 0 ? 0.0f : m * colmul * weight * doc_scale;
   }
@@ -138,18 +138,65 @@ __device__ __forceinline__ void sum_batch_rows(const float* x, int nb, int n, Pu
   }
 }
 
+// A wave's tiles from its workgroup's list of work units (ScoreArgs::
+// group_units): it starts with units `wave` and wave + WAVES and takes the following
+// ones from the counter `taken` in LDS (set to 2 WAVES, visible), the unit after the
+// current one known ahead.  next() is called once per tile, ahead of its use;
+// past the list's end it returns the table's padding entry (token 0), which
+// ended() recognises.  The waves of a SIMD do not share it evenly (the older
+// wave issues first); taking units as they go, all finish with the list.
+template <int WAVES>
+struct TileStream {
+  using TilePtr = const __attribute__((address_space(4))) uint64_t*;
+  TilePtr pad, cur, after;
+  const __attribute__((address_space(4))) int64_t* info;
+  int left, count, units, lane;
+  int* taken;
+  __device__ __forceinline__ TileStream(const ScoreArgs& p, int wave, int lane_, int& counter) {
+    pad = cur = after = as_constant(p.tiles);
+    units = p.group_units;
+    info = as_constant(p.wave_info) + (int64_t)blockIdx.x * units * kScoreInfoWords;
+    lane = lane_;
+    taken = &counter;
+    unit(wave, cur, left);
+    unit(wave + WAVES, after, count);
+  }
+  __device__ __forceinline__ void unit(int k, TilePtr& tp, int& n) const {
+    n = 0;
+    tp = pad;
+    if (k < units) {
+      n = (int)info[(int64_t)k * kScoreInfoWords + 2];
+      tp = pad + info[(int64_t)k * kScoreInfoWords + 3];
+    }
+  }
+  __device__ __forceinline__ uint64_t next() {
+    if (left == 0) {
+      cur = after;
+      left = max(count, 1);  // past the end: the padding entry, again and again
+      if (count > 0) {
+        int k = 0;
+        if (lane == 0) k = atomicAdd(taken, 1);
+        unit(__builtin_amdgcn_readfirstlane(k), after, count);
+      }
+    }
+    --left;
+    return *cur++;
+  }
+  static __device__ __forceinline__ bool ended(uint64_t e) {
+    return ((e >> kTileLastShift) & 3) == 2;  // empty, and no target's last tile
+  }
+};
+
 // 32 sign bits of one lane (dims 32g .. 32g + 31, bit b = dim 32g + b; set =
 // +1) as the fp4 (e2m1) operand of v_mfma_scale_f32_16x16x128_f8f6f4: dword
 // q holds dims 32g + 4i + q in nibble i, +1 as 0x2 and -1 as 0xA: operand
 // element s (of the lane's 32) is dim 32g + 4 (s % 8) + s / 8.
 __device__ __forceinline__ v4i fp4_signs(unsigned w) {
-  const unsigned n = ~w;
-  v4i a;
-  a[0] = (int)(0x22222222u | ((n << 3) & 0x88888888u));
-  a[1] = (int)(0x22222222u | ((n << 2) & 0x88888888u));
-  a[2] = (int)(0x22222222u | ((n << 1) & 0x88888888u));
-  a[3] = (int)(0x22222222u | (n & 0x88888888u));
-  return a;
+  // 0x2 | (not sign ? 0x8) of every nibble: one v_bitop3_b32 (c | (~a & b)).
+  auto dword = [](unsigned x) __attribute__((always_inline)) {
+    return (int)__builtin_amdgcn_bitop3_b32(x, 0x88888888u, 0x22222222u, 0xAE);
+  };
+  return (v4i){dword(w << 3), dword(w << 2), dword(w << 1), dword(w)};
 }
 
 }  // namespace msim
