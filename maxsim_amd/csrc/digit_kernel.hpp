@@ -147,7 +147,6 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
   static_assert(!UNIT || (DOC == kDocSign && !RES && RED == kRedMax), "accumulators as similarities");
   static_assert(!(DOC == kDocSign && RES) || KC == 1, "sign prefix + residual: 128 dims");
   constexpr int kRing = ring_size(DOC, RES, NT, KC, UNIT);
-  static_assert(kRing < (DOC == kDocSign ? kDigitUnitSign : kDigitUnitInt4), "work units cover the tiles loaded ahead");
   static_assert(kRing % 2 == 0, "accumulator sets alternate over an even ring");
   constexpr int kSets = NT == 1 ? 2 : NT;  // accumulators of a step and of the step before it
   constexpr int kCodeBytes = (DOC == kDocInt4 ? 96 : 16) * KC, kResBytes = 96 * KC, kRowBytes = 96 * KC;
@@ -159,6 +158,10 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
   __shared__ __attribute__((aligned(16))) v4i s_q[kVecs];
   __shared__ float s_pool[kWavesPerGroup][16 * NT];
   __shared__ int s_next;
+  if constexpr (!DIRECT) {
+    if (threadIdx.x == 0) s_next = 2 * kWavesPerGroup;
+    __syncthreads();
+  }
   const int lane = lane_id();
   const int wave = wave_uniform(threadIdx.x / kWave);
   const int g = lane >> 4, c = lane & 15;
@@ -166,29 +169,12 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
   const int lr0 = sub * p.pass_rows;                      // first local row of the pass
   const int64_t grow0 = (int64_t)grp * p.grp_rows + lr0;  // its global query row
 
-  // The tile stream.  Work units: a wave starts with units `wave` and wave + 8
-  // of its workgroup's list and takes the following ones from a counter; unit
-  // A holds the current tile, unit B the next one, taken as A starts.  Every
-  // unit but a list's last has more than kRing tiles, so the tiles loaded ahead
-  // (and the entry after them) lie in A or B; past the list's end they are the
-  // table's padding entry (token 0).  The two waves of a SIMD do not share it
-  // evenly (the older wave issues first); taking units as they go, both finish
-  // with the workgroup's list.
-  using TilePtr = const __attribute__((address_space(4))) uint64_t*;
+  // The wave's tiles: work units, or (DIRECT) the tiles of one target.  Either
+  // way the end is an entry that tiles_ended() recognises, of token 0, again and
+  // again.
   const int64_t gw = (int64_t)wave * gridDim.x + blockIdx.x;  // DIRECT: the target
   int64_t ds = 0, doc0 = 0;
-  int ntok = 0, na = 0, nb = 0;
-  const TilePtr pad = as_constant(p.tiles);
-  TilePtr ta = pad, tb = pad;
-  const auto unit_info = as_constant(p.wave_info) + (int64_t)blockIdx.x * p.group_units * kScoreInfoWords;
-  auto unit = [&](int k, TilePtr& tp, int& n) __attribute__((always_inline)) {
-    n = 0;
-    if (k < p.group_units) {
-      const auto rec = unit_info + (int64_t)k * kScoreInfoWords;
-      n = (int)rec[2];
-      tp = pad + rec[3];
-    }
-  };
+  int ntok = 0, na = 0, q = 0;
   if constexpr (DIRECT) {
     if (gw < p.direct_count) {
       doc0 = p.targets ? as_constant(p.targets)[grp * p.targets_grp_stride + gw] : gw;
@@ -196,18 +182,18 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
       ntok = (int)(as_constant(p.direct_offsets)[doc0 + 1] - ds);
       na = ntok == 0 ? 1 : (ntok + 15) / 16;  // an empty document: one tile, not scored
     }
-  } else {
-    unit(wave, ta, na);
-    unit(wave + kWavesPerGroup, tb, nb);
   }
-  // Entry of the tile at position q of unit A (and on into B).
-  auto entry = [&](int q) __attribute__((always_inline)) -> uint64_t {
+  TileStream<kWavesPerGroup> stream(p, DIRECT ? -1 : wave, lane, s_next);
+  auto next_entry = [&]() __attribute__((always_inline)) -> uint64_t {
     if constexpr (DIRECT) {
       const int left = ntok - 16 * q;
       const bool in = left > 0;
-      return score_tile_entry(in ? ds + 16 * (int64_t)q : 0, in ? min(16, left) : 1, q + 1 == na, ntok == 0, 0);
+      const uint64_t e =
+          score_tile_entry(in ? ds + 16 * (int64_t)q : 0, in ? min(16, left) : 1, q + 1 == na, left <= 0, 0);
+      q = min(q + 1, na);
+      return e;
     } else {
-      return *(q < na ? ta + q : q - na < nb ? tb + (q - na) : pad);
+      return stream.next();
     }
   };
 
@@ -268,16 +254,14 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
   };
   Tile ring[kRing];
 #pragma unroll
-  for (int u = 0; u < kRing - 1; ++u) load(entry(u), ring[u]);
-  uint64_t next = entry(kRing - 1);  // the entry of the tile loaded next
-  int q = 0;                         // position (in A) of the current tile
+  for (int u = 0; u < kRing - 1; ++u) load(next_entry(), ring[u]);
+  uint64_t next = next_entry();  // the entry of the tile loaded next
   __builtin_amdgcn_sched_barrier(0);
 
-  if (threadIdx.x == 0) s_next = 2 * kWavesPerGroup;
 #pragma unroll
   for (int x = 0; x < kStage; ++x) s_q[min((int)threadIdx.x + x * kThreads, kVecs - 1)] = stage[x];
   __syncthreads();
-  if (na == 0) return;  // no barriers below
+  if (tiles_ended(ring[0].e)) return;  // no barriers below
   Six bq[NT][kDigits][KC];
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
@@ -460,10 +444,7 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
     const Tile& t = ring[U];
     auto fetch = [&](int m) __attribute__((always_inline)) {
       if (m == 0) load(next, ring[kPrev]);
-      if (m == 1) {
-        next = entry(q + kRing);
-        ++q;
-      }
+      if (m == 1) next = next_entry();
     };
     auto none = [](int) {};
     step(t, 0, NT == 1 ? U & 1 : 0, P, NT - 1, NT == 1 ? (U + 1) & 1 : NT - 1, fetch);
@@ -508,16 +489,7 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
     if constexpr (k == kRing) {
       return true;
     } else {
-      if (q == na) {
-        if (DIRECT || nb == 0) return false;
-        q = 0;  // unit A done: B follows
-        ta = tb;
-        na = nb;
-        int n = 0;
-        if (lane == 0) n = atomicAdd(&s_next, 1);
-        n = __builtin_amdgcn_readfirstlane(n);
-        unit(n, tb, nb);
-      }
+      if (tiles_ended(ring[k].e)) return false;
       tile_steps(u_c);
       return self(self, std::integral_constant<int, k + 1>{});
     }

@@ -83,7 +83,7 @@ __global__ __launch_bounds__(kGroupThreads, 4) void hamming_kernel(ScoreArgs p) 
 #pragma unroll
   for (int u = 0; u < kRing - 1; ++u) load(stream.next(), ring[u]);
   uint64_t next = stream.next();
-  if (TileStream<kWaves>::ended(ring[0].e)) return;  // no barriers below
+  if (tiles_ended(ring[0].e)) return;  // no barriers below
 
   v4i bq[NT];
 #pragma unroll
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(kGroupThreads, 4) void hamming_kernel(ScoreArgs p) 
     if constexpr (k == kRing) {
       return true;
     } else {
-      if (TileStream<kWaves>::ended(ring[k].e)) {
+      if (tiles_ended(ring[k].e)) {
         last_slot0 = NT == 2 ? 2 * ((k + 1) & 1) : 0;  // of slot k - 1
         return false;
       }

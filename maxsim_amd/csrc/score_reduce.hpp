@@ -143,7 +143,7 @@ __device__ __forceinline__ void sum_batch_rows(const float* x, int nb, int n, Pu
 // ones from the counter `taken` in LDS (set to 2 WAVES, visible), the unit after the
 // current one known ahead.  next() is called once per tile, ahead of its use;
 // past the list's end it returns the table's padding entry (token 0), which
-// ended() recognises.  The waves of a SIMD do not share it evenly (the older
+// tiles_ended() recognises.  The waves of a SIMD do not share it evenly (the older
 // wave issues first); taking units as they go, all finish with the list.
 template <int WAVES>
 struct TileStream {
@@ -154,7 +154,7 @@ struct TileStream {
   int* taken;
   __device__ __forceinline__ TileStream(const ScoreArgs& p, int wave, int lane_, int& counter) {
     pad = cur = after = as_constant(p.tiles);
-    units = p.group_units;
+    units = wave < 0 ? 0 : p.group_units;  // (wave -1: no list)
     info = as_constant(p.wave_info) + (int64_t)blockIdx.x * units * kScoreInfoWords;
     lane = lane_;
     taken = &counter;
@@ -182,10 +182,10 @@ struct TileStream {
     --left;
     return *cur++;
   }
-  static __device__ __forceinline__ bool ended(uint64_t e) {
-    return ((e >> kTileLastShift) & 3) == 2;  // empty, and no target's last tile
-  }
 };
+__device__ __forceinline__ bool tiles_ended(uint64_t e) {
+  return ((e >> kTileLastShift) & 3) == 2;  // empty, and no target's last tile
+}
 
 // 32 sign bits of one lane (dims 32g .. 32g + 31, bit b = dim 32g + b; set =
 // +1) as the fp4 (e2m1) operand of v_mfma_scale_f32_16x16x128_f8f6f4: dword
