@@ -192,8 +192,10 @@ void quantize_int8q(msim_int4_docs* h, const float* d_query, int64_t batch, int6
   const int64_t rows_padded = ((rows + 15) / 16) * 16 + 128;
   // The scan (query_tokens <= 128) reads the codes in lane order, one region
   // per pass; the row-pass kernel in row order.
-  const int64_t pass_rows = query_tokens <= 128 ? scan_pass_rows(query_tokens) : 0;
+  const int64_t pass_rows =
+      query_tokens > 0 && query_tokens <= kScanPassRows ? scan_pass_batch(rows / query_tokens, query_tokens) * query_tokens : 0;
   h->qpack.ensure(std::max<int64_t>(rows_padded * 128, scan_qpack_bytes(rows, pass_rows)), "hipMalloc int8q query codes");
+  h->quantized_pass_rows = pass_rows;
   h->qscale.ensure(rows_padded * 4, "hipMalloc int8q query scales");
   h->qbias.ensure(rows_padded * 4, "hipMalloc int8q query bias");
   check_hip(launch_quantize_int8(d_query, rows, rows_padded, h->qpack.as<int8_t>(),
@@ -380,10 +382,16 @@ void score_quantized(msim_int4_docs* h, int64_t batch, int64_t query_tokens, flo
     a.epoch = h->tail_epoch.as<uint32_t>();
     a.tail_wait_ticks = g_fused_wait_ticks;
   }
-  const int64_t per_pass = std::max<int64_t>(1, kScanPassRows / query_tokens);
-  for (int64_t b0 = 0; b0 < batch; b0 += per_pass) {
-    const int64_t nb = std::min(per_pass, batch - b0);
-    a.qpack = h->qpack.as<int8_t>() + (b0 / per_pass) * scan_qpack_bytes(per_pass * query_tokens, per_pass * query_tokens);
+  // Every pass in one launch (one grid row each), or one fused launch per pass.
+  const int64_t per_pass = h->quantized_pass_rows / query_tokens;
+  if (per_pass < 1 || per_pass * query_tokens != h->quantized_pass_rows)
+    throw InvalidArgument("no quantised query of this shape: call quantize first with the same batch and query_tokens");
+  const int64_t per_launch = k > 0 ? per_pass : per_pass * kScanMaxPasses;
+  a.pass_batch = (int32_t)per_pass;
+  a.qpack_pass_stride = scan_qpack_bytes(per_pass * query_tokens, per_pass * query_tokens);
+  for (int64_t b0 = 0; b0 < batch; b0 += per_launch) {
+    const int64_t nb = std::min(per_launch, batch - b0);
+    a.qpack = h->qpack.as<int8_t>() + (b0 / per_pass) * a.qpack_pass_stride;
     a.qscale = h->qscale.as<float>() + b0 * query_tokens;
     a.batch = (int32_t)nb;
     a.scores = k > 0 ? nullptr : d_scores + b0 * a.score_stride;

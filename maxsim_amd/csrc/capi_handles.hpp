@@ -114,6 +114,7 @@ struct msim_int4_docs {
   bool token_scales_fma = false;  // every token scale in [kScanFmaMinScale, kScanFmaMaxScale)
   bool has_residual = false;
   int64_t quantized_rows = -1;  // rows of the query currently quantised in qpack
+  int64_t quantized_pass_rows = 0;     // query rows per scan pass of the quantised codes (0: row order)
   int64_t max_doc_tiles = 1;    // 16-token tiles of the longest document
   std::vector<int64_t> host_offsets;
   int64_t partition_waves = 0;    // wave count the cached scan table was built for

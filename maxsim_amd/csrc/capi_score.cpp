@@ -1120,9 +1120,11 @@ bool binres_scan_prefix(msim_binary_docs* h, const float* d_query, int64_t batch
   a.scale = 1.0;
   a.score_stride = h->num_docs;
   a.num_docs = h->num_docs;
-  const int64_t per_pass = std::max<int64_t>(1, kScanPassRows / query_tokens);
-  for (int64_t b0 = 0; b0 < batch; b0 += per_pass) {
-    const int64_t nb = std::min(per_pass, batch - b0), row0 = b0 * query_tokens;
+  const int64_t per_pass = scan_pass_batch(batch, query_tokens), per_launch = per_pass * kScanMaxPasses;
+  a.pass_batch = (int32_t)per_pass;
+  a.qpack_pass_stride = per_pass * query_tokens * 128;
+  for (int64_t b0 = 0; b0 < batch; b0 += per_launch) {
+    const int64_t nb = std::min(per_launch, batch - b0), row0 = b0 * query_tokens;
     a.qpack = ws.qpack.as<int8_t>() + row0 * 128;
     a.qscale = ws.colmul.as<float>() + row0;
     a.qsum = ws.qsum.as<int32_t>() + row0;

@@ -161,6 +161,17 @@ __global__ __launch_bounds__(kScanThreads) MSIM_SCAN_OCCUPANCY void int8q_scan_k
     const uint64_t* __restrict__ tile_table, const int8_t* __restrict__ qpack,
     const float* __restrict__ qscale, float* __restrict__ scores) {
   constexpr bool kTS = EPI != kScanEpiIntMax;
+  // The pass of this grid row (a fused launch has one).
+  int batch = p.batch;
+  const int32_t* qsum = p.qsum;
+  if constexpr (!kTail) {
+    const int64_t b0 = (int64_t)blockIdx.y * p.pass_batch;
+    batch = min(p.pass_batch, (int)(p.batch - b0));
+    qpack += (int64_t)blockIdx.y * p.qpack_pass_stride;
+    qscale += b0 * p.query_tokens;
+    scores += b0 * p.score_stride;
+    if constexpr (kSign) qsum += b0 * p.query_tokens;
+  }
   // LDS: the workgroup's copy of the query tiles; per wave the tile ring
   // (codes as 64 lanes x 16 B, token scales as 64 lanes x 4 B per slot), the
   // per-row maxima of the document being finished and the query scales.
@@ -242,7 +253,7 @@ __global__ __launch_bounds__(kScanThreads) MSIM_SCAN_OCCUPANCY void int8q_scan_k
     if (fused) lds_load_b32(make_rsrc_words(p.epoch, 24u), 4u * (uint32_t)lane, wave_uniform((int)lds_address(rowmax)));
     // Sign documents: the query rows' code sums into the row-maxima buffer.
     if (kSign) {
-      const v4i rsum = make_rsrc_words(p.qsum, (uint32_t)(16 * NT * 4));
+      const v4i rsum = make_rsrc_words(qsum, (uint32_t)(16 * NT * 4));
       const uint32_t rm_lds = wave_uniform((int)lds_address(rowmax));
       lds_load_b32(rsum, 4u * (uint32_t)lane, rm_lds);
       lds_load_b32(rsum, 4u * (uint32_t)(lane + kWave), rm_lds + 4 * kWave);
@@ -475,7 +486,7 @@ __global__ __launch_bounds__(kScanThreads) MSIM_SCAN_OCCUPANCY void int8q_scan_k
       r = __dadd_rn(r, dpp_f64<0xB1>(r));   // quad_perm [1,0,3,2]
       r = __dadd_rn(r, dpp_f64<0x4E>(r));   // quad_perm [2,3,0,1]
       r = __dadd_rn(r, dpp_f64<0x141>(r));  // row_half_mirror
-      if (c == 0 && g < p.batch) emit(g, d0 + local, pos0 + nempty + nfin, (float)(r * p.scale));
+      if (c == 0 && g < batch) emit(g, d0 + local, pos0 + nempty + nfin, (float)(r * p.scale));
     } else {
 #pragma unroll
       for (int j = 0; j < NT; ++j) mf[j] = unfold(max_over_groups(mf[j]));
@@ -484,7 +495,7 @@ __global__ __launch_bounds__(kScanThreads) MSIM_SCAN_OCCUPANCY void int8q_scan_k
         for (int j = 0; j < NT; ++j) rowmax[16 * j + c] = mf[j];
       }
       wave_sync_lds();
-      scan_finish_doc(rowmax, qs, p.batch, p.query_tokens, p.scale,
+      scan_finish_doc(rowmax, qs, batch, p.query_tokens, p.scale,
                       [&](int b, float v) { emit(b, d0 + local, pos0 + nempty + nfin, v); });
       wave_sync_lds();
     }
@@ -594,12 +605,12 @@ __global__ __launch_bounds__(kScanThreads) MSIM_SCAN_OCCUPANCY void int8q_scan_k
   // entries) are the only ones that can enter its top three.
   for (int e = lane; e < nempty; e += kWave) {
     const int64_t doc = wave_info_ptr[p.num_waves * kWaveInfoWords + e0 + e];
-    for (int b = 0; b < p.batch; ++b) emit(b, doc, pos0 + e, 0.0f, false);
+    for (int b = 0; b < batch; ++b) emit(b, doc, pos0 + e, 0.0f, false);
   }
   if (fused && lane == 0) {
     for (int e = 0; e < min(nempty, 3); ++e) {
       const int64_t doc = wave_info_ptr[p.num_waves * kWaveInfoWords + e0 + e];
-      for (int b = 0; b < p.batch; ++b) emit(b, doc, pos0 + e, 0.0f);
+      for (int b = 0; b < batch; ++b) emit(b, doc, pos0 + e, 0.0f);
     }
   }
   if constexpr (!fused) return;
@@ -681,7 +692,8 @@ __global__ __launch_bounds__(kScanThreads) MSIM_SCAN_OCCUPANCY void int8q_scan_k
 
 template <int EPI, bool kTail, bool kSign>
 static void launch_scan_nt(const ScanArgs& a, int nt, int64_t blocks, hipStream_t stream) {
-  const dim3 grid((unsigned)blocks), block(kScanThreads);
+  const int passes = (a.batch + a.pass_batch - 1) / a.pass_batch;
+  const dim3 grid((unsigned)blocks, (unsigned)passes), block(kScanThreads);
   switch (nt) {
 #define MSIM_SCAN_CASE(N)                                                                                   \
   int8q_scan_kernel<N, EPI, kTail, kSign><<<grid, block, 0, stream>>>(a, a.codes, a.token_scale16, a.offsets, \
@@ -706,8 +718,12 @@ static void launch_scan_epi(const ScanArgs& a, int nt, int64_t blocks, bool tail
 }
 
 hipError_t launch_int8q_scan(const ScanArgs& args, int epilogue, hipStream_t stream) {
-  const int rows = args.batch * args.query_tokens;
-  if (rows <= 0 || rows > 128 || args.num_waves <= 0 || args.num_waves % kScanWaves != 0)
+  if (args.batch <= 0 || args.pass_batch <= 0 || args.query_tokens <= 0 || args.query_tokens > kScanPassRows ||
+      (int64_t)args.pass_batch * args.query_tokens > kScanPassRows || args.batch > args.pass_batch * kScanMaxPasses ||
+      (args.topk_k > 0 && args.batch > args.pass_batch))
+    return hipErrorInvalidValue;
+  const int rows = std::min(args.batch, args.pass_batch) * args.query_tokens;
+  if ( args.num_waves <= 0 || args.num_waves % kScanWaves != 0)
     return hipErrorInvalidValue;
   if (epilogue != kScanEpiIntMax && epilogue != kScanEpiFma && epilogue != kScanEpiCvt) return hipErrorInvalidValue;
   if ((epilogue == kScanEpiIntMax) != (args.token_scale16 == nullptr)) return hipErrorInvalidValue;

@@ -89,14 +89,14 @@ struct ScanArgs {
   const uint64_t* tile_table;   // per-wave tile entries, wave w's at w * tile_stride
   int64_t tile_stride;
   int64_t num_waves;            // a multiple of kScanWavesPerGroup
-  const int8_t* qpack;          // >= rows + 128 rows of MFMA B-order int8 codes (zero past rows)
+  const int8_t* qpack;          // MFMA B-order int8 codes, 128 readable rows past the last pass's start
   int32_t q_row_order;          // qpack rows of 128 bytes (quantize_limbs) instead of the scan's lane order
   int32_t doc_sign;             // sign documents: codes 16 bytes per token (32 sign bits per lane group,
                                 //   bit b = dim 32g + b), token_scale16 the per-token scales themselves,
                                 //   qpack in the sign layout of quantize_limbs
   const int32_t* qsum;          // sign documents: per query row the sum of its int8 codes
   const float* qscale;          // per-row query scale, same row count
-  int32_t batch;                // batch rows of this pass (batch * query_tokens <= 128)
+  int32_t batch;                // batch rows
   int32_t query_tokens;
   double scale;                 // tensor scale (1.0 for per-token corpora)
   float* scores;                // [batch, score_stride] (not used by a fused launch)
@@ -128,6 +128,9 @@ struct ScanArgs {
   uint64_t* tail_rec;
   const int64_t* block_pos;
   int64_t tail_key_words;       // u64 words of the tail_keys allocation (>= batch * kScanTailRow)
+  int32_t pass_batch;           // batch rows per pass (times query_tokens <= 128), one pass per grid row;
+                                //   a fused launch has one pass
+  int64_t qpack_pass_stride;    // bytes between the passes' query codes
 };
 constexpr int kScanTailMaxK = 32;
 constexpr int64_t kScanTailMaxDocs = 4096;
@@ -153,11 +156,22 @@ constexpr uint64_t kScanTailKeyPeriod = (1u << 19) - 1u;
 enum : int { kScanEpiIntMax = 0, kScanEpiFma = 1, kScanEpiCvt = 2 };
 constexpr float kScanFmaMinScale = 0x1p-122f, kScanFmaMaxScale = 0x1p109f;
 hipError_t launch_int8q_scan(const ScanArgs& args, int epilogue, hipStream_t stream);
-// Query rows of one scan launch: whole batch rows, at most 128 rows (one
+// Query rows of one scan pass: whole batch rows, at most 128 rows (one
 // batch row of more than 128 tokens goes to the row-pass kernel instead).
 constexpr int64_t kScanPassRows = 128;
+constexpr int64_t kScanMaxPasses = 32768;  // grid rows of one launch
 inline int64_t scan_pass_rows(int64_t query_tokens) {
   return query_tokens <= 0 ? 0 : (query_tokens >= kScanPassRows ? 1 : kScanPassRows / query_tokens) * query_tokens;
+}
+// Batch rows per pass of a call, spread evenly over its passes, which share one
+// launch (a grid row each): a pass's start and end, about 5 us of idle CUs, are
+// paid once (7 queries of 21 tokens over 3,001 documents: 126 and 21 rows in
+// two launches 13.8 + 7.8 us; 84 and 63 rows in one launch, the call 23.2 ->
+// 21.5 us).
+inline int64_t scan_pass_batch(int64_t batch, int64_t query_tokens) {
+  const int64_t most = query_tokens >= kScanPassRows || query_tokens <= 0 ? 1 : kScanPassRows / query_tokens;
+  const int64_t passes = (batch + most - 1) / most;
+  return passes <= 1 ? (batch < 1 ? 1 : batch) : (batch + passes - 1) / passes;
 }
 // Builds the wave table and tile table for `waves` requested waves (the
 // result may hold more rows: ranges are split at kScanMaxDocsPerWave

@@ -99,7 +99,7 @@ extern "C" int msim_int4_topk_int8q_noalloc(msim_int4_docs* h, const float* d_qu
     scan_corpus_args(h, query_tokens, a);
     a.qpack = qpack;
     a.qscale = qscale;
-    a.batch = (int32_t)batch;
+    a.batch = a.pass_batch = (int32_t)batch;
     if (fused) {
       a.tail_keys = reinterpret_cast<uint64_t*>(base + kKeysOff);
       a.tail_rec = reinterpret_cast<uint64_t*>(base + kRecOff);
