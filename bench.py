@@ -819,8 +819,8 @@ def bench_config5(args):
     full_wall, _ = _timed(full, args.steps, args.warmup, stream)
     got, exp = ti.cpu().numpy(), fi.cpu().numpy()
     overlap = recall(got, exp)
-    # The same cascade with the rescoring pass on the fp32 query (three int8
-    # limbs), against the fused scan of every document on the fp32 query.
+    # The same cascade with the rescoring pass on the fp32 query,
+    # against the fused scan of every document on the fp32 query.
     h.set_rescore_limbs(3)
     fp32_wall, _ = _timed(step, args.steps, args.warmup, stream)
     fp32_full_wall, _ = _timed(full, args.steps, args.warmup, stream)
