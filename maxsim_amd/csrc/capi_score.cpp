@@ -1066,6 +1066,7 @@ DocStreams binres_streams(msim_binary_docs* h, bool fused, int limbs) {
   s.tmul = 1.0f;
   if (fused) {
     s.residual = true;
+    if (limbs == 3) select_device(h->device);  // fp6_rows may allocate
     s.rcodes = limbs == 3 ? fp6_rows(h->residual6, h->residual_packed.as<uint8_t>(), h->num_tokens, h->dim)
                           : h->residual_packed.as<uint8_t>();
     s.rtscale = h->residual_token_scales16.as<float>();
