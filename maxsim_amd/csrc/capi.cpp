@@ -23,7 +23,10 @@ uint64_t g_fused_wait_ticks = kScanTailWaitTicks;  // msim_set_fused_wait_ticks
 void set_error(const std::string& msg) { g_last_error = msg; }
 
 void check_hip(hipError_t e, const char* what) {
-  if (e != hipSuccess) throw RuntimeError(std::string(what) + ": " + hipGetErrorString(e));
+  if (e == hipSuccess) return;
+  const std::string msg = std::string(what) + ": " + hipGetErrorString(e);
+  if (e == hipErrorOutOfMemory) throw OutOfDeviceMemory(msg);
+  throw RuntimeError(msg);
 }
 
 DeviceBuffer::~DeviceBuffer() {

@@ -8,16 +8,28 @@
 
 namespace msim {
 
+// Whole-corpus tables of one work split, on the device: written and waited
+// for before their first use and never rewritten, so that a launch queued on
+// any stream may still be reading them when a call of another split is made.
+struct ScoreTable {
+  int64_t key = 0;      // waves (build_score_tables), or -2 - workgroups (build_score_units)
+  int64_t waves = 0;    // records
+  int64_t units = 0;    // records per workgroup (build_score_units), else 0
+  bool captured = false;  // a captured graph reads it: kept as long as the handle
+  DeviceBuffer info, tiles;
+};
+// Tables kept per handle, most recently used first (half a byte per token
+// each); dropping one frees its memory, for which hipFree waits until the
+// device is idle.
+constexpr size_t kScoreTablesKept = 8;
+
 // Device workspaces of one handle's generalized scoring calls (grow
 // monotonically, freed with the handle; cu:3057-3067).
 struct ScoreWorkspace {
   DeviceBuffer qpack, colmul, qsum, weights, pooled, qbits;
   DeviceBuffer qpack_alt;  // the query also in the int4 layout (QueryInput::alt_int4)
   std::vector<float> weights_host;  // what `weights` holds (a repeated weight vector is not copied again)
-  DeviceBuffer full_info, full_tiles;  // cached whole-corpus tables
-  int64_t full_key = -1;               // waves the cached tables were built for (work units: -2 - workgroups)
-  int64_t full_waves = 0;              // records in the cached table
-  int64_t full_units = 0;              // records per workgroup (work-unit tables), else 0
+  std::vector<std::unique_ptr<ScoreTable>> tables;  // whole-corpus tables, most recently used first
   DeviceBuffer cand_ids, cand_info, cand_tiles;
   // cascade: coarse scores, top-M candidates (scores / ids), fine scores
   DeviceBuffer coarse, top_m_scores, top_m_ids, fine;
@@ -26,9 +38,11 @@ struct ScoreWorkspace {
   // memory that the kernels read and write directly.
   HostBuffer host_query, host_out, host_ids;
   uint64_t bytes() const {
-    return qpack.cap + qpack_alt.cap + colmul.cap + qsum.cap + weights.cap + pooled.cap + qbits.cap + full_info.cap +
-           full_tiles.cap + cand_ids.cap + cand_info.cap + cand_tiles.cap + coarse.cap + top_m_scores.cap +
-           top_m_ids.cap + fine.cap + topk_scratch.cap;
+    uint64_t table_bytes = 0;
+    for (const auto& t : tables) table_bytes += t->info.cap + t->tiles.cap;
+    return qpack.cap + qpack_alt.cap + colmul.cap + qsum.cap + weights.cap + pooled.cap + qbits.cap + table_bytes +
+           cand_ids.cap + cand_info.cap + cand_tiles.cap + coarse.cap + top_m_scores.cap + top_m_ids.cap + fine.cap +
+           topk_scratch.cap;
   }
 };
 

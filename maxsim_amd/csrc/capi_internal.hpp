@@ -20,6 +20,9 @@ struct InvalidArgument : std::runtime_error {
 struct RuntimeError : std::runtime_error {
   using std::runtime_error::runtime_error;
 };
+struct OutOfDeviceMemory : RuntimeError {
+  using RuntimeError::RuntimeError;
+};
 struct NotSupported : std::runtime_error {
   using std::runtime_error::runtime_error;
 };

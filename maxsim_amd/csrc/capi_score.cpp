@@ -26,11 +26,11 @@ T* upload_vec(DeviceBuffer& buf, const std::vector<T>& v, const char* what) {
   return buf.as<T>();
 }
 
-// The same, enqueued on `stream`: a per-call table (weights, candidate
-// tables) is overwritten only after the kernels queued before it on that
-// stream, which may still read the previous call's contents.  From pageable
-// host memory the runtime stages or copies before returning, so `v` may go
-// out of scope afterwards.
+// The same, enqueued on `stream`: what a call may rewrite (the reducer weights)
+// is overwritten only after the kernels queued before it on that stream, which
+// may still read the previous call's contents.  From pageable host memory the
+// runtime stages or copies before returning, so `v` may go out of scope
+// afterwards.
 template <typename T>
 T* upload_vec(DeviceBuffer& buf, const std::vector<T>& v, const char* what, hipStream_t stream) {
   buf.ensure(std::max<size_t>(sizeof(T) * v.size(), sizeof(T)), what);
@@ -105,25 +105,64 @@ void set_streams(ScoreArgs& a, const DocStreams& s) {
   a.unit_tscale = s.unit_tscale;
 }
 
+// Drops the least recently used tables that no captured graph reads until at
+// most `keep` are left.
+void drop_tables(ScoreWorkspace& ws, size_t keep) {
+  for (size_t i = ws.tables.size(); i-- > 0 && ws.tables.size() > keep;)
+    if (!ws.tables[i]->captured) ws.tables.erase(ws.tables.begin() + (int64_t)i);
+}
+
+// The whole-corpus table of `key`; build(info, tiles) makes it, returning the
+// records per workgroup (or 0), at the first call that asks for it.
+template <typename Build>
+const ScoreTable& corpus_table(ScoreWorkspace& ws, int64_t key, hipStream_t stream, Build build) {
+  auto& tables = ws.tables;
+  size_t at = 0;
+  while (at < tables.size() && tables[at]->key != key) ++at;
+  if (at == tables.size()) {
+    auto t = std::make_unique<ScoreTable>();
+    std::vector<int64_t> info;
+    std::vector<uint64_t> tiles;
+    t->key = key;
+    t->units = build(info, tiles);
+    t->waves = (int64_t)info.size() / kScoreInfoWords;
+    drop_tables(ws, kScoreTablesKept - 1);
+    auto upload = [&] {
+      upload_vec(t->info, info, "copy score wave table to device");
+      upload_vec(t->tiles, tiles, "copy score tile table to device");
+      check_hip(hipStreamSynchronize(nullptr), "synchronize score tables");
+    };
+    try {
+      upload();
+    } catch (const OutOfDeviceMemory&) {
+      (void)hipGetLastError();  // (a later launch would report it)
+      drop_tables(ws, 0);       // the other tables make room
+      upload();
+    }
+    tables.push_back(std::move(t));
+    at = tables.size() - 1;
+  }
+  std::rotate(tables.begin(), tables.begin() + (int64_t)at, tables.begin() + (int64_t)at + 1);
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (stream != nullptr && hipStreamIsCapturing(stream, &capture) == hipSuccess &&
+      capture != hipStreamCaptureStatusNone)
+    tables[0]->captured = true;
+  return *tables[0];
+}
+
 // Every document as work units for `workgroups` workgroups at once: a list per
 // workgroup and pass; few documents are spread over as many workgroups.
 void set_units(ScoreWorkspace& ws, const std::vector<int64_t>& off, int64_t workgroups, int64_t subs, int64_t min_tiles,
-               ScoreArgs& a) {
+               ScoreArgs& a, hipStream_t stream) {
   const int64_t num_docs = (int64_t)off.size() - 1;
   const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(workgroups / subs, num_docs));
-  if (ws.full_key != -2 - wgs) {
-    std::vector<int64_t> info;
-    std::vector<uint64_t> tiles;
-    ws.full_units = build_score_units(off.data(), nullptr, num_docs, wgs, info, tiles, min_tiles);
-    upload_vec(ws.full_info, info, "copy score wave table to device");
-    upload_vec(ws.full_tiles, tiles, "copy score tile table to device");
-    ws.full_key = -2 - wgs;
-    ws.full_waves = (int64_t)info.size() / kScoreInfoWords;
-  }
-  a.wave_info = ws.full_info.as<int64_t>();
-  a.tiles = ws.full_tiles.as<uint64_t>();
-  a.num_waves = ws.full_waves;
-  a.group_units = (int32_t)ws.full_units;
+  const ScoreTable& t = corpus_table(ws, -2 - wgs, stream, [&](auto& info, auto& tiles) {
+    return build_score_units(off.data(), nullptr, num_docs, wgs, info, tiles, min_tiles);
+  });
+  a.wave_info = t.info.as<int64_t>();
+  a.tiles = t.tiles.as<uint64_t>();
+  a.num_waves = t.waves;
+  a.group_units = (int32_t)t.units;
 }
 
 // Sign-bit queries against every sign document (MaxSim, unit token scales).
@@ -134,7 +173,7 @@ void run_hamming_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, cons
   const HammingPlan plan = hamming_plan(batch, query_tokens);
   ScoreArgs a{};
   set_streams(a, s);
-  set_units(ws, off, 2 * device_cu_count(), plan.subs, kDigitUnitSign, a);
+  set_units(ws, off, 2 * device_cu_count(), plan.subs, kDigitUnitSign, a, stream);
   a.qbits = d_qbits;
   a.subs = (int32_t)plan.subs;
   a.pass_rows = (int32_t)plan.pass_rows;
@@ -193,7 +232,8 @@ void run_digit_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, const 
     a.direct_offsets = t.d_offsets;
     a.direct_count = targets;
   } else {
-    set_units(ws, off, device_cu_count(), plan.subs, s.doc == kDocSign ? kDigitUnitSign : kDigitUnitInt4, a);
+    set_units(ws, off, device_cu_count(), plan.subs, s.doc == kDocSign ? kDigitUnitSign : kDigitUnitInt4, a,
+              stream);
   }
   a.qpack = ws.qpack.as<int8_t>();
   a.rows_padded = rows_padded;
@@ -325,19 +365,13 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
       a.info_grp_stride = w4 * kScoreInfoWords;
     }
   } else {
-    if (ws.full_key != waves) {
-      std::vector<int64_t> info;
-      std::vector<uint64_t> tiles;
+    const ScoreTable& tab = corpus_table(ws, waves, stream, [&](auto& info, auto& tiles) -> int64_t {
       build_score_tables(off.data(), nullptr, num_docs, waves, info, tiles);
-      upload_vec(ws.full_info, info, "copy score wave table to device");
-      upload_vec(ws.full_tiles, tiles, "copy score tile table to device");
-      ws.full_key = waves;
-      ws.full_units = 0;
-      ws.full_waves = (int64_t)info.size() / kScoreInfoWords;
-    }
-    a.wave_info = ws.full_info.as<int64_t>();
-    a.tiles = ws.full_tiles.as<uint64_t>();
-    a.num_waves = ws.full_waves;
+      return 0;
+    });
+    a.wave_info = tab.info.as<int64_t>();
+    a.tiles = tab.tiles.as<uint64_t>();
+    a.num_waves = tab.waves;
     a.info_grp_stride = 0;
   }
 

@@ -420,6 +420,85 @@ def test_score_async_weights_ordered_on_side_stream(gpu):
         np.testing.assert_array_equal(out.cpu().numpy(), h.score_batch(query, "weighted_maxsim", w))
 
 
+def test_async_calls_of_changing_batch_on_a_side_stream(gpu):
+    """Back-to-back async calls on a non-blocking stream whose batches need
+    different work splits, more of them than a handle keeps tables for: each
+    output equals the synchronous call's."""
+    import torch
+
+    from maxsim_amd import _maxsim_hip, synthetic
+    from maxsim_amd._native import check, ptr
+
+    corpus = synthetic.make_corpus(3000, 16, 64, seed=93)
+    offsets, n, k = corpus.offsets, 3000, 10
+    _, h = _int4_handle(corpus.embeddings, offsets, "token")
+    rng = np.random.default_rng(94)
+    signs = _maxsim_hip.CudaPackedDocs(rng.integers(0, 256, (int(offsets[-1]), 16), dtype=np.uint8), offsets, 128)
+    signs.set_token_scale_vector(rng.uniform(0.5, 1.5, int(offsets[-1])).astype(np.float32))
+    signs.set_residual_int4(rng.integers(0, 256, (int(offsets[-1]), 64), dtype=np.uint8), 1.0,
+                            rng.uniform(0.01, 0.02, int(offsets[-1])).astype(np.float32))
+    signs.set_rescore_limbs(3)
+    batches = [2, 16, 4, 40, 6, 64, 8, 10, 2, 12, 14, 20, 64, 2]
+    queries = [rng.standard_normal((b, 32, 128)).astype(np.float32) for b in batches]
+    bits = [rng.integers(0, 256, (8 * b, 32, 16), dtype=np.uint8) for b in batches]
+    side = torch.cuda.Stream()
+    sptr = _maxsim_hip._stream_ptr(side)
+    runs = []
+    for query, qb in zip(queries, bits):
+        b, b8 = len(query), len(qb)
+        runs.append((torch.from_numpy(query).cuda(), torch.from_numpy(qb).cuda(), torch.empty((b, n), device="cuda"),
+                     torch.empty((b8, k), device="cuda"), torch.empty((b8, k), dtype=torch.int64, device="cuda"),
+                     torch.empty((b, k), device="cuda"), torch.empty((b, k), dtype=torch.int64, device="cuda")))
+    torch.cuda.synchronize()
+    for dq, dqb, out, hs, hi, cs, ci in runs:
+        check(h._lib.msim_int4_score_async(h._h, ptr(dq), dq.shape[0], 32, b"maxsim", None, 0, 0, 0, 1.0, 0, ptr(out),
+                                           sptr))
+        signs.topk_hamming_async(dqb, k, hs, hi, side)
+        signs.cascade_topk_async(dq, k, n, cs, ci, side)
+    side.synchronize()
+    for query, qb, (_, _, out, hs, hi, cs, ci) in zip(queries, bits, runs):
+        np.testing.assert_array_equal(out.cpu().numpy(), h.score_batch(query, "maxsim"))
+        for got_s, got_i, (exp_s, exp_i) in ((hs, hi, signs.topk_hamming(qb, k)),
+                                             (cs, ci, signs.binres_topk_batch(query, k))):
+            np.testing.assert_array_equal(got_s.cpu().numpy(), exp_s)
+            np.testing.assert_array_equal(got_i.cpu().numpy(), exp_i)
+
+
+def test_captured_call_keeps_its_tables(gpu):
+    """A captured sign-query search replays right after more calls of other
+    work splits (of smaller batches: the workspaces do not grow) than a handle
+    keeps tables for."""
+    import torch
+
+    from maxsim_amd import _maxsim_hip
+
+    rng = np.random.default_rng(95)
+    offsets = np.concatenate(([0], np.cumsum(rng.integers(1, 60, 2000)))).astype(np.int64)
+    h = _maxsim_hip.CudaPackedDocs(rng.integers(0, 256, (int(offsets[-1]), 16), dtype=np.uint8), offsets, 128)
+    bits = rng.integers(0, 256, (3, 128, 32, 16), dtype=np.uint8)
+    exp = [h.topk_hamming(b, 10) for b in bits]
+    static = torch.from_numpy(bits[0]).cuda()
+    scores = torch.empty((128, 10), device="cuda")
+    ids = torch.empty((128, 10), dtype=torch.int64, device="cuda")
+    side = torch.cuda.Stream()
+    h.topk_hamming_async(static, 10, scores, ids, side)
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        h.topk_hamming_async(static, 10, scores, ids, torch.cuda.current_stream())
+    for replay in range(6):
+        for b in range(8, 120, 9):
+            got_s, got_i = h.topk_hamming(bits[1][:b], 10)
+            np.testing.assert_array_equal(got_s, exp[1][0][:b])
+            np.testing.assert_array_equal(got_i, exp[1][1][:b])
+        static.copy_(torch.from_numpy(bits[replay % 3]))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(scores.cpu().numpy(), exp[replay % 3][0])
+        np.testing.assert_array_equal(ids.cpu().numpy(), exp[replay % 3][1])
+
+
 def test_maxsim_cuda_free_functions_match_reference_lut(gpu, oracle):
     """maxsim_cuda / maxsim_cuda_batch (cuda_extension.cu:3308-3412), the
     handle module's free functions the reference's _score_binary calls for
