@@ -12,15 +12,16 @@ namespace msim {
 // for before their first use and never rewritten, so that a launch queued on
 // any stream may still be reading them when a call of another split is made.
 struct ScoreTable {
-  int64_t key = 0;      // waves (build_score_tables), or -2 - workgroups (build_score_units)
-  int64_t waves = 0;    // records
-  int64_t units = 0;    // records per workgroup (build_score_units), else 0
+  int64_t first = 0;      // its first document
+  int64_t split = 0;      // waves (build_score_tables), or -2 - workgroups (build_score_units)
+  int64_t waves = 0;      // records
+  int64_t units = 0;      // records per workgroup (build_score_units), else 0
   bool captured = false;  // a captured graph reads it: kept as long as the handle
   DeviceBuffer info, tiles;
 };
-// Tables kept per handle, most recently used first (half a byte per token
-// each); dropping one frees its memory, for which hipFree waits until the
-// device is idle.
+// Work splits whose tables a handle keeps (half a byte per token each);
+// dropping a table frees its memory, for which hipFree waits until the device
+// is idle.
 constexpr size_t kScoreTablesKept = 8;
 
 // Device workspaces of one handle's generalized scoring calls (grow

@@ -112,21 +112,28 @@ void drop_tables(ScoreWorkspace& ws, size_t keep) {
     if (!ws.tables[i]->captured) ws.tables.erase(ws.tables.begin() + (int64_t)i);
 }
 
-// The whole-corpus table of `key`; build(info, tiles) makes it, returning the
-// records per workgroup (or 0), at the first call that asks for it.
+// Documents one launch of work units covers (a tile entry holds 24 bits of
+// target index): larger corpora are scored range by range.
+int64_t doc_ranges(int64_t num_docs) { return ceil_div(num_docs, kScoreMaxUnitTargets); }
+
+// The table of `split` over the documents from `first` on; build(info, tiles)
+// makes it, returning the records per workgroup (or 0), at the first call that
+// asks for it.  `ranges`: tables a call of one split uses.
 template <typename Build>
-const ScoreTable& corpus_table(ScoreWorkspace& ws, int64_t key, hipStream_t stream, Build build) {
+const ScoreTable& corpus_table(ScoreWorkspace& ws, int64_t first, int64_t split, int64_t ranges, hipStream_t stream,
+                               Build build) {
   auto& tables = ws.tables;
   size_t at = 0;
-  while (at < tables.size() && tables[at]->key != key) ++at;
+  while (at < tables.size() && (tables[at]->first != first || tables[at]->split != split)) ++at;
   if (at == tables.size()) {
     auto t = std::make_unique<ScoreTable>();
     std::vector<int64_t> info;
     std::vector<uint64_t> tiles;
-    t->key = key;
+    t->first = first;
+    t->split = split;
     t->units = build(info, tiles);
     t->waves = (int64_t)info.size() / kScoreInfoWords;
-    drop_tables(ws, kScoreTablesKept - 1);
+    drop_tables(ws, kScoreTablesKept * (size_t)ranges - 1);
     auto upload = [&] {
       upload_vec(t->info, info, "copy score wave table to device");
       upload_vec(t->tiles, tiles, "copy score tile table to device");
@@ -150,15 +157,16 @@ const ScoreTable& corpus_table(ScoreWorkspace& ws, int64_t key, hipStream_t stre
   return *tables[0];
 }
 
-// Every document as work units for `workgroups` workgroups at once: a list per
-// workgroup and pass; few documents are spread over as many workgroups.
-void set_units(ScoreWorkspace& ws, const std::vector<int64_t>& off, int64_t workgroups, int64_t subs, int64_t min_tiles,
-               ScoreArgs& a, hipStream_t stream) {
-  const int64_t num_docs = (int64_t)off.size() - 1;
-  const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(workgroups / subs, num_docs));
-  const ScoreTable& t = corpus_table(ws, -2 - wgs, stream, [&](auto& info, auto& tiles) {
-    return build_score_units(off.data(), nullptr, num_docs, wgs, info, tiles, min_tiles);
-  });
+// Documents first .. first + count - 1 as work units for `workgroups`
+// workgroups at once: a list per workgroup and pass; few documents are spread
+// over as many workgroups.
+void set_units(ScoreWorkspace& ws, const std::vector<int64_t>& off, int64_t first, int64_t count, int64_t workgroups,
+               int64_t subs, int64_t min_tiles, ScoreArgs& a, hipStream_t stream) {
+  const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(workgroups / subs, count));
+  const ScoreTable& t =
+      corpus_table(ws, first, -2 - wgs, doc_ranges((int64_t)off.size() - 1), stream, [&](auto& info, auto& tiles) {
+        return build_score_units(off.data() + first, nullptr, count, wgs, info, tiles, min_tiles);
+      });
   a.wave_info = t.info.as<int64_t>();
   a.tiles = t.tiles.as<uint64_t>();
   a.num_waves = t.waves;
@@ -173,27 +181,32 @@ void run_hamming_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, cons
   const HammingPlan plan = hamming_plan(batch, query_tokens);
   ScoreArgs a{};
   set_streams(a, s);
-  set_units(ws, off, 2 * device_cu_count(), plan.subs, kDigitUnitSign, a, stream);
   a.qbits = d_qbits;
   a.subs = (int32_t)plan.subs;
   a.pass_rows = (int32_t)plan.pass_rows;
   a.grp_rows = (int32_t)rows;
   a.query_tokens = (int32_t)query_tokens;
   a.chunks = 1;
-  if (plan.whole) {
-    a.out = d_out;
-    a.out_stride = out_stride;
-    a.iout = d_iout;
-    a.iout_stride = num_docs;
+  for (int64_t first = 0; first < num_docs; first += kScoreMaxUnitTargets) {
+    const int64_t count = std::min(kScoreMaxUnitTargets, num_docs - first);
+    float* out = d_out ? d_out + first : nullptr;
+    int32_t* iout = d_iout ? d_iout + first : nullptr;
+    set_units(ws, off, first, count, 2 * device_cu_count(), plan.subs, kDigitUnitSign, a, stream);
+    if (plan.whole) {
+      a.out = out;
+      a.out_stride = out_stride;
+      a.iout = iout;
+      a.iout_stride = num_docs;
+      check_hip(launch_hamming(a, stream), "launch fp4 hamming kernel");
+      continue;
+    }
+    ws.pooled.ensure(sizeof(float) * count * rows, "hipMalloc pooled rows");
+    a.pooled = ws.pooled.as<float>();
     check_hip(launch_hamming(a, stream), "launch fp4 hamming kernel");
-    return;
+    check_hip(launch_pool_sum(ws.pooled.as<float>(), batch, query_tokens, count, query_tokens, rows, out, out_stride,
+                              iout, num_docs, stream),
+              "launch pooled sum kernel");
   }
-  ws.pooled.ensure(sizeof(float) * num_docs * rows, "hipMalloc pooled rows");
-  a.pooled = ws.pooled.as<float>();
-  check_hip(launch_hamming(a, stream), "launch fp4 hamming kernel");
-  check_hip(launch_pool_sum(ws.pooled.as<float>(), batch, query_tokens, num_docs, query_tokens, rows, d_out, out_stride,
-                            d_iout, stream),
-            "launch pooled sum kernel");
 }
 
 // fp32 queries: digits, then one launch over every document (work units) or
@@ -202,7 +215,6 @@ void run_digit_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, const 
                      int reducer, float temperature, int64_t batch, int64_t query_tokens, const float* h_row_weights,
                      const Targets& t, float* d_out, int64_t out_stride, hipStream_t stream) {
   const int64_t num_docs = (int64_t)off.size() - 1;
-  const int64_t targets = (t.host || t.device) ? t.count : num_docs;
   const int64_t rows = batch * query_tokens, rows_padded = ceil_div(rows, 16) * 16 + 128;
   const int64_t groups = t.per_row ? batch : 1;
   const DigitPlan plan = digit_plan(t.per_row ? 1 : batch, query_tokens, s.chunks);
@@ -223,18 +235,6 @@ void run_digit_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, const 
   ScoreArgs a{};
   set_streams(a, s);
   a.weights = row_weights_device(ws, h_row_weights, rows, rows_padded, stream);
-  if (t.host || t.device || num_docs >= kScoreMaxUnitTargets) {
-    // (Tile entries hold 24 bits of target index: more documents go one per
-    // wave.)
-    if (t.d_offsets == nullptr) throw InvalidArgument("candidate lists need the token offsets");
-    a.targets = t.device ? t.device : t.host ? ws.cand_ids.as<int64_t>() : nullptr;
-    a.targets_grp_stride = t.per_row ? t.count : 0;
-    a.direct_offsets = t.d_offsets;
-    a.direct_count = targets;
-  } else {
-    set_units(ws, off, device_cu_count(), plan.subs, s.doc == kDocSign ? kDigitUnitSign : kDigitUnitInt4, a,
-              stream);
-  }
   a.qpack = ws.qpack.as<int8_t>();
   a.rows_padded = rows_padded;
   a.colmul = ws.colmul.as<float>();
@@ -244,20 +244,39 @@ void run_digit_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, const 
   a.temperature = temperature;
   a.query_tokens = (int32_t)query_tokens;
   a.chunks = s.chunks;
-  if (plan.whole) {  // the kernel sums each batch row's tokens
-    a.out = d_out;
-    a.out_stride = out_stride;
+  // Scores of `count` targets into out.
+  auto score = [&](int64_t count, float* out) {
+    if (plan.whole) {  // the kernel sums each batch row's tokens
+      a.out = out;
+      a.out_stride = out_stride;
+      check_hip(launch_digit_score(a, s.doc, s.residual, plan.nt, reducer, groups, stream), "launch score kernel");
+      return;
+    }
+    ws.pooled.ensure(sizeof(float) * std::max<int64_t>(1, groups * count * a.grp_rows), "hipMalloc pooled rows");
+    a.pooled = ws.pooled.as<float>();
+    a.pooled_grp_stride = count * a.grp_rows;
     check_hip(launch_digit_score(a, s.doc, s.residual, plan.nt, reducer, groups, stream), "launch score kernel");
+    check_hip(launch_pool_sum(ws.pooled.as<float>(), batch, query_tokens, count,
+                              t.per_row ? count * query_tokens : query_tokens, t.per_row ? query_tokens : rows, out,
+                              out_stride, nullptr, 0, stream),
+              "launch pooled sum kernel");
+  };
+  if (t.host || t.device) {
+    if (t.d_offsets == nullptr) throw InvalidArgument("candidate lists need the token offsets");
+    a.targets = t.device ? t.device : ws.cand_ids.as<int64_t>();
+    a.targets_grp_stride = t.per_row ? t.count : 0;
+    a.direct_offsets = t.d_offsets;
+    a.direct_count = t.count;
+    score(t.count, d_out);
     return;
   }
-  ws.pooled.ensure(sizeof(float) * std::max<int64_t>(1, groups * targets * a.grp_rows), "hipMalloc pooled rows");
-  a.pooled = ws.pooled.as<float>();
-  a.pooled_grp_stride = targets * a.grp_rows;
-  check_hip(launch_digit_score(a, s.doc, s.residual, plan.nt, reducer, groups, stream), "launch score kernel");
-  check_hip(launch_pool_sum(ws.pooled.as<float>(), batch, query_tokens, targets,
-                            t.per_row ? targets * query_tokens : query_tokens, t.per_row ? query_tokens : rows, d_out,
-                            out_stride, nullptr, stream),
-            "launch pooled sum kernel");
+  for (int64_t first = 0; first < num_docs; first += kScoreMaxUnitTargets) {
+    const int64_t count = std::min(kScoreMaxUnitTargets, num_docs - first);
+    set_units(ws, off, first, count, device_cu_count(), plan.subs, s.doc == kDocSign ? kDigitUnitSign : kDigitUnitInt4,
+              a, stream);
+    a.doc_scale = s.doc_scale ? s.doc_scale + first : nullptr;
+    score(count, d_out + first);
+  }
 }
 
 }  // namespace
@@ -293,8 +312,7 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
 
   // Sign-bit queries over every document on unit token scales: the fp4
   // Hamming kernel reads the query bits itself.
-  if (g_hamming_fp4 != 0 && q.d_qbits && !s.residual && s.unit_tscale && !t.host && !t.device && !s.doc_scale &&
-      num_docs < kScoreMaxUnitTargets) {
+  if (g_hamming_fp4 != 0 && q.d_qbits && !s.residual && s.unit_tscale && !t.host && !t.device && !s.doc_scale) {
     run_hamming_score(ws, off, s, q.d_qbits, batch, query_tokens, d_out, out_stride, d_iout, stream);
     return;
   }
@@ -365,7 +383,7 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
       a.info_grp_stride = w4 * kScoreInfoWords;
     }
   } else {
-    const ScoreTable& tab = corpus_table(ws, waves, stream, [&](auto& info, auto& tiles) -> int64_t {
+    const ScoreTable& tab = corpus_table(ws, 0, waves, 1, stream, [&](auto& info, auto& tiles) -> int64_t {
       build_score_tables(off.data(), nullptr, num_docs, waves, info, tiles);
       return 0;
     });
@@ -407,7 +425,7 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
   const int64_t bs = t.per_row ? per_target * query_tokens : query_tokens;
   const int64_t ts = t.per_row ? query_tokens : rows;
   check_hip(launch_pool_sum(ws.pooled.as<float>(), batch, query_tokens, per_target, bs, ts, d_out, out_stride, d_iout,
-                            stream),
+                            per_target, stream),
             "launch pooled sum kernel");
 }
 

@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
   int ntok = 0, na = 0, q = 0;
   if constexpr (DIRECT) {
     if (gw < p.direct_count) {
-      doc0 = p.targets ? as_constant(p.targets)[grp * p.targets_grp_stride + gw] : gw;
+      doc0 = as_constant(p.targets)[grp * p.targets_grp_stride + gw];
       ds = as_constant(p.direct_offsets)[doc0];
       ntok = (int)(as_constant(p.direct_offsets)[doc0 + 1] - ds);
       na = ntok == 0 ? 1 : (ntok + 15) / 16;  // an empty document: one tile, not scored

@@ -178,6 +178,7 @@ hipError_t launch_digit_score(const ScoreArgs& a, int doc, bool residual, int nt
   const int64_t waves = group_waves(residual, a.chunks);
   int64_t blocks;
   if (a.direct_offsets != nullptr) {
+    if (a.targets == nullptr) return hipErrorInvalidValue;
     // As many workgroups as CUs before a workgroup gets a second document:
     // a wave alone on its SIMD runs faster than one of two.
     const int64_t spread = std::max<int64_t>(1, kSpreadGroups / (groups * a.subs));

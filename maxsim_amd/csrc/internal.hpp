@@ -305,7 +305,8 @@ hipError_t launch_quantize_limbs(const float* d_query, int64_t rows, int64_t row
 hipError_t launch_quantize_bits(const uint8_t* d_qbits, int64_t rows, int64_t rows_padded, int8_t* qpack,
                                 float* colmul, int32_t* qsum, hipStream_t stream);
 hipError_t launch_pool_sum(const float* pooled, int64_t batch, int64_t query_tokens, int64_t targets, int64_t bs,
-                           int64_t ts, float* out, int64_t out_stride, int32_t* iout, hipStream_t stream);
+                           int64_t ts, float* out, int64_t out_stride, int32_t* iout, int64_t iout_stride,
+                           hipStream_t stream);
 // Tables for `num_targets` targets (targets == nullptr: every document) split
 // over about `waves` waves, balanced by tiles + 1 per target.
 void build_score_tables(const int64_t* offsets, const int64_t* targets, int64_t num_targets, int64_t waves,

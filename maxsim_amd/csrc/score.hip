@@ -542,14 +542,14 @@ __global__ __launch_bounds__(256) void quantize_bits_kernel(const uint8_t* __res
 __global__ __launch_bounds__(256) void pool_sum_kernel(const float* __restrict__ pooled, int64_t batch,
                                                        int64_t query_tokens, int64_t targets, int64_t bs,
                                                        int64_t ts, float* __restrict__ out, int64_t out_stride,
-                                                       int32_t* __restrict__ iout) {
+                                                       int32_t* __restrict__ iout, int64_t iout_stride) {
   const int64_t idx = (int64_t)blockIdx.x * (blockDim.x / 16) + threadIdx.x / 16;
   if (idx >= batch * targets) return;
   const int64_t b = idx / targets, t = idx % targets;
   const float sum = token_sum16(pooled + b * bs + t * ts, (int)query_tokens);
   if ((threadIdx.x & 15) != 0) return;
   if (out) out[b * out_stride + t] = sum;
-  if (iout) iout[b * targets + t] = (int32_t)sum;
+  if (iout) iout[b * iout_stride + t] = (int32_t)sum;
 }
 
 }  // namespace
@@ -594,11 +594,12 @@ hipError_t launch_quantize_bits(const uint8_t* d_qbits, int64_t rows, int64_t ro
 }
 
 hipError_t launch_pool_sum(const float* pooled, int64_t batch, int64_t query_tokens, int64_t targets, int64_t bs,
-                           int64_t ts, float* out, int64_t out_stride, int32_t* iout, hipStream_t stream) {
+                           int64_t ts, float* out, int64_t out_stride, int32_t* iout, int64_t iout_stride,
+                           hipStream_t stream) {
   const int64_t n = batch * targets;
   if (n <= 0) return hipSuccess;
   pool_sum_kernel<<<dim3((unsigned)((n + 15) / 16)), dim3(256), 0, stream>>>(pooled, batch, query_tokens, targets,
-                                                                             bs, ts, out, out_stride, iout);
+                                                                             bs, ts, out, out_stride, iout, iout_stride);
   return hipGetLastError();
 }
 
