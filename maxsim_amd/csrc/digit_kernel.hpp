@@ -284,7 +284,10 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
 
   ReducerState<RED> st[NT];
 #pragma unroll
-  for (int j = 0; j < NT; ++j) st[j].init();
+  for (int j = 0; j < NT; ++j) {
+    st[j].init();
+    if constexpr (RED == kRedLse) st[j].k = 0.0f;  // of the masked tile before the first
+  }
   v4f acc[kSets], accr[RES ? kSets : 1];
   int len = 0;  // tokens of the current target so far
   auto rows_of = [](uint64_t e) -> int { return (int)((e >> kTileRowsShift) & 15) + 1; };
@@ -337,7 +340,7 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
 
   // What the epilogue of a tile needs once its ring slot is reused.  mask: -inf
   // for rows past the tile's, else -0 (x + -0 = x for every x), which joins
-  // the similarity's fma.
+  // the similarity's fma (SmoothSim: that of its scaled form).
   struct Pend {
     float s[UNIT ? 1 : 4], sr[RES ? 4 : 1], mask[UNIT ? 1 : 4];
     uint64_t e;
@@ -346,7 +349,7 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
   // its reducer.
   auto zval = [&](const Pend& P, const v4f& x, const v4f& y, int k) __attribute__((always_inline)) -> float {
     if constexpr (UNIT) return x[k];
-    const float z = fmaf(x[k], P.s[k], P.mask[k]);
+    const float z = RED == kRedLse ? x[k] * P.s[k] : fmaf(x[k], P.s[k], P.mask[k]);
     if constexpr (RES) return fmaf(y[k], P.sr[k], z);
     return z;
   };
@@ -358,7 +361,8 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
         for (int k = 0; k < 4; ++k) z[k] = 4 * g + k >= rows ? kNegInf : z[k];
       }
     }
-    st[j].add4(z, k2);
+    if constexpr (RED == kRedLse) st[j].add4(z, P.mask);
+    else st[j].add4(z);
   };
   // MFMAs stay before the pins of their result, and its reads behind the next
   // one: the compiler otherwise sinks a chain to its epilogue in a later
@@ -461,7 +465,7 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
       }
       set_masks(rows_of(P.e));
     }
-    if (fresh) begin_target(P.e);
+    if (len == 0) begin_target(P.e);  // (after the start's masked tile too)
 #pragma unroll
     for (int j = 1; j < NT; ++j) step(t, j, j, P, j - 1, j - 1, none);
   };
@@ -482,7 +486,6 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
 #pragma unroll
   for (int x = 0; x < (RES ? kSets : 1); ++x) accr[x] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
   len = -1;  // that tile's row count
-  begin_target(ring[0].e);
   // The tiles of slots k .. kRing - 1; false at the stream's end.
   auto round = [&](auto self, auto u_c) __attribute__((always_inline)) -> bool {
     constexpr int k = decltype(u_c)::value;

@@ -21,7 +21,7 @@ struct ReducerState<kRedMax> {
   float m;
   __device__ void init() { m = kNegInf; }
   // Two three-way maxima (v_max3_f32) for four values: exact, any order.
-  __device__ void add4(const float (&z)[4], float) { m = max5_op(m, z[0], z[1], z[2], z[3]); }
+  __device__ void add4(const float (&z)[4]) { m = max5_op(m, z[0], z[1], z[2], z[3]); }
   __device__ float finish(int len, float colmul, float, float weight, float doc_scale) const {
     return len == 0 ? 0.0f : m * colmul * weight * doc_scale;
   }
@@ -46,7 +46,7 @@ struct TopState {
 #pragma unroll
     for (int i = 0; i < K; ++i) t[i] = n[i];
   }
-  __device__ void add4(const float (&z)[4], float) {
+  __device__ void add4(const float (&z)[4]) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) insert(z[r]);
   }
@@ -82,10 +82,12 @@ struct ReducerState<kRedLse> {
     m = kLowest;
     s = 0.0f;
   }
-  __device__ void add4(const float (&z)[4], float) {
+  // mask: -inf for rows that do not count, else -0, joined after the product
+  // with k (-inf times a k of 0 would be NaN, times a negative one +inf).
+  __device__ void add4(const float (&z)[4], const float (&mask)[4]) {
     float u[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) u[r] = z[r] * k;
+    for (int r = 0; r < 4; ++r) u[r] = fmaf(z[r], k, mask[r]);
     const float mn = max3_op(max3_op(m, u[0], u[1]), u[2], u[3]);
     float acc = s * exp2_nonpos(m - mn);
 #pragma unroll

@@ -109,3 +109,33 @@ def test_rows_that_are_not_finite_leave_the_others_alone(gpu, bad):
     np.testing.assert_array_equal(got[[0, 1, 3]], clean[[0, 1, 3]])
     if np.isinf(bad):
         assert np.isnan(got[2]).all()
+
+
+@pytest.mark.parametrize("tau", [0.5, 3.0])
+@pytest.mark.parametrize("shape", [(1, 8), (2, 16), (1, 32), (3, 17), (2, 32), (1, 64), (2, 65)])
+def test_smoothsim_at_document_scales_that_are_zero_or_negative(gpu, oracle, shape, tau):
+    """Documents of whole tiles and with masked rows, first in their wave (every
+    document of a candidate call is) and later ones; a zero scale's score is
+    tau ln(tokens) per query token."""
+    from maxsim_amd._maxsim_hip import CudaPackedDocs
+
+    rng = np.random.default_rng(shape[0] * 100 + shape[1])
+    lengths = np.array((16, 32, 5, 48, 17, 0, 160, 1) * 50, np.int64)
+    offsets = np.concatenate(([0], np.cumsum(lengths))).astype(np.int64)
+    bits = rng.integers(0, 2, (int(offsets[-1]), 128))
+    scale = np.resize(np.array([0.0, 0.25, -0.5, 0.0, 0.0, -1.0, -0.25, -0.125, 0.5], np.float32), lengths.size)
+    h = CudaPackedDocs(np.packbits(bits, axis=1, bitorder="little"), offsets, 128)
+    h.set_scale_vector(scale)
+    docs = (2 * bits - 1).astype(np.float32) * np.repeat(scale, lengths)[:, None]
+    query = rng.standard_normal((*shape, 128)).astype(np.float32)
+    args = {"temperature": tau}
+    got = h.score_batch(query, "smoothsim", None, use_scale_vector=True, **args)
+    exp = oracle.dense_scores(query, docs, offsets, reducer="smoothsim", **args)
+    q64 = np.abs(query.reshape(-1, 128)).astype(np.float64)
+    mag = np.abs(docs).astype(np.float64)
+    sims = _doc_max(mag @ q64.T, offsets).T.reshape(*shape, lengths.size)
+    rows = (_doc_max(mag.sum(1)[:, None], offsets).T * q64.max(1)[:, None]).reshape(*shape, lengths.size)
+    assert (np.abs(got.astype(np.float64) - exp) <= _bound(query, sims, rows, 1, 1, 160 * tau)).all()
+    ids = rng.integers(0, lengths.size, 61)
+    np.testing.assert_array_equal(
+        h.score_candidates_batch(query, ids, "smoothsim", None, use_scale_vector=True, **args), got[:, ids])
