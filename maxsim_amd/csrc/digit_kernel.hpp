@@ -223,8 +223,10 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
     float s[UNIT ? 1 : 4], sr[RES ? 4 : 1];
   };
   // A tile's loads: one buffer per stream at the tile's first token, the lane's
-  // part a constant offset.  Rows past a short document are the next tokens
-  // (or the kScanPadTokens zero tokens after the last one), masked below.
+  // part a constant offset.  Rows past a short document hold the next tokens'
+  // codes (or those of the kScanPadTokens zero tokens after the last one) and a
+  // scale of 0 (the buffers end there: a product with the next document's scale
+  // may not be finite, and -inf then does not mask it).
   const int va = DOC == kDocInt4 ? c * kCodeBytes + 16 * g : c * kCodeBytes + 4 * g;
   const int vr = c * kResBytes + 16 * g, vs = 16 * g;
   auto load = [&](uint64_t e, Tile& t) __attribute__((always_inline)) {
@@ -242,11 +244,12 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
       for (int kc = 0; kc < KC; ++kc) t.res[kc] = load_six(rr, vr + 96 * kc, vr + 96 * kc + 64 - 8 * g);
     }
     if constexpr (!UNIT) {
-      const v4u sv = load_b128(make_rsrc(p.tscale + start, 64u), vs);
+      const uint32_t scale_bytes = 4u * (uint32_t)(((e >> kTileRowsShift) & 15) + 1);
+      const v4u sv = load_b128(make_rsrc(p.tscale + start, scale_bytes), vs);
 #pragma unroll
       for (int k = 0; k < 4; ++k) t.s[k] = __uint_as_float(sv[k]);
       if constexpr (RES) {
-        const v4u rv = load_b128(make_rsrc(p.rtscale + start, 64u), vs);
+        const v4u rv = load_b128(make_rsrc(p.rtscale + start, scale_bytes), vs);
 #pragma unroll
         for (int k = 0; k < 4; ++k) t.sr[k] = __uint_as_float(rv[k]);
       }

@@ -139,3 +139,30 @@ def test_smoothsim_at_document_scales_that_are_zero_or_negative(gpu, oracle, sha
     ids = rng.integers(0, lengths.size, 61)
     np.testing.assert_array_equal(
         h.score_candidates_batch(query, ids, "smoothsim", None, use_scale_vector=True, **args), got[:, ids])
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan, 3e38])
+@pytest.mark.parametrize("reducer", ["maxsim", "topk2", "topk4", "smoothsim"])
+def test_token_scales_of_one_document_leave_the_others_alone(gpu, reducer, bad):
+    """A token scale that is not finite (or whose products are not): only its
+    own document's scores may differ, not those of the document before it,
+    whose last tile holds that token among its masked rows."""
+    from maxsim_amd._maxsim_hip import CudaPackedDocs
+
+    rng = np.random.default_rng(6)
+    offsets = np.concatenate(([0], np.cumsum(np.resize([10, 16, 1, 33, 47], 200)))).astype(np.int64)
+    h = CudaPackedDocs(rng.integers(0, 256, (int(offsets[-1]), 16), dtype=np.uint8), offsets, 128)
+    scale = rng.uniform(0.5, 1.5, int(offsets[-1])).astype(np.float32)
+    ids = np.arange(offsets.size - 1)
+    for shape in ((1, 8), (2, 32), (3, 17)):
+        query = rng.standard_normal((*shape, 128)).astype(np.float32)
+        h.set_token_scale_vector(scale)
+        clean = h.score_batch(query, reducer, use_token_scale=True)
+        marked = ids[1::4]
+        scale2 = scale.copy()
+        scale2[offsets[marked]] = bad
+        h.set_token_scale_vector(scale2)
+        others = np.setdiff1d(ids, marked)
+        np.testing.assert_array_equal(h.score_batch(query, reducer, use_token_scale=True)[:, others], clean[:, others])
+        got = h.score_candidates_batch(query, ids, reducer, use_token_scale=True)
+        np.testing.assert_array_equal(got[:, others], clean[:, others])
