@@ -165,7 +165,7 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
   const int lane = lane_id();
   const int wave = wave_uniform(threadIdx.x / kWave);
   const int g = lane >> 4, c = lane & 15;
-  const int grp = (int)blockIdx.y / p.subs, sub = (int)blockIdx.y % p.subs;
+  const int pass = (int)blockIdx.y + p.first_pass, grp = pass / p.subs, sub = pass % p.subs;
   const int lr0 = sub * p.pass_rows;                      // first local row of the pass
   const int64_t grow0 = (int64_t)grp * p.grp_rows + lr0;  // its global query row
 

@@ -129,11 +129,14 @@ __global__ __launch_bounds__(256) void quantize_digits_kernel(const float* __res
 
 hipError_t launch_encode_fp6(const uint8_t* codes, int64_t tokens, int64_t row_bytes, int chunks, uint8_t* out,
                              hipStream_t stream) {
-  const int64_t groups = tokens * chunks * 4;
-  if (groups <= 0) return hipSuccess;
-  if (row_bytes <= 0 || row_bytes > 64 * (int64_t)chunks || (groups + 255) / 256 > INT32_MAX) return hipErrorInvalidValue;
-  encode_fp6_kernel<<<dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, stream>>>(codes, groups, row_bytes,
-                                                                                    4 * (int64_t)chunks, out);
+  if (row_bytes <= 0 || row_bytes > 64 * (int64_t)chunks) return hipErrorInvalidValue;
+  // (A launch has fewer than 2^32 threads.)
+  constexpr int64_t kMost = int64_t(1) << 26;
+  for (int64_t first = 0; first < tokens; first += kMost) {
+    const int64_t groups = std::min(kMost, tokens - first) * chunks * 4;
+    encode_fp6_kernel<<<dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, stream>>>(
+        codes + first * row_bytes, groups, row_bytes, 4 * (int64_t)chunks, out + first * 96 * chunks);
+  }
   return hipGetLastError();
 }
 
@@ -187,11 +190,18 @@ hipError_t launch_digit_score(const ScoreArgs& a, int doc, bool residual, int nt
     if (a.group_units <= 0 || a.num_waves <= 0 || a.num_waves % a.group_units != 0) return hipErrorInvalidValue;
     blocks = a.num_waves / a.group_units;
   }
-  if (blocks <= 0 || groups * a.subs > 65535) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)blocks, (unsigned)(groups * a.subs));
-  if (a.chunks > 1) return launch_wide(a, doc, residual, nt, reducer, grid, stream);
-  if (doc == kDocInt4) return launch_int4(a, residual, nt, reducer, grid, stream);
-  return launch_sign(a, residual, nt, reducer, grid, stream);
+  if (blocks <= 0) return hipErrorInvalidValue;
+  ScoreArgs part = a;
+  for (int64_t first = 0; first < groups * a.subs; first += kMaxGridRows) {
+    const dim3 grid((unsigned)blocks, (unsigned)std::min(kMaxGridRows, groups * a.subs - first));
+    part.first_pass = (int32_t)first;
+    hipError_t e;
+    if (a.chunks > 1) e = launch_wide(part, doc, residual, nt, reducer, grid, stream);
+    else if (doc == kDocInt4) e = launch_int4(part, residual, nt, reducer, grid, stream);
+    else e = launch_sign(part, residual, nt, reducer, grid, stream);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace msim

@@ -26,6 +26,8 @@
 // 256: 3,380 -> 2,154 (call; 10.1 ns per block and SIMD, the MFMAs alone 8.1 to
 // 8.6).  One workgroup per CU instead of two: 15 % slower; units followed by
 // position instead of TileStream's running pointer: another 8 %.
+#include <algorithm>
+
 #include "common.hpp"
 #include "internal.hpp"
 #include "score_reduce.hpp"
@@ -58,7 +60,7 @@ __global__ __launch_bounds__(kGroupThreads, 4) void hamming_kernel(ScoreArgs p) 
   const int lane = lane_id();
   const int wave = wave_uniform(threadIdx.x / kWave);
   const int g = lane >> 4, c = lane & 15;
-  const int lr0 = (int)blockIdx.y * p.pass_rows;  // first query row of the pass
+  const int lr0 = ((int)blockIdx.y + p.first_pass) * p.pass_rows;  // first query row of the pass
 
   // The tile stream (see digit_score_kernel).
   TileStream<kWaves> stream(p, wave, lane, s_next);
@@ -244,16 +246,20 @@ HammingPlan hamming_plan(int64_t batch, int64_t query_tokens) {
 }
 
 hipError_t launch_hamming(const ScoreArgs& a, hipStream_t stream) {
-  if (a.group_units <= 0 || a.num_waves <= 0 || a.num_waves % a.group_units != 0 || a.subs <= 0 || a.subs > 65535 ||
+  if (a.group_units <= 0 || a.num_waves <= 0 || a.num_waves % a.group_units != 0 || a.subs <= 0 ||
       a.pass_rows <= 0 || a.pass_rows > kHammingRowsPerPass || (a.out && a.iout) || a.qbits == nullptr || a.wave_info == nullptr ||
       a.tiles == nullptr)
     return hipErrorInvalidValue;
-  const dim3 grid((unsigned)(a.num_waves / a.group_units), (unsigned)a.subs);
-  if (a.pass_rows <= 32) hamming_kernel<2><<<grid, kGroupThreads, 0, stream>>>(a);
-  else if (a.pass_rows <= 64) hamming_kernel<4><<<grid, kGroupThreads, 0, stream>>>(a);
-  else if (a.pass_rows <= 128) hamming_kernel<8><<<grid, kGroupThreads, 0, stream>>>(a);
-  else if (a.pass_rows <= 192) hamming_kernel<12><<<grid, kGroupThreads, 0, stream>>>(a);
-  else hamming_kernel<16><<<grid, kGroupThreads, 0, stream>>>(a);
+  ScoreArgs part = a;
+  for (int64_t first = 0; first < a.subs; first += kMaxGridRows) {
+    const dim3 grid((unsigned)(a.num_waves / a.group_units), (unsigned)std::min(kMaxGridRows, a.subs - first));
+    part.first_pass = (int32_t)first;
+    if (a.pass_rows <= 32) hamming_kernel<2><<<grid, kGroupThreads, 0, stream>>>(part);
+    else if (a.pass_rows <= 64) hamming_kernel<4><<<grid, kGroupThreads, 0, stream>>>(part);
+    else if (a.pass_rows <= 128) hamming_kernel<8><<<grid, kGroupThreads, 0, stream>>>(part);
+    else if (a.pass_rows <= 192) hamming_kernel<12><<<grid, kGroupThreads, 0, stream>>>(part);
+    else hamming_kernel<16><<<grid, kGroupThreads, 0, stream>>>(part);
+  }
   return hipGetLastError();
 }
 

@@ -237,6 +237,7 @@ struct ScoreArgs {
   const float* weights;        // [rows_padded] weighted MaxSim factors or nullptr
   int32_t subs;                // passes per group (query rows / rows per pass)
   int32_t pass_rows;           // query rows per pass (fp32 and sign-bit queries)
+  int32_t first_pass;          // (group, pass) of grid row 0, set by the launch functions
   int32_t grp_rows;            // query rows per group
   const float* doc_scale;      // [num_docs] per-document scale or nullptr
   float scale;                 // document scale when doc_scale is null
@@ -258,6 +259,8 @@ struct ScoreArgs {
   // documents by the fp4 Hamming kernel (launch_hamming: work units, pass_rows, chunks 1).
   const uint8_t* qbits;
 };
+// Grid rows of one launch at most; more groups x passes take several launches.
+constexpr int64_t kMaxGridRows = 65535;
 // Query rows per pass of the fp4 Hamming kernel at most (sixteen 16-row blocks).
 constexpr int kHammingRowsPerPass = 256;
 struct HammingPlan {

@@ -23,6 +23,8 @@
 // four lane groups are merged and the per-row pooled values are summed over
 // each batch row's query tokens, or written to pooled[target][row] for
 // pool_sum_kernel.
+#include <algorithm>
+
 #include "common.hpp"
 #include "internal.hpp"
 #include "score_reduce.hpp"
@@ -76,7 +78,7 @@ __global__ __launch_bounds__(kThreads, NT == 8 ? 2 : 1) void score_kernel(ScoreA
   const int lane = lane_id();
   const int wave = wave_uniform(threadIdx.x / kWave);
   const int g = lane >> 4, c = lane & 15;
-  const int grp = (int)blockIdx.y / p.subs, sub = (int)blockIdx.y % p.subs;
+  const int pass = (int)blockIdx.y + p.first_pass, grp = pass / p.subs, sub = pass % p.subs;
   const int64_t gw = (int64_t)blockIdx.x * kWavesPerGroup + wave;
   const auto targets = p.targets ? as_constant(p.targets) + grp * p.targets_grp_stride : nullptr;
   const int lr0 = sub * 16 * NT;                           // first local row of the pass
@@ -543,13 +545,14 @@ __global__ __launch_bounds__(256) void pool_sum_kernel(const float* __restrict__
                                                        int64_t query_tokens, int64_t targets, int64_t bs,
                                                        int64_t ts, float* __restrict__ out, int64_t out_stride,
                                                        int32_t* __restrict__ iout, int64_t iout_stride) {
-  const int64_t idx = (int64_t)blockIdx.x * (blockDim.x / 16) + threadIdx.x / 16;
-  if (idx >= batch * targets) return;
-  const int64_t b = idx / targets, t = idx % targets;
-  const float sum = token_sum16(pooled + b * bs + t * ts, (int)query_tokens);
-  if ((threadIdx.x & 15) != 0) return;
-  if (out) out[b * out_stride + t] = sum;
-  if (iout) iout[b * iout_stride + t] = (int32_t)sum;
+  for (int64_t idx = (int64_t)blockIdx.x * (blockDim.x / 16) + threadIdx.x / 16; idx < batch * targets;
+       idx += (int64_t)gridDim.x * (blockDim.x / 16)) {
+    const int64_t b = idx / targets, t = idx % targets;
+    const float sum = token_sum16(pooled + b * bs + t * ts, (int)query_tokens);
+    if ((threadIdx.x & 15) != 0) continue;
+    if (out) out[b * out_stride + t] = sum;
+    if (iout) iout[b * iout_stride + t] = (int32_t)sum;
+  }
 }
 
 }  // namespace
@@ -561,16 +564,20 @@ hipError_t launch_score(const ScoreArgs& a, bool residual, int64_t groups, hipSt
   if (a.num_waves <= 0 || a.num_waves % kWavesPerGroup != 0 || a.subs <= 0 || groups <= 0) return hipErrorInvalidValue;
   if (a.tscale == nullptr || (residual && (a.rcodes == nullptr || a.rtscale == nullptr))) return hipErrorInvalidValue;
   const bool narrow = score_rows_per_pass(a.grp_rows) == 32;
-  const dim3 grid((unsigned)(a.num_waves / kWavesPerGroup), (unsigned)(groups * a.subs));
-  if (residual) {
-    if (narrow) score_kernel<true, 2, false><<<grid, kThreads, 0, stream>>>(a);
-    else score_kernel<true, 8, false><<<grid, kThreads, 0, stream>>>(a);
-  } else if (a.unit_tscale) {
-    if (narrow) score_kernel<false, 2, true><<<grid, kThreads, 0, stream>>>(a);
-    else score_kernel<false, 8, true><<<grid, kThreads, 0, stream>>>(a);
-  } else {
-    if (narrow) score_kernel<false, 2, false><<<grid, kThreads, 0, stream>>>(a);
-    else score_kernel<false, 8, false><<<grid, kThreads, 0, stream>>>(a);
+  ScoreArgs part = a;
+  for (int64_t first = 0; first < groups * a.subs; first += kMaxGridRows) {
+    const dim3 grid((unsigned)(a.num_waves / kWavesPerGroup), (unsigned)std::min(kMaxGridRows, groups * a.subs - first));
+    part.first_pass = (int32_t)first;
+    if (residual) {
+      if (narrow) score_kernel<true, 2, false><<<grid, kThreads, 0, stream>>>(part);
+      else score_kernel<true, 8, false><<<grid, kThreads, 0, stream>>>(part);
+    } else if (a.unit_tscale) {
+      if (narrow) score_kernel<false, 2, true><<<grid, kThreads, 0, stream>>>(part);
+      else score_kernel<false, 8, true><<<grid, kThreads, 0, stream>>>(part);
+    } else {
+      if (narrow) score_kernel<false, 2, false><<<grid, kThreads, 0, stream>>>(part);
+      else score_kernel<false, 8, false><<<grid, kThreads, 0, stream>>>(part);
+    }
   }
   return hipGetLastError();
 }
@@ -598,8 +605,10 @@ hipError_t launch_pool_sum(const float* pooled, int64_t batch, int64_t query_tok
                            hipStream_t stream) {
   const int64_t n = batch * targets;
   if (n <= 0) return hipSuccess;
-  pool_sum_kernel<<<dim3((unsigned)((n + 15) / 16)), dim3(256), 0, stream>>>(pooled, batch, query_tokens, targets,
-                                                                             bs, ts, out, out_stride, iout, iout_stride);
+  // (A launch has fewer than 2^32 threads: large outputs are walked.)
+  const int64_t blocks = std::min<int64_t>((n + 15) / 16, 1 << 18);
+  pool_sum_kernel<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(pooled, batch, query_tokens, targets, bs, ts, out,
+                                                                  out_stride, iout, iout_stride);
   return hipGetLastError();
 }
 

@@ -72,3 +72,30 @@ def test_sign_scores_of_more_than_2_24_documents(gpu):
     h.set_scale_vector(scale)
     signs = np.unpackbits(bits.view(np.uint8), axis=1, bitorder="little").astype(np.float32)[None] * 2 - 1
     np.testing.assert_array_equal(h.maxsim_batch(signs, use_scale_vector=True)[0], exp * scale)
+
+
+@pytest.mark.parametrize("kind", ["int4", "binary_int8", "binary_fp32"])
+def test_more_batch_rows_than_grid_rows(gpu, kind):
+    """Per-row candidate lists take a grid row per batch row, and a launch has
+    at most 65,535: the results are those of the same rows a part at a time."""
+    from maxsim_amd._maxsim_hip import CudaInt4PackedDocs, CudaPackedDocs
+
+    rng = np.random.default_rng(43)
+    offsets = np.array([0, 3, 3, 20, 21, 40], np.int64)
+    dim = 8 if kind == "int4" else 128
+    codes = rng.integers(0, 256, (40, dim // 2), dtype=np.uint8)
+    scale = rng.uniform(0.5, 1.5, 40).astype(np.float32)
+    if kind == "int4":
+        h = CudaInt4PackedDocs(codes, offsets, dim, 1.0)
+        h.set_residual_int4(rng.integers(0, 256, codes.shape, dtype=np.uint8), 0.1, scale)
+    else:
+        h = CudaPackedDocs(rng.integers(0, 256, (40, 16), dtype=np.uint8), offsets, dim)
+        h.set_token_scale_vector(scale)
+        h.set_residual_int4(codes, 0.1, scale)
+        h.set_rescore_limbs(3 if kind == "binary_fp32" else 1)
+    query = rng.standard_normal((66_000, 1, dim)).astype(np.float32)
+    scores, ids = h.cascade_topk(query, 2, 3)
+    for part in (slice(0, 1000), slice(65_000, 66_000)):
+        exp_s, exp_i = h.cascade_topk(query[part], 2, 3)
+        np.testing.assert_array_equal(scores[part], exp_s)
+        np.testing.assert_array_equal(ids[part], exp_i)
