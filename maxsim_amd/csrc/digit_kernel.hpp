@@ -36,7 +36,7 @@
 // (80 ns per 16 x 16 block of int4 at four blocks, 73 of signs, against 56 and 48
 // of the MFMAs alone; one int4 query is bound by memory, 6.4 TB/s of fp6 rows.)
 //
-// Work split: the eight waves (two per SIMD) of a workgroup share one pass of
+// Work split: the waves of a workgroup (group_waves) share one pass of
 // query rows; its digits are staged once in LDS and held in registers (NT
 // blocks of 16 rows, 30 VGPRs each per 128 dims).  A wave walks 16-token tiles
 // (the MFMA's A operand), held in a ring of registers filled by buffer loads
@@ -64,9 +64,13 @@ typedef int v2i __attribute__((ext_vector_type(2)));
 typedef int v8i __attribute__((ext_vector_type(8)));
 
 constexpr int kDigits = kScoreDigits;
-// Waves per workgroup: two per SIMD, one where four chunks of two streams
-// take more than half of a SIMD's registers.
-constexpr int group_waves(bool res, int kc) { return res && kc == 4 ? 4 : 8; }
+// Waves per workgroup: two per SIMD; one at four chunks, so that a pass holds
+// 32 query rows (240 VGPRs of digits) and three tiles in flight (28 each).  With
+// two waves a pass held 16 rows and one tile was in flight, and the calls waited
+// for memory: 4,096 documents of 512 dims, queries of 32 tokens, the call: 1 / 4
+// queries 101 / 287 us, now 73 / 164; with a residual stream 161 / 525, now
+// 113 / 297; signs 113 / 318, now 85 / 193.
+constexpr int group_waves(int kc) { return kc == 4 ? 4 : 8; }
 constexpr int kFormatFp6 = 2, kFormatFp4 = 4;  // cbsz / blgp: e2m3, e2m1
 
 // E8M0 scale bytes: 2^-5i of digit i, and of the document operand (int4 codes
@@ -102,10 +106,11 @@ __device__ __forceinline__ v4f mfma_digit(const v8i& a, const v8i& b, const v4f&
 }
 
 // Tiles held per wave (one computed, the rest in flight): what the registers
-// left by the query digits take.  Signs are small (256 bytes per tile), so
+// left by the query digits take (rings of eight at four chunks were no faster).  Signs are small (256 bytes per tile), so
 // only many of them in flight cover the memory latency.
 constexpr int ring_size(int doc, bool res, int nt, int kc, bool unit) {
   if (doc == kDocSign && !res && kc == 1) return unit ? 8 : nt == 4 ? 4 : 8;
+  if (kc == 4) return res && nt == 2 ? 2 : 4;
   if (res) return nt * kc >= 4 ? 2 : 4;
   return kc == 1 ? 4 : nt * kc >= 4 ? 2 : 4;
 }
@@ -141,9 +146,9 @@ __device__ __forceinline__ ReducerState<RED> swap_merge(const ReducerState<RED>&
 // accumulator itself.  DIRECT: one target per wave, its document's token range
 // from p.direct_offsets; else work units.
 template <int DOC, bool RES, int NT, int RED, int KC, bool UNIT, bool DIRECT>
-__global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) / 4) void digit_score_kernel(
+__global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void digit_score_kernel(
     ScoreArgs p) {
-  constexpr int kWavesPerGroup = group_waves(RES, KC), kThreads = kWavesPerGroup * kWave;
+  constexpr int kWavesPerGroup = group_waves(KC), kThreads = kWavesPerGroup * kWave;
   static_assert(!UNIT || (DOC == kDocSign && !RES && RED == kRedMax), "accumulators as similarities");
   static_assert(!(DOC == kDocSign && RES) || KC == 1, "sign prefix + residual: 128 dims");
   constexpr int kRing = ring_size(DOC, RES, NT, KC, UNIT);
@@ -523,7 +528,7 @@ __global__ __launch_bounds__(kWave * group_waves(RES, KC), group_waves(RES, KC) 
 
 template <int DOC, bool RES, int NT, int RED, int KC, bool UNIT = false>
 hipError_t launch_mode(const ScoreArgs& a, dim3 grid, hipStream_t s) {
-  constexpr int kThreads = kWave * group_waves(RES, KC);
+  constexpr int kThreads = kWave * group_waves(KC);
   if (a.direct_offsets) digit_score_kernel<DOC, RES, NT, RED, KC, UNIT, true><<<grid, kThreads, 0, s>>>(a);
   else digit_score_kernel<DOC, RES, NT, RED, KC, UNIT, false><<<grid, kThreads, 0, s>>>(a);
   return hipGetLastError();
@@ -542,7 +547,9 @@ hipError_t launch_reducer(const ScoreArgs& a, int reducer, dim3 grid, hipStream_
 // The instantiations by document format (one source file each).
 hipError_t launch_int4(const ScoreArgs& a, bool residual, int nt, int reducer, dim3 grid, hipStream_t s);
 hipError_t launch_sign(const ScoreArgs& a, bool residual, int nt, int reducer, dim3 grid, hipStream_t s);
-hipError_t launch_wide(const ScoreArgs& a, int doc, bool residual, int nt, int reducer, dim3 grid, hipStream_t s);
+hipError_t launch_wide2(const ScoreArgs& a, int doc, bool residual, int nt, int reducer, dim3 grid, hipStream_t s);
+hipError_t launch_wide4(const ScoreArgs& a, int doc, bool residual, int nt, int reducer, dim3 grid, hipStream_t s);
+hipError_t launch_wide4_residual(const ScoreArgs& a, int nt, int reducer, dim3 grid, hipStream_t s);
 
 }  // namespace digit
 }  // namespace msim

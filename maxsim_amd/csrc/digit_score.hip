@@ -152,10 +152,10 @@ hipError_t launch_quantize_digits(const float* d_query, int64_t rows, int64_t ro
 }
 
 DigitPlan digit_plan(int64_t batch, int64_t query_tokens, int chunks) {
-  // The most rows a pass holds in registers: 64, 32 or 16 at one, two or four
-  // chunks.  Whole batch rows per pass where one fits (the kernel then sums
+  // The most rows a pass holds in registers: 64, or 32 of more than 128 dims.
+  // Whole batch rows per pass where one fits (the kernel then sums
   // their tokens), spread evenly over the passes; blocks of 1, 2 or 4.
-  const int64_t most = 64 / chunks;
+  const int64_t most = chunks == 1 ? 64 : 32;
   DigitPlan d;
   if (query_tokens <= most) {
     const int64_t per = most / query_tokens, passes = (batch + per - 1) / per;
@@ -178,7 +178,7 @@ hipError_t launch_digit_score(const ScoreArgs& a, int doc, bool residual, int nt
   if (a.subs <= 0 || groups <= 0 || a.pass_rows <= 0 || a.pass_rows > 16 * nt || a.tscale == nullptr ||
       (residual && (a.rcodes == nullptr || a.rtscale == nullptr)))
     return hipErrorInvalidValue;
-  const int64_t waves = group_waves(residual, a.chunks);
+  const int64_t waves = group_waves(a.chunks);
   int64_t blocks;
   if (a.direct_offsets != nullptr) {
     if (a.targets == nullptr) return hipErrorInvalidValue;
@@ -196,7 +196,8 @@ hipError_t launch_digit_score(const ScoreArgs& a, int doc, bool residual, int nt
     const dim3 grid((unsigned)blocks, (unsigned)std::min(kMaxGridRows, groups * a.subs - first));
     part.first_pass = (int32_t)first;
     hipError_t e;
-    if (a.chunks > 1) e = launch_wide(part, doc, residual, nt, reducer, grid, stream);
+    if (a.chunks == 4) e = launch_wide4(part, doc, residual, nt, reducer, grid, stream);
+    else if (a.chunks == 2) e = launch_wide2(part, doc, residual, nt, reducer, grid, stream);
     else if (doc == kDocInt4) e = launch_int4(part, residual, nt, reducer, grid, stream);
     else e = launch_sign(part, residual, nt, reducer, grid, stream);
     if (e != hipSuccess) return e;

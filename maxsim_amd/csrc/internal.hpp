@@ -271,7 +271,7 @@ HammingPlan hamming_plan(int64_t batch, int64_t query_tokens);
 hipError_t launch_hamming(const ScoreArgs& a, hipStream_t stream);
 // Dims above 128 (fp32 queries) are scored in 128-dim chunks whose MFMA dots
 // accumulate in one accumulator: 2 chunks up to 256 dims, 4 up to 512 (0:
-// above; a 16-row pass of 512 dims takes 120 VGPRs of query digits).
+// above; 32 query rows of 512 dims take 240 VGPRs of digits).
 constexpr int64_t kScoreMaxDim = 512;
 inline int score_chunks(int64_t dim) { return dim <= 128 ? 1 : dim <= 256 ? 2 : dim <= 512 ? 4 : 0; }
 int score_rows_per_pass(int64_t rows);
