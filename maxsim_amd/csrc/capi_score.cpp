@@ -162,7 +162,12 @@ const ScoreTable& corpus_table(ScoreWorkspace& ws, int64_t first, int64_t split,
 // over as many workgroups.
 void set_units(ScoreWorkspace& ws, const std::vector<int64_t>& off, int64_t first, int64_t count, int64_t workgroups,
                int64_t subs, int64_t min_tiles, ScoreArgs& a, hipStream_t stream) {
-  const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(workgroups / subs, count));
+  int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(workgroups / subs, count));
+  // Dims above 128 (bound by memory): a multiple of eight lists where that
+  // idles at most one workgroup in 16, so that every pass of a list is on one
+  // XCD (workgroups go to the eight XCDs in turn) and its L2 serves them all.
+  // 33,000 tiles, three passes: 256 dims 74 -> 62 us a call, 512 dims 149 -> 139.
+  if (a.chunks > 1 && 16 * (wgs & ~7) >= 15 * wgs) wgs &= ~7;
   const ScoreTable& t =
       corpus_table(ws, first, -2 - wgs, doc_ranges((int64_t)off.size() - 1), stream, [&](auto& info, auto& tiles) {
         return build_score_units(off.data() + first, nullptr, count, wgs, info, tiles, min_tiles);
@@ -211,13 +216,16 @@ void run_hamming_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, cons
 
 // fp32 queries: digits, then one launch over every document (work units) or
 // over candidate documents (one per wave).
-void run_digit_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, const DocStreams& s, const QueryInput& q,
-                     int reducer, float temperature, int64_t batch, int64_t query_tokens, const float* h_row_weights,
-                     const Targets& t, float* d_out, int64_t out_stride, hipStream_t stream) {
+void run_digit_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int64_t num_tokens, const DocStreams& s,
+                     const QueryInput& q, int reducer, float temperature, int64_t batch, int64_t query_tokens,
+                     const float* h_row_weights, const Targets& t, float* d_out, int64_t out_stride,
+                     hipStream_t stream) {
   const int64_t num_docs = (int64_t)off.size() - 1;
   const int64_t rows = batch * query_tokens, rows_padded = ceil_div(rows, 16) * 16 + 128;
   const int64_t groups = t.per_row ? batch : 1;
-  const DigitPlan plan = digit_plan(t.per_row ? 1 : batch, query_tokens, s.chunks);
+  const int64_t targets = (t.host || t.device) ? t.count : num_docs;
+  const int64_t doc_tiles = std::max<int64_t>(1, ceil_div(num_tokens, 16 * num_docs));  // of an average document
+  const DigitPlan plan = digit_plan(t.per_row ? 1 : batch, query_tokens, s.chunks, targets * doc_tiles);
 
   ws.qpack.ensure(digit_bytes(rows_padded, s.chunks), "hipMalloc query digits");
   ws.colmul.ensure(sizeof(float) * rows_padded, "hipMalloc query scales");
@@ -300,8 +308,8 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
     return;
   }
   if (q.limbs == 3) {
-    run_digit_score(ws, off, s, q, reducer, temperature, batch, query_tokens, h_row_weights, t, d_out, out_stride,
-                    stream);
+    run_digit_score(ws, off, num_tokens, s, q, reducer, temperature, batch, query_tokens, h_row_weights, t, d_out,
+                    out_stride, stream);
     return;
   }
   // int8 and sign-bit queries: sign documents (with or without the residual

@@ -9,6 +9,13 @@ namespace msim {
 namespace {
 
 constexpr int64_t kSpreadGroups = 256;  // CUs of an MI355X
+// Tiles times passes that pay for pool_sum_kernel (2 us beside the scores it
+// reads); half of it at four chunks, whose tiles take twice as long.  Whole
+// rows / packed, the call in us: 8,200 tiles, 4 queries of 40 tokens (four
+// passes / three) 39.6 / 40.0; 12,000: 43.8 / 43.3; 16,400: 49.1 / 47.1; 33,000:
+// 69 / 63, 8 queries 103 / 83, 16 of 33 tokens 177 / 121; 256 dims, 3 of 20:
+// 74.6 / 54.4.
+constexpr int64_t kPackTiles = 12288;
 
 // Six-bit fields of one lane's 32 operand elements: element s is bits 6 s ..
 // 6 s + 5 of 192 (six dwords).
@@ -151,22 +158,25 @@ hipError_t launch_quantize_digits(const float* d_query, int64_t rows, int64_t ro
   return hipGetLastError();
 }
 
-DigitPlan digit_plan(int64_t batch, int64_t query_tokens, int chunks) {
+DigitPlan digit_plan(int64_t batch, int64_t query_tokens, int chunks, int64_t tiles) {
   // The most rows a pass holds in registers: 64, or 32 of more than 128 dims.
-  // Whole batch rows per pass where one fits (the kernel then sums
-  // their tokens), spread evenly over the passes; blocks of 1, 2 or 4.
+  // Whole batch rows per pass where one fits (the kernel then sums their
+  // tokens), spread evenly over the passes; blocks of 1, 2 or 4.  Batch rows
+  // that fill their passes badly (33 of 64) are cut at the passes' ends where
+  // that saves kPackTiles tiles: pool_sum_kernel then sums their tokens.
   const int64_t most = chunks == 1 ? 64 : 32;
+  const int64_t packed = (batch * query_tokens + most - 1) / most;
   DigitPlan d;
+  d.pass_rows = most;
+  d.subs = packed;
+  d.whole = false;
   if (query_tokens <= most) {
     const int64_t per = most / query_tokens, passes = (batch + per - 1) / per;
-    const int64_t rows = (batch + passes - 1) / passes * query_tokens;
-    d.pass_rows = rows;
-    d.subs = (batch * query_tokens + rows - 1) / rows;
-    d.whole = true;
-  } else {
-    d.pass_rows = most;
-    d.subs = (batch * query_tokens + most - 1) / most;
-    d.whole = false;
+    if ((passes - packed) * tiles * (chunks == 4 ? 2 : 1) < kPackTiles) {
+      d.pass_rows = (batch + passes - 1) / passes * query_tokens;
+      d.subs = (batch * query_tokens + d.pass_rows - 1) / d.pass_rows;
+      d.whole = true;
+    }
   }
   d.nt = d.pass_rows <= 16 ? 1 : d.pass_rows <= 32 ? 2 : 4;
   return d;

@@ -292,7 +292,7 @@ struct DigitPlan {
   int nt;      // 16-row blocks per pass: 1, 2 or 4
   bool whole;  // passes hold whole batch rows
 };
-DigitPlan digit_plan(int64_t batch, int64_t query_tokens, int chunks);
+DigitPlan digit_plan(int64_t batch, int64_t query_tokens, int chunks, int64_t tiles);
 hipError_t launch_encode_fp6(const uint8_t* codes, int64_t tokens, int64_t row_bytes, int chunks, uint8_t* out,
                              hipStream_t stream);
 hipError_t launch_quantize_digits(const float* d_query, int64_t rows, int64_t rows_padded, uint8_t* qpack,

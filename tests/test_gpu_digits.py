@@ -166,3 +166,29 @@ def test_token_scales_of_one_document_leave_the_others_alone(gpu, reducer, bad):
         np.testing.assert_array_equal(h.score_batch(query, reducer, use_token_scale=True)[:, others], clean[:, others])
         got = h.score_candidates_batch(query, ids, reducer, use_token_scale=True)
         np.testing.assert_array_equal(got[:, others], clean[:, others])
+
+
+@pytest.mark.parametrize("dim, shapes", [(128, [(3, 33), (4, 40), (5, 50), (16, 33)]), (256, [(8, 17), (3, 20)]),
+                                         (512, [(8, 17), (3, 20)])])
+def test_batch_rows_cut_at_the_ends_of_passes(gpu, dim, shapes):
+    """Corpora large enough that badly filled passes are not taken: the scores
+    are bit for bit those of each query by itself."""
+    from maxsim_amd._maxsim_hip import CudaInt4PackedDocs
+
+    rng = np.random.default_rng(dim)
+    lengths = rng.integers(0, 130, 4000)
+    offsets = np.concatenate(([0], np.cumsum(lengths))).astype(np.int64)
+    _, packed = _codes(rng, int(offsets[-1]), dim)
+    h = CudaInt4PackedDocs(packed, offsets, dim, 0.1)
+    h.set_residual_int4(_codes(rng, int(offsets[-1]), dim)[1], 0.01, np.ones(int(offsets[-1]), np.float32))
+    ids = rng.integers(0, 4000, 3500)
+    for shape in shapes:
+        query = rng.standard_normal((*shape, dim)).astype(np.float32)
+        weights = rng.uniform(0.5, 1.5, shape).astype(np.float32)
+        for reducer, w in (("weighted_maxsim", weights), ("smoothsim", None)):
+            each = [h.score_batch(query[b : b + 1], reducer, None if w is None else w[b])[0] for b in range(shape[0])]
+            np.testing.assert_array_equal(h.score_batch(query, reducer, w), np.stack(each))
+            got = h.score_candidates_batch(query, ids, reducer, w)
+            np.testing.assert_array_equal(got, np.stack(each)[:, ids])
+        each = [h.score_residual_batch(query[b : b + 1])[0] for b in range(shape[0])]
+        np.testing.assert_array_equal(h.score_residual_batch(query), np.stack(each))
