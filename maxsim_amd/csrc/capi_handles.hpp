@@ -58,8 +58,18 @@ struct QueryInput {
   bool from_alt = false;             // score the rows an earlier alt_int4 call left in qpack_alt
 };
 
-// The document streams and scales of one scoring call (int4 codes as fp6 rows
-// where the query is fp32).
+// An int4 stream as fp6 rows (96 bytes per token and 128-dim chunk), which fp32
+// queries are scored from without decoding nibbles: see fp6_rows.
+struct Fp6Copy {
+  DeviceBuffer rows;
+  int64_t scored = 0;  // tokens scored from the nibbles
+  void reset() {
+    rows.reset();
+    scored = 0;
+  }
+};
+
+// The document streams and scales of one scoring call.
 struct DocStreams {
   int doc = kDocInt4;
   bool residual = false;
@@ -69,6 +79,7 @@ struct DocStreams {
   const uint8_t* rcodes = nullptr;
   const float* rtscale = nullptr;
   float rmul = 1.0f;
+  int code_bytes = 0;  // fp32 queries: int4 streams are nibbles of so many bytes per token; 0: fp6 rows
   const float* doc_scale = nullptr;
   float scale = 1.0f;
   bool unit_tscale = false;  // tscale is all ones
@@ -139,10 +150,10 @@ struct msim_int4_docs {
   int64_t block_pos_off = 0;      // index of the workgroup start positions in wave_info
   msim::DeviceBuffer wave_info, tile_table;
   msim::DeviceBuffer packed, offsets, token_scales, token_scales16, residual_packed, residual_token_scales16;
-  // fp32 queries: the codes as fp6 rows (96 bytes per token and 128-dim
-  // chunk), made on the device at the first such call, and per-token 1/16 when
-  // the corpus has no token scales.
-  msim::DeviceBuffer codes6, residual6, ones16;
+  // fp32 queries: the codes as fp6 rows, and per-token 1/16 when the corpus has
+  // no token scales.
+  msim::Fp6Copy codes6, residual6;
+  msim::DeviceBuffer ones16;
   // workspaces (grow monotonically, freed with the handle; cu:3057-3067)
   msim::DeviceBuffer qpack, qscale, qbias, scores, rowmax;
   msim::HostBuffer host_io;  // synchronous calls: query in, results out (pinned)
@@ -153,7 +164,7 @@ struct msim_int4_docs {
 
   uint64_t resident_bytes() const {
     return packed_size + offsets_size * 8 + token_scales.cap + token_scales16.cap + residual_packed.cap +
-           residual_token_scales16.cap + codes6.cap + residual6.cap + ones16.cap;
+           residual_token_scales16.cap + codes6.rows.cap + residual6.rows.cap + ones16.cap;
   }
   uint64_t workspace_bytes() const {
     return qpack.cap + qscale.cap + qbias.cap + scores.cap +
@@ -177,7 +188,7 @@ struct msim_binary_docs {
   double residual_scale = 1.0;
   int64_t max_doc_tiles = 1;  // 16-token tiles of the longest document
   msim::DeviceBuffer residual_packed, residual_token_scales16;
-  msim::DeviceBuffer residual6;  // the residual codes as fp6 rows (fp32 rescoring)
+  msim::Fp6Copy residual6;  // fp32 rescoring
   // Query of the fused (prefix + residual) scoring and of a cascade's
   // rescoring pass: 1 = the int8 query, 3 = the fp32 query.
   int rescore_limbs = 1;
@@ -192,7 +203,7 @@ struct msim_binary_docs {
 
   uint64_t resident_bytes() const {
     return packed.cap + offsets.cap + scale_vector.cap + token_scales.cap + ones.cap + residual_packed.cap +
-           residual_token_scales16.cap + residual6.cap;
+           residual_token_scales16.cap + residual6.rows.cap;
   }
   uint64_t workspace_bytes() const {
     return scores.cap + iscores.cap + scale_override.cap + scan_wave_info.cap +

@@ -100,6 +100,7 @@ void set_streams(ScoreArgs& a, const DocStreams& s) {
   a.rcodes = s.rcodes;
   a.rtscale = s.rtscale;
   a.rmul = s.rmul;
+  a.code_bytes = s.code_bytes;
   a.doc_scale = s.doc_scale;
   a.scale = s.scale;
   a.unit_tscale = s.unit_tscale;
@@ -547,29 +548,69 @@ void copy_scores_out(ScoreWorkspace& ws, void* out, const void* d, size_t bytes)
 
 // ------------------------------------------------------------------ int4
 
-// int4 codes as fp6 rows, made at the first fp32 query of the handle (about
-// 30 us per half million tokens) and waited for, so that a later call may come
-// on any stream.
-const uint8_t* fp6_rows(DeviceBuffer& rows, const uint8_t* codes, int64_t num_tokens, int64_t dim) {
-  if (rows.ptr == nullptr && num_tokens > 0) {
-    const int chunks = score_chunks(dim);
-    DeviceBuffer made;
-    // (and the kScanPadTokens zero rows a tile may read past the last token)
-    const int64_t words = 24 * chunks;  // floats per row
-    made.ensure((size_t)((num_tokens + kScanPadTokens) * words * 4), "hipMalloc fp6 document rows");
-    check_hip(launch_encode_fp6(codes, num_tokens, dim / 2, chunks, made.as<uint8_t>(), nullptr),
-              "launch fp6 document kernel");
-    check_hip(launch_fill_f32(made.as<float>() + num_tokens * words, kScanPadTokens * words, 0.0f, nullptr),
-              "zero fp6 document padding");
-    check_hip(hipStreamSynchronize(nullptr), "synchronize fp6 document kernel");
-    std::swap(rows.ptr, made.ptr);
-    std::swap(rows.cap, made.cap);
+// The int4 stream as fp6 rows for a call that scores `tokens` of its tokens, or
+// null: the call decodes the nibbles itself.  The copy, half as large again as
+// the corpus, takes about 300 us (an allocation; encoding half a million tokens
+// 30 us), so it is made once decoding may have cost as much: after 2^24 tokens
+// beyond the first search, or 32 searches.  A handle that serves one search, or
+// short candidate lists, keeps to the memory of its corpus.  From nibbles / from
+// the copy, calls of 4 queries of 32 tokens: 4,096 documents 64 / 53 us, 16,384
+// 157 / 115; a first call with the copy / without, 512 documents 450 / 189 us, of
+// 100 candidates 354 / 94.  The copy takes at most half of the free device
+// memory, or is tried again much later; it is waited for, so that a later call
+// may come on any stream; and a captured call makes none.  Rows the kernel cannot
+// load (dims that are no multiple of 8) are copied at once.
+const uint8_t* fp6_rows(Fp6Copy& copy, const uint8_t* codes, int64_t num_tokens, int64_t dim, int64_t tokens,
+                        hipStream_t stream) {
+  if (copy.rows.ptr != nullptr || num_tokens == 0) return copy.rows.as<uint8_t>();
+  const bool must = dim % 8 != 0;
+  if (!must && copy.scored < std::min(32 * num_tokens, num_tokens + (int64_t(1) << 24))) {
+    copy.scored += tokens;
+    return nullptr;
   }
-  return rows.as<uint8_t>();
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (!must && stream != nullptr && hipStreamIsCapturing(stream, &capture) == hipSuccess &&
+      capture != hipStreamCaptureStatusNone)
+    return nullptr;
+  const int chunks = score_chunks(dim);
+  // (and the kScanPadTokens zero rows a tile may read past the last token)
+  const int64_t words = 24 * chunks;  // floats per row
+  const size_t bytes = (size_t)((num_tokens + kScanPadTokens) * words * 4);
+  size_t free_bytes = 0, total_bytes = 0;
+  DeviceBuffer made;
+  try {
+    if (!must) {
+      check_hip(hipMemGetInfo(&free_bytes, &total_bytes), "hipMemGetInfo");
+      if (bytes > free_bytes / 2) throw OutOfDeviceMemory("fp6 document rows");
+    }
+    made.ensure(bytes, "hipMalloc fp6 document rows");
+  } catch (const OutOfDeviceMemory&) {
+    if (must) throw;
+    (void)hipGetLastError();  // (a later launch would report it)
+    copy.scored = -1024 * num_tokens;
+    return nullptr;
+  }
+  check_hip(launch_encode_fp6(codes, num_tokens, dim / 2, chunks, made.as<uint8_t>(), nullptr),
+            "launch fp6 document kernel");
+  check_hip(launch_fill_f32(made.as<float>() + num_tokens * words, kScanPadTokens * words, 0.0f, nullptr),
+            "zero fp6 document padding");
+  check_hip(hipStreamSynchronize(nullptr), "synchronize fp6 document kernel");
+  std::swap(copy.rows.ptr, made.ptr);
+  std::swap(copy.rows.cap, made.cap);
+  return copy.rows.as<uint8_t>();
 }
 
-DocStreams int4_streams(msim_int4_docs* h, bool residual) {
+// Tokens of `targets` documents, about.
+template <typename H>
+int64_t target_tokens(const H* h, int64_t targets) {
+  return ceil_div(h->num_tokens, std::max<int64_t>(1, h->num_docs)) * targets;
+}
+
+// The streams of a call that scores about `tokens` tokens on `stream`.
+DocStreams int4_streams(msim_int4_docs* h, bool residual, int64_t tokens, hipStream_t stream) {
   if (h->dim > kScoreMaxDim) throw NotSupported("fp32-query int4 scoring currently supports dim <= 512");
+  if (residual && !h->has_residual)
+    throw InvalidArgument("residual int4 data was requested but is not loaded on this CUDA handle");
   if (h->num_tokens > 0 && !h->has_token_scale && h->ones16.cap < (size_t)h->num_tokens * 4) {
     std::vector<float> ones((size_t)(h->num_tokens + kScanPadTokens), 0.0625f);
     h->ones16.ensure(ones.size() * 4, "hipMalloc int4 unit token scales");
@@ -578,17 +619,20 @@ DocStreams int4_streams(msim_int4_docs* h, bool residual) {
   DocStreams s;
   s.doc = kDocInt4;
   s.chunks = score_chunks(h->dim);
-  s.codes = fp6_rows(h->codes6, h->packed.as<uint8_t>(), h->num_tokens, h->dim);
+  s.codes = fp6_rows(h->codes6, h->packed.as<uint8_t>(), h->num_tokens, h->dim, tokens, stream);
   s.tscale = h->has_token_scale ? h->token_scales16.as<float>() : h->ones16.as<float>();
   s.tmul = (float)h->scale;
   s.scale = 1.0f;
   if (residual) {
-    if (!h->has_residual)
-      throw InvalidArgument("residual int4 data was requested but is not loaded on this CUDA handle");
     s.residual = true;
-    s.rcodes = fp6_rows(h->residual6, h->residual_packed.as<uint8_t>(), h->num_tokens, h->dim);
+    s.rcodes = fp6_rows(h->residual6, h->residual_packed.as<uint8_t>(), h->num_tokens, h->dim, tokens, stream);
     s.rtscale = h->residual_token_scales16.as<float>();
     s.rmul = (float)h->residual_scale;
+  }
+  if (s.codes == nullptr || (residual && s.rcodes == nullptr)) {  // both streams as nibbles
+    s.codes = h->packed.as<uint8_t>();
+    s.rcodes = residual ? h->residual_packed.as<uint8_t>() : nullptr;
+    s.code_bytes = (int)(h->dim / 2);
   }
   return s;
 }
@@ -603,7 +647,7 @@ float* int4_score_device(msim_int4_docs* h, const float* query, int64_t batch, i
                          int reducer, const std::vector<float>& w, float temperature, const int64_t* cand,
                          int64_t m, bool residual, hipStream_t stream) {
   const int64_t targets = cand ? m : h->num_docs;
-  const DocStreams s = int4_streams(h, residual);
+  const DocStreams s = int4_streams(h, residual, target_tokens(h, targets), stream);
   const float* d_query = stage_query(h->ws, query, batch * query_tokens, dim);
   h->scores.ensure(sizeof(float) * std::max<int64_t>(1, batch * targets), "hipMalloc score cache");
   QueryInput qi;
@@ -1067,7 +1111,8 @@ extern "C" int msim_int4_cascade_topk(msim_int4_docs* h, const float* query, int
       throw InvalidArgument("residual int4 data was requested but is not loaded on this CUDA handle");
     if (batch == 0) return;
     select_device(h->device);
-    const DocStreams prefix = int4_streams(h, false), fused = int4_streams(h, true);
+    // (the prefix's tokens count as the fused stream's)
+    const DocStreams prefix = int4_streams(h, false, 0, nullptr), fused = int4_streams(h, true, h->num_tokens, nullptr);
     QueryInput qi;
     qi.d_query = stage_query(h->ws, query, batch * query_tokens, dim);
     qi.limbs = 3;
@@ -1112,8 +1157,10 @@ extern "C" int msim_int4_cascade_topk(msim_int4_docs* h, const float* query, int
 
 namespace {
 
-// limbs 3: the residual codes as fp6 rows (the fp32 query's form).
-DocStreams binres_streams(msim_binary_docs* h, bool fused, int limbs) {
+// limbs 3: the residual codes for the fp32 query, of which the call scores about
+// `tokens` on `stream`.
+DocStreams binres_streams(msim_binary_docs* h, bool fused, int limbs, int64_t tokens = 0,
+                          hipStream_t stream = nullptr) {
   if (h->dim != 128) throw InvalidArgument("binary residual scoring currently requires dim=128");
   if (!h->has_token_scale)
     throw InvalidArgument("binary residual scoring needs the prefix scales: call set_token_scale_vector first");
@@ -1126,9 +1173,12 @@ DocStreams binres_streams(msim_binary_docs* h, bool fused, int limbs) {
   s.tmul = 1.0f;
   if (fused) {
     s.residual = true;
-    if (limbs == 3) select_device(h->device);  // fp6_rows may allocate
-    s.rcodes = limbs == 3 ? fp6_rows(h->residual6, h->residual_packed.as<uint8_t>(), h->num_tokens, h->dim)
-                          : h->residual_packed.as<uint8_t>();
+    if (limbs == 3)
+      s.rcodes = fp6_rows(h->residual6, h->residual_packed.as<uint8_t>(), h->num_tokens, h->dim, tokens, stream);
+    if (s.rcodes == nullptr) {
+      s.rcodes = h->residual_packed.as<uint8_t>();
+      s.code_bytes = (int)(h->dim / 2);
+    }
     s.rtscale = h->residual_token_scales16.as<float>();
     s.rmul = (float)h->residual_scale;
   }
@@ -1198,7 +1248,8 @@ bool binres_scan_prefix(msim_binary_docs* h, const float* d_query, int64_t batch
 
 void binres_cascade(msim_binary_docs* h, const float* d_query, int64_t batch, int64_t query_tokens, int64_t k,
                     int64_t m, float* d_top_s, int64_t* d_top_i, hipStream_t stream) {
-  const DocStreams prefix = binres_streams(h, false, 1), fused = binres_streams(h, true, h->rescore_limbs);
+  const DocStreams prefix = binres_streams(h, false, 1);
+  const DocStreams fused = binres_streams(h, true, h->rescore_limbs, h->num_tokens, stream);
   QueryInput qi;
   qi.d_query = d_query;
   qi.limbs = h->rescore_limbs;
@@ -1301,7 +1352,7 @@ extern "C" int msim_binary_binres_score(msim_binary_docs* h, const float* query,
   return guarded([&] {
     require_handle(h);
     check_binary_query(h, batch, query_tokens, dim);
-    const DocStreams s = binres_streams(h, fused != 0, h->rescore_limbs);
+    binres_streams(h, fused != 0, 1);
     if (candidates) {
       if (num_candidates < 0) throw InvalidArgument("candidate_indices must have shape [batch, candidates]");
       check_candidates(candidates, batch * num_candidates, h->num_docs);
@@ -1309,6 +1360,7 @@ extern "C" int msim_binary_binres_score(msim_binary_docs* h, const float* query,
     const int64_t targets = candidates ? num_candidates : h->num_docs;
     if (batch == 0 || targets == 0) return;
     select_device(h->device);
+    const DocStreams s = binres_streams(h, fused != 0, h->rescore_limbs, target_tokens(h, batch * targets), nullptr);
     QueryInput qi;
     qi.d_query = stage_query(h->ws, query, batch * query_tokens, dim);
     qi.limbs = fused ? h->rescore_limbs : 1;
@@ -1332,9 +1384,10 @@ extern "C" int msim_binary_binres_topk(msim_binary_docs* h, const float* query, 
     require_handle(h);
     check_binary_query(h, batch, query_tokens, dim);
     check_k(k, h->num_docs);
-    const DocStreams s = binres_streams(h, true, h->rescore_limbs);
+    binres_streams(h, true, 1);
     if (batch == 0) return;
     select_device(h->device);
+    const DocStreams s = binres_streams(h, true, h->rescore_limbs, h->num_tokens, nullptr);
     QueryInput qi;
     qi.d_query = stage_query(h->ws, query, batch * query_tokens, dim);
     qi.limbs = h->rescore_limbs;
@@ -1395,7 +1448,7 @@ extern "C" int msim_int4_score_async(msim_int4_docs* h, const float* d_query, in
         row_weights(reducer, weights, weights_ndim, weights_dim0, weights_dim1, batch, query_tokens);
     if (batch == 0 || h->num_docs == 0) return;
     select_device(h->device);
-    const DocStreams s = int4_streams(h, residual != 0);
+    const DocStreams s = int4_streams(h, residual != 0, h->num_tokens, as_stream(stream));
     QueryInput qi;
     qi.d_query = d_query;
     qi.limbs = 3;

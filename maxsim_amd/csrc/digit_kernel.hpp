@@ -11,10 +11,11 @@
 // The grid keeps every bit of the row's largest elements and resolves the
 // row to 2^-25..2^-24 of max|q|.
 //
-// Documents.  int4 codes are integers up to 8, exact in e2m3 too: a handle
-// keeps a copy of its codes as fp6 rows (96 bytes per token and 128 dims,
-// encode_fp6_kernel), because unpacking nibbles to 6-bit fields in registers
-// costs about a hundred VALU instructions per tile.  Sign documents become
+// Documents.  int4 codes are integers up to 8, exact in e2m3 too.  A handle in
+// steady use keeps a copy of its codes as fp6 rows (96 bytes per token and 128
+// dims, encode_fp6_kernel), because decoding nibbles to 6-bit fields in registers
+// takes 82 VALU instructions per tile and chunk (decode_fp6: first calls,
+// candidates, no memory for the copy).  Sign documents become
 // fp4 +-1 with two instructions per dword (fp4_signs).  The MFMA's E8M0 scales
 // hold the digits' weights 32^-i, so one v_mfma_scale_f32_16x16x128_f8f6f4
 // per digit and 128 dims adds all digits into one fp32 accumulator, lowest
@@ -97,6 +98,33 @@ __device__ __forceinline__ v8i operand(const Six& x) {
 }
 __device__ __forceinline__ v8i operand(const v4i& x) { return (v8i){x[0], x[1], x[2], x[3], 0, 0, 0, 0}; }
 
+// One lane's 32 nibbles of int4 codes as the fp6 fields the copy of the corpus
+// holds (encode_fp6_kernel): 82 VALU instructions.
+__device__ __forceinline__ Six decode_fp6(const v4i& nibbles) {
+  uint32_t pair[4][4];  // [8 fields][field 2 d and 2 d + 1 as 12 bits]
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const uint32_t w = (uint32_t)nibbles[d], neg = w & 0x88888888u, one = neg >> 3;
+    const uint32_t mag = (w ^ (neg | (neg - one))) + one;  // |v| of each nibble
+    // Fields as bytes: sign bit 5, magnitude below it.
+    const uint32_t even = (mag & 0x0F0F0F0Fu) | ((neg & 0x08080808u) << 2);
+    const uint32_t odd = ((mag >> 4) & 0x0F0F0F0Fu) | ((neg & 0x80808080u) >> 2);
+    pair[0][d] = __builtin_amdgcn_udot4(even, 0x00400001u, 0u, false);
+    pair[1][d] = __builtin_amdgcn_udot4(odd, 0x00400001u, 0u, false);
+    pair[2][d] = __builtin_amdgcn_udot4(even, 0x40000100u, 0u, false);
+    pair[3][d] = __builtin_amdgcn_udot4(odd, 0x40000100u, 0u, false);
+  }
+  Six x;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {  // 16 fields, three dwords
+    const uint32_t(&a)[4] = pair[2 * h], (&b)[4] = pair[2 * h + 1];
+    x.w[3 * h] = (int)(a[0] | (a[1] << 12) | (a[2] << 24));
+    x.w[3 * h + 1] = (int)((a[2] >> 8) | (a[3] << 4) | (b[0] << 16) | (b[1] << 28));
+    x.w[3 * h + 2] = (int)((b[1] >> 4) | (b[2] << 8) | (b[3] << 20));
+  }
+  return x;
+}
+
 // acc + documents (A) x digit D of the query (B).
 template <int DOC, int D>
 __device__ __forceinline__ v4f mfma_digit(const v8i& a, const v8i& b, const v4f& c, int sa, int s03, int s4) {
@@ -144,8 +172,9 @@ __device__ __forceinline__ ReducerState<RED> swap_merge(const ReducerState<RED>&
 
 // UNIT: sign documents without token scales, MaxSim: the similarity is the
 // accumulator itself.  DIRECT: one target per wave, its document's token range
-// from p.direct_offsets; else work units.
-template <int DOC, bool RES, int NT, int RED, int KC, bool UNIT, bool DIRECT>
+// from p.direct_offsets; else work units.  RAW: int4 streams as nibbles
+// (p.code_bytes a token), decoded tile by tile: handles without the fp6 copy.
+template <int DOC, bool RES, int NT, int RED, int KC, bool UNIT, bool DIRECT, bool RAW>
 __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void digit_score_kernel(
     ScoreArgs p) {
   constexpr int kWavesPerGroup = group_waves(KC), kThreads = kWavesPerGroup * kWave;
@@ -154,7 +183,7 @@ __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void 
   constexpr int kRing = ring_size(DOC, RES, NT, KC, UNIT);
   static_assert(kRing % 2 == 0, "accumulator sets alternate over an even ring");
   constexpr int kSets = NT == 1 ? 2 : NT;  // accumulators of a step and of the step before it
-  constexpr int kCodeBytes = (DOC == kDocInt4 ? 96 : 16) * KC, kResBytes = 96 * KC, kRowBytes = 96 * KC;
+  constexpr int kCodeBytes = 16 * KC, kResBytes = 96 * KC, kRowBytes = 96 * KC;
   constexpr float kStart = UNIT ? kNegInf : 0.0f;  // accumulators before the first tile
   constexpr int kChain = kDigits * KC, kSteps = RES ? 2 * kChain : kChain;  // MFMAs of a step
 
@@ -220,11 +249,12 @@ __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void 
   }
   __builtin_amdgcn_sched_barrier(0);
 
+  using Codes = std::conditional_t<RAW, v4i, Six>;  // one chunk of an int4 stream
   struct Tile {
     uint64_t e;
-    Six code[DOC == kDocInt4 ? KC : 1];
+    Codes code[DOC == kDocInt4 ? KC : 1];
     unsigned sign[DOC == kDocSign ? KC : 1];
-    Six res[RES ? KC : 1];
+    Codes res[RES ? KC : 1];
     float s[UNIT ? 1 : 4], sr[RES ? 4 : 1];
   };
   // A tile's loads: one buffer per stream at the tile's first token, the lane's
@@ -232,24 +262,38 @@ __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void 
   // codes (or those of the kScanPadTokens zero tokens after the last one) and a
   // scale of 0 (the buffers end there: a product with the next document's scale
   // may not be finite, and -inf then does not mask it).
-  const int va = DOC == kDocInt4 ? c * kCodeBytes + 16 * g : c * kCodeBytes + 4 * g;
-  const int vr = c * kResBytes + 16 * g, vs = 16 * g;
+  const int va = c * kCodeBytes + 4 * g;  // sign documents
+  const int vr = c * kResBytes + 16 * g, vs = 16 * g, vn = RAW ? c * p.code_bytes + 16 * g : 0;
+  // (Nibbles past a token's row are the next token's, or 0 past the tile's last
+  // row: they meet zero query digits.)
+  auto load_codes = [&](const uint8_t* codes, int64_t start, int rows, Codes (&out)[KC]) __attribute__((always_inline)) {
+    if constexpr (RAW) {
+      const __amdgpu_buffer_rsrc_t r = make_rsrc(codes + start * p.code_bytes, (uint32_t)(rows * p.code_bytes));
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) {
+        const v4u w = load_b128(r, vn + 64 * kc);
+        out[kc] = (v4i){(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+      }
+    } else {
+      const __amdgpu_buffer_rsrc_t r = make_rsrc(codes + start * kResBytes, 16 * kResBytes);
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) out[kc] = load_six(r, vr + 96 * kc, vr + 96 * kc + 64 - 8 * g);
+    }
+  };
   auto load = [&](uint64_t e, Tile& t) __attribute__((always_inline)) {
     t.e = e;
     const int64_t start = (int64_t)(e & kTileStartMask);
-    const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.codes + start * kCodeBytes, 16 * kCodeBytes);
+    const int rows = (int)((e >> kTileRowsShift) & 15) + 1;
+    if constexpr (DOC == kDocInt4) {
+      load_codes(p.codes, start, rows, t.code);
+    } else {
+      const __amdgpu_buffer_rsrc_t ra = make_rsrc(p.codes + start * kCodeBytes, 16 * kCodeBytes);
 #pragma unroll
-    for (int kc = 0; kc < KC; ++kc) {
-      if constexpr (DOC == kDocInt4) t.code[kc] = load_six(ra, va + 96 * kc, va + 96 * kc + 64 - 8 * g);
-      else t.sign[kc] = load_b32(ra, va + 16 * kc);
+      for (int kc = 0; kc < KC; ++kc) t.sign[kc] = load_b32(ra, va + 16 * kc);
     }
-    if constexpr (RES) {
-      const __amdgpu_buffer_rsrc_t rr = make_rsrc(p.rcodes + start * kResBytes, 16 * kResBytes);
-#pragma unroll
-      for (int kc = 0; kc < KC; ++kc) t.res[kc] = load_six(rr, vr + 96 * kc, vr + 96 * kc + 64 - 8 * g);
-    }
+    if constexpr (RES) load_codes(p.rcodes, start, rows, t.res);
     if constexpr (!UNIT) {
-      const uint32_t scale_bytes = 4u * (uint32_t)(((e >> kTileRowsShift) & 15) + 1);
+      const uint32_t scale_bytes = 4u * (uint32_t)rows;
       const v4u sv = load_b128(make_rsrc(p.tscale + start, scale_bytes), vs);
 #pragma unroll
       for (int k = 0; k < 4; ++k) t.s[k] = __uint_as_float(sv[k]);
@@ -381,7 +425,19 @@ __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void 
   // One step: the MFMAs of row block j of tile t into accumulator set `set`.
   // Between them, from the third MFMA on, the epilogue of the step before
   // (tile P, its block jp and set), and what extra(m) puts after MFMA m.
-  auto step = [&](const Tile& t, int j, int set, const Pend& P, int jp, int setp, auto extra)
+  struct Fp6 {  // decoded streams of a tile (RAW)
+    Six code[RAW && DOC == kDocInt4 ? KC : 1], res[RAW && RES ? KC : 1];
+  };
+  auto decode = [&](const Tile& t, Fp6& f) __attribute__((always_inline)) {
+    if constexpr (RAW) {
+#pragma unroll
+      for (int kc = 0; kc < KC; ++kc) {
+        if constexpr (DOC == kDocInt4) f.code[kc] = decode_fp6(t.code[kc]);
+        if constexpr (RES) f.res[kc] = decode_fp6(t.res[kc]);
+      }
+    }
+  };
+  auto step = [&](const Tile& t, const Fp6& f, int j, int set, const Pend& P, int jp, int setp, auto extra)
                   __attribute__((always_inline)) {
     constexpr int kWait = 2, kSpan = kSteps - kWait;  // >= 3 slots
     const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -404,8 +460,9 @@ __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void 
     v8i a[KC];
 #pragma unroll
     for (int kc = 0; kc < KC; ++kc) {
-      if constexpr (DOC == kDocInt4) a[kc] = operand(t.code[kc]);
-      else a[kc] = operand(fp4_signs(t.sign[kc]));
+      if constexpr (DOC == kDocSign) a[kc] = operand(fp4_signs(t.sign[kc]));
+      else if constexpr (RAW) a[kc] = operand(f.code[kc]);
+      else a[kc] = operand(t.code[kc]);
     }
     auto digits = [&](auto digit_c, v4f& dst, const v8i (&ops)[KC], auto doc_c, int scale)
                       __attribute__((always_inline)) {
@@ -430,7 +487,10 @@ __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void 
     if constexpr (RES) {
       v8i r[KC];
 #pragma unroll
-      for (int kc = 0; kc < KC; ++kc) r[kc] = operand(t.res[kc]);
+      for (int kc = 0; kc < KC; ++kc) {
+        if constexpr (RAW) r[kc] = operand(f.res[kc]);
+        else r[kc] = operand(t.res[kc]);
+      }
       chain(accr[set], r, std::integral_constant<int, kDocInt4>{}, sr);
     }
   };
@@ -459,7 +519,9 @@ __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void 
       if (m == 1) next = next_entry();
     };
     auto none = [](int) {};
-    step(t, 0, NT == 1 ? U & 1 : 0, P, NT - 1, NT == 1 ? (U + 1) & 1 : NT - 1, fetch);
+    Fp6 f;
+    decode(t, f);
+    step(t, f, 0, NT == 1 ? U & 1 : 0, P, NT - 1, NT == 1 ? (U + 1) & 1 : NT - 1, fetch);
     const bool fresh = ((P.e >> kTileLastShift) & 1) != 0;
     len += rows_of(P.e);
     if (fresh) finish_target(P.e);
@@ -475,7 +537,7 @@ __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void 
     }
     if (len == 0) begin_target(P.e);  // (after the start's masked tile too)
 #pragma unroll
-    for (int j = 1; j < NT; ++j) step(t, j, j, P, j - 1, j - 1, none);
+    for (int j = 1; j < NT; ++j) step(t, f, j, j, P, j - 1, j - 1, none);
   };
   // Before the first tile: zero accumulators and every row masked, whose
   // epilogue changes nothing (no copy of the loop's body for the first tile:
@@ -526,20 +588,20 @@ __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void 
   finish_target(P.e);
 }
 
-template <int DOC, bool RES, int NT, int RED, int KC, bool UNIT = false>
+template <int DOC, bool RES, int NT, int RED, int KC, bool UNIT = false, bool RAW = false>
 hipError_t launch_mode(const ScoreArgs& a, dim3 grid, hipStream_t s) {
   constexpr int kThreads = kWave * group_waves(KC);
-  if (a.direct_offsets) digit_score_kernel<DOC, RES, NT, RED, KC, UNIT, true><<<grid, kThreads, 0, s>>>(a);
-  else digit_score_kernel<DOC, RES, NT, RED, KC, UNIT, false><<<grid, kThreads, 0, s>>>(a);
+  if (a.direct_offsets) digit_score_kernel<DOC, RES, NT, RED, KC, UNIT, true, RAW><<<grid, kThreads, 0, s>>>(a);
+  else digit_score_kernel<DOC, RES, NT, RED, KC, UNIT, false, RAW><<<grid, kThreads, 0, s>>>(a);
   return hipGetLastError();
 }
-template <int DOC, bool RES, int NT, int KC>
+template <int DOC, bool RES, int NT, int KC, bool RAW = false>
 hipError_t launch_reducer(const ScoreArgs& a, int reducer, dim3 grid, hipStream_t s) {
   switch (reducer) {
-    case kRedMax: return launch_mode<DOC, RES, NT, kRedMax, KC>(a, grid, s);
-    case kRedTop2: return launch_mode<DOC, RES, NT, kRedTop2, KC>(a, grid, s);
-    case kRedTop4: return launch_mode<DOC, RES, NT, kRedTop4, KC>(a, grid, s);
-    case kRedLse: return launch_mode<DOC, RES, NT, kRedLse, KC>(a, grid, s);
+    case kRedMax: return launch_mode<DOC, RES, NT, kRedMax, KC, false, RAW>(a, grid, s);
+    case kRedTop2: return launch_mode<DOC, RES, NT, kRedTop2, KC, false, RAW>(a, grid, s);
+    case kRedTop4: return launch_mode<DOC, RES, NT, kRedTop4, KC, false, RAW>(a, grid, s);
+    case kRedLse: return launch_mode<DOC, RES, NT, kRedLse, KC, false, RAW>(a, grid, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -550,6 +612,9 @@ hipError_t launch_sign(const ScoreArgs& a, bool residual, int nt, int reducer, d
 hipError_t launch_wide2(const ScoreArgs& a, int doc, bool residual, int nt, int reducer, dim3 grid, hipStream_t s);
 hipError_t launch_wide4(const ScoreArgs& a, int doc, bool residual, int nt, int reducer, dim3 grid, hipStream_t s);
 hipError_t launch_wide4_residual(const ScoreArgs& a, int nt, int reducer, dim3 grid, hipStream_t s);
+// ScoreArgs::code_bytes set.
+hipError_t launch_raw(const ScoreArgs& a, int doc, bool residual, int nt, int reducer, dim3 grid, hipStream_t s);
+hipError_t launch_raw_wide(const ScoreArgs& a, bool residual, int reducer, dim3 grid, hipStream_t s);
 
 }  // namespace digit
 }  // namespace msim

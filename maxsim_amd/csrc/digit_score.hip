@@ -186,7 +186,8 @@ hipError_t launch_digit_score(const ScoreArgs& a, int doc, bool residual, int nt
                               hipStream_t stream) {
   using namespace digit;
   if (a.subs <= 0 || groups <= 0 || a.pass_rows <= 0 || a.pass_rows > 16 * nt || a.tscale == nullptr ||
-      (residual && (a.rcodes == nullptr || a.rtscale == nullptr)))
+      (residual && (a.rcodes == nullptr || a.rtscale == nullptr)) || a.code_bytes % 4 != 0 || a.code_bytes < 0 ||
+      a.code_bytes > 64 * a.chunks)
     return hipErrorInvalidValue;
   const int64_t waves = group_waves(a.chunks);
   int64_t blocks;
@@ -206,7 +207,8 @@ hipError_t launch_digit_score(const ScoreArgs& a, int doc, bool residual, int nt
     const dim3 grid((unsigned)blocks, (unsigned)std::min(kMaxGridRows, groups * a.subs - first));
     part.first_pass = (int32_t)first;
     hipError_t e;
-    if (a.chunks == 4) e = launch_wide4(part, doc, residual, nt, reducer, grid, stream);
+    if (a.code_bytes != 0) e = launch_raw(part, doc, residual, nt, reducer, grid, stream);
+    else if (a.chunks == 4) e = launch_wide4(part, doc, residual, nt, reducer, grid, stream);
     else if (a.chunks == 2) e = launch_wide2(part, doc, residual, nt, reducer, grid, stream);
     else if (doc == kDocInt4) e = launch_int4(part, residual, nt, reducer, grid, stream);
     else e = launch_sign(part, residual, nt, reducer, grid, stream);

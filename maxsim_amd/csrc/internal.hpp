@@ -207,12 +207,14 @@ constexpr int kScoreInfoWords = 4;
 enum : int { kDocInt4 = 0, kDocSign = 1 };
 enum : int { kRedMax = 0, kRedTop2 = 1, kRedTop4 = 2, kRedLse = 3 };
 struct ScoreArgs {
-  const uint8_t* codes;        // sign bits [T, 16 chunks]; fp32 queries: or int4 as fp6 [T, 96 chunks]
+  const uint8_t* codes;        // sign bits [T, 16 chunks]; fp32 queries: or int4, see code_bytes
   const float* tscale;         // [T] per-token scale of `codes` (never null)
   float tmul;                  // constant factor of the `codes` similarity
-  const uint8_t* rcodes;       // residual int4 codes [T, 64], fp32 queries: as fp6 [T, 96 chunks]
+  const uint8_t* rcodes;       // residual int4 codes [T, 64]; fp32 queries: see code_bytes
   const float* rtscale;        // [T] residual per-token scale
   float rmul;
+  int32_t code_bytes;          // fp32 queries: int4 streams as nibbles of so many bytes per token (a multiple
+                               //   of four), 0: as fp6 rows [T, 96 chunks]
   const int64_t* wave_info;    // [groups][num_waves][kScoreInfoWords]
   const uint64_t* tiles;
   // Work units (fp32 and sign-bit queries over every document, eight waves per
