@@ -325,10 +325,10 @@ __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void 
                                 16u * g, 64u + 8u * g);
   }
   // Factors of a similarity before (int4 token scales are stored / 16) and
-  // after the reduction; one stream takes its constant factor after it.
+  // after the reduction; one stream takes its constant factor after it, before
+  // colmul (the two alone may leave the floats' range).
   const float mul = DOC == kDocInt4 ? 16.0f * p.tmul : p.tmul;
   const float after_mul = RES ? 1.0f : mul;
-  const float colmul = colmul_row * after_mul;
   const float k2 = kLog2e / p.temperature;
   int sa = DOC == kDocInt4 ? 130 : 127, sr = 130, s03 = kDigitScales, s4 = kDigitScale4;
   asm volatile("" : "+v"(sa), "+v"(sr), "+v"(s03), "+v"(s4));  // kept in VGPRs
@@ -365,7 +365,7 @@ __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void 
     const ReducerState<RED> y = NT > 2 ? swap_merge<RED>(st[NT > 2 ? 2 : 0], st[NT > 3 ? 3 : 0], sw32) : none;
     const ReducerState<RED> all = swap_merge<RED>(x, y, sw16);
     const bool empty = ((e >> kTileEmptyShift) & 1) != 0;
-    const float v = all.finish(empty ? 0 : len, colmul, p.temperature, weight, scale_of(tg));
+    const float v = all.finish(empty ? 0 : len, after_mul, colmul_row, p.temperature, weight, scale_of(tg));
 #pragma unroll
     for (int j = 0; j < NT; ++j) st[j].init();
     len = 0;

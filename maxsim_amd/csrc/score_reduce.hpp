@@ -22,8 +22,8 @@ struct ReducerState<kRedMax> {
   __device__ void init() { m = kNegInf; }
   // Two three-way maxima (v_max3_f32) for four values: exact, any order.
   __device__ void add4(const float (&z)[4]) { m = max5_op(m, z[0], z[1], z[2], z[3]); }
-  __device__ float finish(int len, float colmul, float, float weight, float doc_scale) const {
-    return len == 0 ? 0.0f : m * colmul * weight * doc_scale;
+  __device__ float finish(int len, float mul, float colmul, float, float weight, float doc_scale) const {
+    return len == 0 ? 0.0f : m * mul * colmul * weight * doc_scale;
   }
 };
 
@@ -50,14 +50,14 @@ struct TopState {
 #pragma unroll
     for (int r = 0; r < 4; ++r) insert(z[r]);
   }
-  __device__ float finish(int len, float colmul, float, float, float doc_scale) const {
+  __device__ float finish(int len, float mul, float colmul, float, float, float doc_scale) const {
     const int kept = len < K ? len : K;
     if (kept == 0) return 0.0f;
     float total = 0.0f;
 #pragma unroll
     for (int i = 0; i < K; ++i)
       if (i < kept) total += t[i];
-    return total / (float)kept * colmul * doc_scale;
+    return total / (float)kept * mul * colmul * doc_scale;
   }
 };
 template <>
@@ -101,7 +101,7 @@ struct ReducerState<kRedLse> {
     s = s * exp2_nonpos(m - mn) + so * exp2_nonpos(mo - mn);
     m = mn;
   }
-  __device__ float finish(int len, float, float temperature, float, float) const {
+  __device__ float finish(int len, float, float, float temperature, float, float) const {
     return len == 0 ? 0.0f : (m + log2f(s)) * (temperature * kLn2);
   }
 };

@@ -192,3 +192,30 @@ def test_batch_rows_cut_at_the_ends_of_passes(gpu, dim, shapes):
             np.testing.assert_array_equal(got, np.stack(each)[:, ids])
         each = [h.score_residual_batch(query[b : b + 1])[0] for b in range(shape[0])]
         np.testing.assert_array_equal(h.score_residual_batch(query), np.stack(each))
+
+
+@pytest.mark.parametrize("scale, row, token", [(1e-7, -117, 10), (1.0, 127, -20), (1e5, 120, -30)])
+def test_factors_whose_product_alone_leaves_the_floats_range(gpu, scale, row, token):
+    """Query rows, token scales and a tensor scale far from 1 whose similarities
+    are ordinary floats (rows of up to 2^row, token scales of 2^token)."""
+    from maxsim_amd._maxsim_hip import CudaInt4PackedDocs
+
+    rng = np.random.default_rng(8)
+    offsets = np.arange(0, 33 * 40, 33, dtype=np.int64)
+    tokens = int(offsets[-1])
+    values, packed = _codes(rng, tokens, 128)
+    h = CudaInt4PackedDocs(packed, offsets, 128, scale)
+    h.set_token_scale_vector(np.full(tokens, 2.0**token, np.float32))
+    query = rng.uniform(-1, 1, (2, 32, 128)).astype(np.float32) * np.float32(2.0**row)
+    docs = values * (2.0**token * float(np.float32(scale)))
+    sims = docs @ query.reshape(-1, 128).T.astype(np.float64)
+    mag = np.abs(docs) @ np.abs(query.reshape(-1, 128).T.astype(np.float64))
+    rows = _doc_max(np.abs(docs).sum(1)[:, None], offsets).T * np.abs(query.reshape(-1, 128)).max(1).astype(np.float64)[:, None]
+    shape = (2, 32, offsets.size - 1)
+    bound = _bound(query, _doc_max(mag, offsets).T.reshape(shape), rows.reshape(shape), 1, 1, 0.0)
+    ordered = np.sort(sims.reshape(offsets.size - 1, 33, 64), axis=1)[:, ::-1]
+    for reducer, k in (("maxsim", 1), ("topk2", 2), ("topk4", 4)):
+        exp = ordered[:, :k].mean(1).T.reshape(shape).sum(1)
+        got = h.score_batch(query, reducer)
+        assert np.isfinite(got).all()
+        assert (np.abs(got.astype(np.float64) - exp) <= bound).all(), reducer
