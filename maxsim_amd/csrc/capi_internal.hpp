@@ -37,7 +37,6 @@ void set_error(const std::string& msg);
 void check_hip(hipError_t e, const char* what);
 void validate_offsets(const int64_t* offsets, int64_t count, int64_t num_tokens);
 void validate_positive_scales(const float* v, int64_t n, const char* msg);
-int device_cu_count();
 int32_t docs_per_wave_for(int64_t num_docs, int waves_per_cu);
 hipStream_t as_stream(void* s);
 

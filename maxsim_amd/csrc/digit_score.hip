@@ -8,7 +8,6 @@ namespace msim {
 
 namespace {
 
-constexpr int64_t kSpreadGroups = 256;  // CUs of an MI355X
 // Tiles times passes that pay for pool_sum_kernel (2 us beside the scores it
 // reads); half of it at four chunks, whose tiles take twice as long.  Whole
 // rows / packed, the call in us: 8,200 tiles, 4 queries of 40 tokens (four
@@ -195,7 +194,7 @@ hipError_t launch_digit_score(const ScoreArgs& a, int doc, bool residual, int nt
     if (a.targets == nullptr) return hipErrorInvalidValue;
     // As many workgroups as CUs before a workgroup gets a second document:
     // a wave alone on its SIMD runs faster than one of two.
-    const int64_t spread = std::max<int64_t>(1, kSpreadGroups / (groups * a.subs));
+    const int64_t spread = std::max<int64_t>(1, device_cu_count() / (groups * a.subs));
     blocks = std::max<int64_t>((a.direct_count + waves - 1) / waves, std::min(a.direct_count, spread));
   } else {
     if (a.group_units <= 0 || a.num_waves <= 0 || a.num_waves % a.group_units != 0) return hipErrorInvalidValue;

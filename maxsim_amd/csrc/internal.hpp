@@ -8,6 +8,8 @@
 
 namespace msim {
 
+int device_cu_count();  // of the current device
+
 // Arguments of the int4 x int8-query scoring kernel (int8q.hip).
 struct Int8qArgs {
   const uint8_t* codes;       // [num_tokens, 64] int4 nibbles
