@@ -171,7 +171,7 @@ void set_units(ScoreWorkspace& ws, const std::vector<int64_t>& off, int64_t firs
   if (a.chunks > 1 && 16 * (wgs & ~7) >= 15 * wgs) wgs &= ~7;
   const ScoreTable& t =
       corpus_table(ws, first, -2 - wgs, doc_ranges((int64_t)off.size() - 1), stream, [&](auto& info, auto& tiles) {
-        return build_score_units(off.data() + first, nullptr, count, wgs, info, tiles, min_tiles);
+        return build_score_units(off.data() + first, count, wgs, min_tiles, info, tiles);
       });
   a.wave_info = t.info.as<int64_t>();
   a.tiles = t.tiles.as<uint64_t>();

@@ -318,18 +318,17 @@ hipError_t launch_pool_sum(const float* pooled, int64_t batch, int64_t query_tok
 // over about `waves` waves, balanced by tiles + 1 per target.
 void build_score_tables(const int64_t* offsets, const int64_t* targets, int64_t num_targets, int64_t waves,
                         std::vector<int64_t>& info, std::vector<uint64_t>& tiles);
-// Work units of the fp32-query scorer (ScoreArgs::group_units): the
-// targets balanced over `workgroups` lists (tiles + 1 per target, longest
-// first onto the least-loaded list), each list cut into units of whole
-// targets, longest first, every unit but the list's last of at least
-// min_tiles tiles (what a wave loads ahead); lists padded with empty records to the same
-// count, which is returned.  Tile entries hold absolute target indices, so
-// num_targets must be below 2^24 (kScoreMaxUnitTargets).
-constexpr int64_t kScoreUnitMinTiles = 4;
+// Work units of the fp32-query and Hamming scorers (ScoreArgs::group_units):
+// the documents balanced over `workgroups` lists (tiles + 1 per document,
+// longest first onto the least-loaded list), each list cut into units of whole
+// documents, longest first, every unit but the list's last of at least
+// min_tiles tiles (what a wave loads ahead); lists padded with empty records to
+// the same count, which is returned.  tiles[0] is an empty entry that ends no
+// document: what a wave loads past its list's end.  Tile entries hold document
+// indices, so num_docs is at most 2^24 (kScoreMaxUnitTargets).
 constexpr int64_t kScoreMaxUnitTargets = int64_t(1) << 24;
-int64_t build_score_units(const int64_t* offsets, const int64_t* targets, int64_t num_targets, int64_t workgroups,
-                          std::vector<int64_t>& info, std::vector<uint64_t>& tiles,
-                          int64_t min_tiles = kScoreUnitMinTiles);
+int64_t build_score_units(const int64_t* offsets, int64_t num_docs, int64_t workgroups, int64_t min_tiles,
+                          std::vector<int64_t>& info, std::vector<uint64_t>& tiles);
 
 // Cascade helpers (cascade.hip): tile tables of per-group candidate lists
 // written on the device (groups x waves waves of at most per_wave

@@ -85,16 +85,12 @@ void build_score_tables(const int64_t* off, const int64_t* targets, int64_t n, i
   }
 }
 
-int64_t build_score_units(const int64_t* off, const int64_t* targets, int64_t n, int64_t workgroups,
-                          std::vector<int64_t>& info, std::vector<uint64_t>& tiles, int64_t min_tiles) {
+int64_t build_score_units(const int64_t* off, int64_t n, int64_t workgroups, int64_t min_tiles,
+                          std::vector<int64_t>& info, std::vector<uint64_t>& tiles) {
   info.clear();
   tiles.clear();
   workgroups = std::max<int64_t>(1, std::min(workgroups, std::max<int64_t>(1, n)));
-  auto doc_of = [&](int64_t t) { return targets ? targets[t] : t; };
-  auto tiles_of = [&](int64_t t) {
-    const int64_t d = doc_of(t);
-    return std::max<int64_t>(1, (off[d + 1] - off[d] + 15) / 16);
-  };
+  auto tiles_of = [&](int64_t d) { return std::max<int64_t>(1, (off[d + 1] - off[d] + 15) / 16); };
   std::vector<int64_t> order((size_t)n);
   for (int64_t t = 0; t < n; ++t) order[(size_t)t] = t;
   std::stable_sort(order.begin(), order.end(), [&](int64_t a, int64_t b) { return tiles_of(a) > tiles_of(b); });
@@ -121,8 +117,7 @@ int64_t build_score_units(const int64_t* off, const int64_t* targets, int64_t n,
       count = 0;
     };
     for (int64_t t : mine[(size_t)w]) {
-      const int64_t d = doc_of(t);
-      const int64_t s = off[d], e = off[d + 1];
+      const int64_t s = off[t], e = off[t + 1];
       if (s == e) tiles.push_back(score_tile_entry(0, 1, true, true, t));
       for (int64_t x = s; x < e; x += 16)
         tiles.push_back(score_tile_entry(x, std::min<int64_t>(16, e - x), x + 16 >= e, false, t));
