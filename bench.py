@@ -922,13 +922,14 @@ def bench_pack(args):
 
 OTHER_CONFIGS = {3: bench_config3, 4: bench_config4, 5: bench_config5}
 
-RATE_TESTS = ("mfma", "mfma_fma2", "mfma_fma3", "mfma_fma4", "mfma_fma6", "scan_tile", "xor_bcnt", "mfma_sign")
+RATE_TESTS = ("mfma", "mfma_fma2", "mfma_fma3", "mfma_fma4", "mfma_fma6", "scan_tile", "xor_bcnt", "mfma_sign",
+              "fp6", "fp6_fma2", "fp4fp6", "fp4fp6_fma2", "fp4", "fp4_max2")
 
 
 def bench_rates(args):
     """Instruction-rate tests (no memory traffic in the loops) on every CU,
     with one and two waves per SIMD: nanoseconds per unit per SIMD (an MFMA
-    for the mfma* tests, a 16-token tile for scan_tile, a 128-bit (query row,
+    for the mfma* and fp* tests, a 16-token tile for scan_tile, a 128-bit (query row,
     token) Hamming pair for xor_bcnt and mfma_sign), and chip-wide rates."""
     import torch
 
@@ -948,12 +949,15 @@ def bench_rates(args):
         simds = 4 * cus
         if name.startswith("mfma") and name != "mfma_sign":
             row["int8_tops_2w"] = 32768 * simds / row["ns_per_unit_2w"] / 1e3
+        if name.startswith("fp"):
+            row["f8f6f4_tops_2w"] = 65536 * simds / row["ns_per_unit_2w"] / 1e3
         if name in ("xor_bcnt", "mfma_sign"):
             row["pairs_per_ns_chip_2w"] = simds / row["ns_per_unit_2w"]
         out[name] = row
         print(f"{name:10s} " + " ".join(f"{k}={v:.3f}" for k, v in row.items()), file=sys.stderr, flush=True)
     return {"metric": "instruction-rate tests", "cus": cus, "tests": out,
-            "units": {"mfma*": "one v_mfma_i32_16x16x64_i8 (with its fmas)", "scan_tile": "one 16-token tile",
+            "units": {"mfma*": "one v_mfma_i32_16x16x64_i8 (with its fmas)",
+                      "fp*": "one v_mfma_scale_f32_16x16x128_f8f6f4 (with its fmas or maxima)", "scan_tile": "one 16-token tile",
                       "xor_bcnt": "one 128-dim (query row, token) pair", "mfma_sign": "one 128-dim pair"},
             "metadata": host_metadata()}
 

@@ -12,6 +12,11 @@
 //                (accumulating), 64 (query row, token) pairs per unit
 //   mfma_sign    the same 64 pairs on the matrix core: int8 +-1 query bytes
 //                against 0/1 sign bytes, 128 dims = 2 MFMAs per 16 x 16 pairs
+//   fp6, fp4fp6, fp4          one v_mfma_scale_f32_16x16x128_f8f6f4 of e2m3 x
+//                e2m3, e2m1 x e2m3 and e2m1 x e2m1 operands (20 per unit: four
+//                accumulators, five each, in turn)
+//   fp6_fma2, fp4fp6_fma2     the same with two independent fp32 fmas after each
+//   fp4_max2     with two v_max3_f32 after each, as the Hamming scorer
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -62,6 +67,53 @@ __global__ __launch_bounds__(256) void mfma_kernel(const v4i* __restrict__ in, f
   float s = 0.0f;
   for (int k = 0; k < 8; ++k) s += f[k];
   for (int j = 0; j < 8; ++j) s += (float)(acc0[j][0] + acc1[j][3]);
+  out[blockIdx.x * 256 + threadIdx.x] = s;
+}
+
+// 20 MFMAs of fp6 / fp4 operands per unit (formats 2 and 4), NV fmas (or, MAX,
+// v_max3) after each, which read the other accumulator set.
+template <int FA, int FB, int NV, bool MAX>
+__global__ __launch_bounds__(256, 2) void mfma_f6_kernel(const v4i* __restrict__ in, float* __restrict__ out, int iters) {
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  typedef int v8i __attribute__((ext_vector_type(8)));
+  constexpr int NT = 4, ND = 5;
+  const int lane = threadIdx.x & 63;
+  auto six = [&](int at) -> v8i {
+    const v4i lo = in[64 * at + lane], hi = in[64 * (at + 1) + lane];
+    return (v8i){lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], 0, 0};
+  };
+  v8i a = six(0), b[NT][ND];
+  for (int j = 0; j < NT; ++j)
+    for (int d = 0; d < ND; ++d) b[j][d] = six(2 + j * ND + d);
+  v4f acc0[NT] = {}, acc1[NT] = {};
+  float f[8];
+  for (int k = 0; k < 8; ++k) f[k] = (float)(in[lane][k & 3] & 255);
+  const float y = f[1] * 0.00390625f;
+  auto unit = [&](v4f (&q)[NT], const v4f (&p)[NT]) {
+#pragma unroll
+    for (int d = 0; d < ND; ++d)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        q[j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(a, b[j][d], d ? q[j] : p[j], FA, FB, 0, 127, 0, 127);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          const int s = (d * NT + j) * NV + v;
+          // (max3_op's operands get no wait states from the compiler: block j's
+          // last MFMA is four back.)
+          if (MAX) f[s & 7] = max3_op(f[s & 7], p[j][2 * v], p[j][2 * v + 1]);
+          else f[s & 7] = __builtin_fmaf(f[s & 7], y, p[s & 3][(s >> 2) & 3]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+  };
+  for (int i = 0; i < iters; i += 2) {
+    unit(acc0, acc1);
+    unit(acc1, acc0);
+    a[0] ^= i;
+  }
+  float s = 0.0f;
+  for (int k = 0; k < 8; ++k) s += f[k];
+  for (int j = 0; j < NT; ++j) s += acc0[j][0] + acc1[j][3];
   out[blockIdx.x * 256 + threadIdx.x] = s;
 }
 
@@ -207,13 +259,20 @@ extern "C" int msim_rate_test(const char* name, int cus, int waves_per_simd, int
     else if (!strcmp(name, "mfma_fma6")) mfma_kernel<6><<<wgs, 256>>>(vi, dout, iters);
     else if (!strcmp(name, "scan_tile")) scan_tile_kernel<<<wgs, 256>>>(vu, dout, iters);
     else if (!strcmp(name, "xor_bcnt")) xor_bcnt_kernel<<<wgs, 256>>>(vu, dout, iters);
+    else if (!strcmp(name, "fp6")) mfma_f6_kernel<2, 2, 0, false><<<wgs, 256>>>(vi, dout, iters);
+    else if (!strcmp(name, "fp6_fma2")) mfma_f6_kernel<2, 2, 2, false><<<wgs, 256>>>(vi, dout, iters);
+    else if (!strcmp(name, "fp4fp6")) mfma_f6_kernel<4, 2, 0, false><<<wgs, 256>>>(vi, dout, iters);
+    else if (!strcmp(name, "fp4fp6_fma2")) mfma_f6_kernel<4, 2, 2, false><<<wgs, 256>>>(vi, dout, iters);
+    else if (!strcmp(name, "fp4")) mfma_f6_kernel<4, 4, 0, false><<<wgs, 256>>>(vi, dout, iters);
+    else if (!strcmp(name, "fp4_max2")) mfma_f6_kernel<4, 4, 2, true><<<wgs, 256>>>(vi, dout, iters);
     else if (!strcmp(name, "mfma_sign")) mfma_sign_kernel<<<wgs, 256>>>(vi, dout, iters);
     else return false;
     return true;
   };
-  // Units: mfma*: per MFMA (16 per iteration); xor_bcnt: per pair (8 x 64
+  // Units: mfma*, fp*: per MFMA (16, 20 per iteration); xor_bcnt: per pair (8 x 64
   // per iteration and wave); mfma_sign: per pair (2048 per iteration).
   if (!strncmp(name, "mfma_fma", 8) || !strcmp(name, "mfma")) mult = 16.0;
+  else if (!strncmp(name, "fp", 2)) mult = 20.0;
   else if (!strcmp(name, "xor_bcnt")) mult = 8.0 * 64.0;
   else if (!strcmp(name, "mfma_sign")) mult = 2048.0;
   hipEvent_t e0 = nullptr, e1 = nullptr;

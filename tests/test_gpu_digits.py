@@ -70,6 +70,7 @@ def test_digit_scores_at_the_edges(gpu, oracle, kind, dim, shape):
     flat = query.reshape(-1, dim)
     flat[0] = 0.0
     flat[-1, 0] = 64.0  # one element far above the rest of its row
+    near = query.copy()
     if shape[0] > 1:  # whole batch rows far from the others
         query[1] *= np.float32(1e30)
         query[-1] *= np.float32(1e-41) if shape[0] > 2 else np.float32(1)
@@ -78,12 +79,12 @@ def test_digit_scores_at_the_edges(gpu, oracle, kind, dim, shape):
     mag = np.abs(docs).astype(np.float64)
     if kind == "residual":
         mag = np.abs(values * scale[:, None]).astype(np.float64) + np.abs(values2 * scale2[:, None])
-    q64 = np.abs(flat).astype(np.float64)
-    sims = _doc_max(mag @ q64.T, offsets).T.reshape(*shape, lengths.size)
-    rows = (_doc_max(mag.sum(1)[:, None], offsets).T * q64.max(1)[:, None]).reshape(*shape, lengths.size)
     for reducer, temperature in (("maxsim", 0.0), ("topk2", 0.0), ("topk4", 0.0), ("smoothsim", 0.5)):
-        if reducer == "smoothsim" and shape[0] > 1:
-            continue  # exponents of rows of 1e30
+        if reducer == "smoothsim":
+            query = near  # (no exponents of rows of 1e30)
+        q64 = np.abs(query.reshape(-1, dim)).astype(np.float64)
+        sims = _doc_max(mag @ q64.T, offsets).T.reshape(*shape, lengths.size)
+        rows = (_doc_max(mag.sum(1)[:, None], offsets).T * q64.max(1)[:, None]).reshape(*shape, lengths.size)
         args = {"temperature": temperature} if reducer == "smoothsim" else {}
         got = score(query, reducer, None, **args, **kw)
         exp = oracle.dense_scores(query, docs, offsets, reducer=reducer, **args)
