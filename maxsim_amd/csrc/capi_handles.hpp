@@ -17,7 +17,8 @@ struct ScoreTable {
   int64_t waves = 0;      // records
   int64_t units = 0;      // records per workgroup (build_score_units), else 0
   bool captured = false;  // a captured graph reads it: kept as long as the handle
-  DeviceBuffer info, tiles;
+  int64_t info_at = 0;    // bytes from `data` to the records, behind the tile entries
+  DeviceBuffer data;
 };
 // Work splits whose tables a handle keeps (half a byte per token each);
 // dropping a table frees its memory, for which hipFree waits until the device
@@ -40,7 +41,7 @@ struct ScoreWorkspace {
   HostBuffer host_query, host_out, host_ids;
   uint64_t bytes() const {
     uint64_t table_bytes = 0;
-    for (const auto& t : tables) table_bytes += t->info.cap + t->tiles.cap;
+    for (const auto& t : tables) table_bytes += t->data.cap;
     return qpack.cap + qpack_alt.cap + colmul.cap + qsum.cap + weights.cap + pooled.cap + qbits.cap + table_bytes +
            cand_ids.cap + cand_info.cap + cand_tiles.cap + coarse.cap + top_m_scores.cap + top_m_ids.cap + fine.cap +
            topk_scratch.cap;

@@ -119,7 +119,9 @@ int64_t doc_ranges(int64_t num_docs) { return ceil_div(num_docs, kScoreMaxUnitTa
 
 // The table of `split` over the documents from `first` on; build(info, tiles)
 // makes it, returning the records per workgroup (or 0), at the first call that
-// asks for it.  `ranges`: tables a call of one split uses.
+// asks for it: one copy, before the call's launches, which it would wait for
+// (both arrays by themselves, behind the query's launch: 35 us more of a first
+// search).  `ranges`: tables a call of one split uses.
 template <typename Build>
 const ScoreTable& corpus_table(ScoreWorkspace& ws, int64_t first, int64_t split, int64_t ranges, hipStream_t stream,
                                Build build) {
@@ -134,19 +136,20 @@ const ScoreTable& corpus_table(ScoreWorkspace& ws, int64_t first, int64_t split,
     t->split = split;
     t->units = build(info, tiles);
     t->waves = (int64_t)info.size() / kScoreInfoWords;
+    tiles.resize((tiles.size() + 3) & ~(size_t)3);  // (records of 32 bytes behind the entries)
+    t->info_at = (int64_t)(sizeof(uint64_t) * tiles.size());
+    tiles.insert(tiles.end(), info.begin(), info.end());
+    const size_t bytes = sizeof(uint64_t) * tiles.size();
     drop_tables(ws, kScoreTablesKept * (size_t)ranges - 1);
-    auto upload = [&] {
-      upload_vec(t->info, info, "copy score wave table to device");
-      upload_vec(t->tiles, tiles, "copy score tile table to device");
-      check_hip(hipStreamSynchronize(nullptr), "synchronize score tables");
-    };
     try {
-      upload();
+      t->data.ensure(bytes, "hipMalloc score tables");
     } catch (const OutOfDeviceMemory&) {
       (void)hipGetLastError();  // (a later launch would report it)
       drop_tables(ws, 0);       // the other tables make room
-      upload();
+      t->data.ensure(bytes, "hipMalloc score tables");
     }
+    check_hip(hipMemcpy(t->data.ptr, tiles.data(), bytes, hipMemcpyHostToDevice), "copy score tables to device");
+    check_hip(hipStreamSynchronize(nullptr), "synchronize score tables");
     tables.push_back(std::move(t));
     at = tables.size() - 1;
   }
@@ -156,6 +159,12 @@ const ScoreTable& corpus_table(ScoreWorkspace& ws, int64_t first, int64_t split,
       capture != hipStreamCaptureStatusNone)
     tables[0]->captured = true;
   return *tables[0];
+}
+
+void set_table(ScoreArgs& a, const ScoreTable& t) {
+  a.wave_info = reinterpret_cast<const int64_t*>(t.data.as<char>() + t.info_at);
+  a.tiles = t.data.as<uint64_t>();
+  a.num_waves = t.waves;
 }
 
 // Documents first .. first + count - 1 as work units for `workgroups`
@@ -173,9 +182,7 @@ void set_units(ScoreWorkspace& ws, const std::vector<int64_t>& off, int64_t firs
       corpus_table(ws, first, -2 - wgs, doc_ranges((int64_t)off.size() - 1), stream, [&](auto& info, auto& tiles) {
         return build_score_units(off.data() + first, count, wgs, min_tiles, info, tiles);
       });
-  a.wave_info = t.info.as<int64_t>();
-  a.tiles = t.tiles.as<uint64_t>();
-  a.num_waves = t.waves;
+  set_table(a, t);
   a.group_units = (int32_t)t.units;
 }
 
@@ -236,10 +243,12 @@ void run_digit_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int64_
     staged = stage_ids(ws, t.host, ids);
     ws.cand_ids.ensure(sizeof(int64_t) * std::max<int64_t>(ids, 1), "hipMalloc candidates");
   }
-  if (!q.quantized)
-    check_hip(launch_quantize_digits(q.d_query, rows, rows_padded, ws.qpack.as<uint8_t>(), ws.colmul.as<float>(),
-                                     s.chunks, staged, ws.cand_ids.as<int64_t>(), ids, stream),
-              "launch query digit kernel");
+  auto quantize = [&] {
+    if (!q.quantized)
+      check_hip(launch_quantize_digits(q.d_query, rows, rows_padded, ws.qpack.as<uint8_t>(), ws.colmul.as<float>(),
+                                       s.chunks, staged, ws.cand_ids.as<int64_t>(), ids, stream),
+                "launch query digit kernel");
+  };
 
   ScoreArgs a{};
   set_streams(a, s);
@@ -276,6 +285,7 @@ void run_digit_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int64_
     a.targets_grp_stride = t.per_row ? t.count : 0;
     a.direct_offsets = t.d_offsets;
     a.direct_count = t.count;
+    quantize();
     score(t.count, d_out);
     return;
   }
@@ -284,6 +294,7 @@ void run_digit_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int64_
     set_units(ws, off, first, count, device_cu_count(), plan.subs, s.doc == kDocSign ? kDigitUnitSign : kDigitUnitInt4,
               a, stream);
     a.doc_scale = s.doc_scale ? s.doc_scale + first : nullptr;
+    if (first == 0) quantize();  // (behind the table's copy)
     score(count, d_out + first);
   }
 }
@@ -326,26 +337,7 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
     return;
   }
 
-  // 1. Quantise the query rows.
-  ws.qpack.ensure((size_t)rows_padded * 128, "hipMalloc query codes");
-  ws.colmul.ensure(sizeof(float) * rows_padded, "hipMalloc query scales");
-  ws.qsum.ensure(sizeof(int32_t) * rows_padded, "hipMalloc query code sums");
-  if (q.alt_int4) ws.qpack_alt.ensure((size_t)rows_padded * 128, "hipMalloc query codes (int4 layout)");
-  if (q.quantized || q.from_alt) {
-    // reuse the workspace's quantised rows
-  } else if (q.d_qbits)
-    check_hip(launch_quantize_bits(q.d_qbits, rows, rows_padded, ws.qpack.as<int8_t>(), ws.colmul.as<float>(),
-                                   ws.qsum.as<int32_t>(), stream),
-              "launch sign query kernel");
-  else
-    // A sign stream paired with an int4 residual is unpacked in the int4
-    // lane order, so both share the int4 query layout.
-    check_hip(launch_quantize_limbs(q.d_query, rows, rows_padded, s.residual ? kDocInt4 : s.doc, q.recip,
-                                    ws.qpack.as<int8_t>(), ws.colmul.as<float>(), ws.qsum.as<int32_t>(), stream,
-                                    kDocInt4, q.alt_int4 ? ws.qpack_alt.as<int8_t>() : nullptr),
-              "launch query quantize kernel");
-
-  // 2. Work split.
+  // 1. Work split.
   const int64_t groups = t.per_row ? batch : 1;
   const int64_t grp_rows = t.per_row ? query_tokens : rows;
   const int64_t rpp = score_rows_per_pass(grp_rows);
@@ -396,11 +388,28 @@ void run_generic_score(ScoreWorkspace& ws, const std::vector<int64_t>& off, int6
       build_score_tables(off.data(), nullptr, num_docs, waves, info, tiles);
       return 0;
     });
-    a.wave_info = tab.info.as<int64_t>();
-    a.tiles = tab.tiles.as<uint64_t>();
-    a.num_waves = tab.waves;
+    set_table(a, tab);
     a.info_grp_stride = 0;
   }
+
+  // 2. Quantise the query rows.
+  ws.qpack.ensure((size_t)rows_padded * 128, "hipMalloc query codes");
+  ws.colmul.ensure(sizeof(float) * rows_padded, "hipMalloc query scales");
+  ws.qsum.ensure(sizeof(int32_t) * rows_padded, "hipMalloc query code sums");
+  if (q.alt_int4) ws.qpack_alt.ensure((size_t)rows_padded * 128, "hipMalloc query codes (int4 layout)");
+  if (q.quantized || q.from_alt) {
+    // reuse the workspace's quantised rows
+  } else if (q.d_qbits)
+    check_hip(launch_quantize_bits(q.d_qbits, rows, rows_padded, ws.qpack.as<int8_t>(), ws.colmul.as<float>(),
+                                   ws.qsum.as<int32_t>(), stream),
+              "launch sign query kernel");
+  else
+    // A sign stream paired with an int4 residual is unpacked in the int4
+    // lane order, so both share the int4 query layout.
+    check_hip(launch_quantize_limbs(q.d_query, rows, rows_padded, s.residual ? kDocInt4 : s.doc, q.recip,
+                                    ws.qpack.as<int8_t>(), ws.colmul.as<float>(), ws.qsum.as<int32_t>(), stream,
+                                    kDocInt4, q.alt_int4 ? ws.qpack_alt.as<int8_t>() : nullptr),
+              "launch query quantize kernel");
 
   // 3. Score; the batch-row sums over query tokens are taken in the kernel
   // or by pool_sum_kernel over pooled[target][row].
