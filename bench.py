@@ -57,11 +57,10 @@ RAMP_US = 2.1
 TAIL_US = 4.8
 # Config 3's MaxSim score launch: its loop issues 20 fp6 MFMAs
 # (v_mfma_scale_f32_16x16x128_f8f6f4) per 16-token tile and pass (five digits,
-# four row blocks) with about two other VALU instructions each, which a rate
-# test of that mix on random operands puts at 12.3 ns per MFMA and SIMD (11.2 ns
-# without the VALU).  Ramp and tail: the first tile's latency and the last
+# four row blocks) with about two other VALU instructions each, a mix that takes
+# 12.36 ns per MFMA and SIMD (--rates, fp6_fma2; 9.97 without the VALU).  Ramp and tail: the first tile's latency and the last
 # waves' end, about 2 us and 1 us.
-MIX3_NS_PER_MFMA = 12.3
+MIX3_NS_PER_MFMA = 12.36
 MFMA_FP6_PEAK_TOPS = 10066.0  # 1024 SIMDs x 2 x 16 x 16 x 128 per 16 cycles at 2.4 GHz
 RAMP3_US = 2.0
 TAIL3_US = 1.0

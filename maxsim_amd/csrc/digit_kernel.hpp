@@ -19,23 +19,27 @@
 // fp4 +-1 with two instructions per dword (fp4_signs).  The MFMA's E8M0 scales
 // hold the digits' weights 32^-i, so one v_mfma_scale_f32_16x16x128_f8f6f4
 // per digit and 128 dims adds all digits into one fp32 accumulator, lowest
-// digit first (measured: each MFMA's 128 products are summed exactly and
-// rounded once with the accumulator, so the smaller digits keep their bits
-// until the last steps; dots against float64: 3.1e-8 rms, a plain fp32 dot
-// 5.6e-8).  A similarity is then one fma (times the token scale, the row mask
-// as addend), or nothing for sign documents without token scales.
+// digit first, so that the smaller digits keep their bits until the last steps.
+// Each MFMA rounds: it cuts the accumulator at about 2^-25 of its largest
+// product's power of two, downwards, and rounds its partial sums.  Similarities
+// of unit queries against float64, int4 of 64..512 dims: 8.5e-8..1.1e-7 (2-norm,
+// relative), of queries whose elements spread widely 1.5e-7..3.7e-7; three int8
+// limbs 1.0e-7..1.2e-7 and 2.2e-7..5.5e-7.  A similarity is then one fma (times
+// the token scale, the row mask as addend), or nothing for sign documents
+// without token scales.
 //
 // Why digits rather than int8 limbs: three exact int8 limb dots need six MFMAs
 // of 64 dims per 16 x 16 block and 4.5 VALU instructions per similarity to
 // recombine (9 for sign documents); five MFMAs of 128 dims and one (or no)
-// VALU instruction do the same.  Rates measured per MFMA and SIMD, two waves,
-// random operands: i8 16x16x64 7.9 ns, fp6 x fp6 16x16x128 11.2 ns, fp4 x fp6
-// 9.5 ns.  MaxSim launches before (three limbs) and now, 32 query tokens:
-//   int4, 16,384 documents of 64..192 tokens, 4 queries   117.6 -> 93.0 us
-//   int4,  4,096 of the same, 2 queries                    20.8 -> 19.7 us
-//   signs, 10,240 documents of 256..1,024 tokens, 1 / 2    125 / 206 -> 76 / 117 us
-// (80 ns per 16 x 16 block of int4 at four blocks, 73 of signs, against 56 and 48
-// of the MFMAs alone; one int4 query is bound by memory, 6.4 TB/s of fp6 rows.)
+// VALU instruction do the same.  Rates per MFMA and SIMD, two waves
+// (microbench/rates.hip): i8 16x16x64 9.1 ns, fp6 x fp6 16x16x128 10.0, fp4 x fp6
+// 9.4; with two fmas after each 10.0, 12.4 and 11.7.  MaxSim launches with three
+// limbs and now, 32 query tokens:
+//   int4, 16,384 documents of 64..192 tokens, 4 queries   117.6 -> 79.7 us
+//   int4,  4,096 of the same, 2 queries                    20.8 -> 17.6 us
+//   signs, 10,240 documents of 256..1,024 tokens, 1 / 2    125 / 206 -> 62 / 96 us
+// (74 ns per 16 x 16 block of int4 at four blocks, 59 of signs, against 50 and 47
+// of the MFMAs alone; one int4 query, 35.7 us, is bound by memory.)
 //
 // Work split: the waves of a workgroup (group_waves) share one pass of
 // query rows; its digits are staged once in LDS and held in registers (NT
@@ -43,9 +47,9 @@
 // (the MFMA's A operand), held in a ring of registers filled by buffer loads
 // (an address is a descriptor in SGPRs and a constant offset: 64-bit VGPR
 // addresses would share registers with pending loads and make the compiler wait
-// for them, 101 us where this takes 93; filling the ring in LDS by DMA took
-// 120), from work units its workgroup's waves take from a
-// counter in LDS (every document), or of one candidate document per wave.
+// for them, 9 % slower; filling the ring in LDS by DMA took 29 % longer), from
+// work units its workgroup's waves take from a counter in LDS (every document),
+// or of one candidate document per wave.
 // Step j of a tile issues row block j's MFMAs; the epilogue of the block one
 // step back (the previous tile's last block for j = 0) is spread between them
 // from the third MFMA on, so that its accumulators are at least two further
@@ -134,8 +138,9 @@ __device__ __forceinline__ v4f mfma_digit(const v8i& a, const v8i& b, const v4f&
 }
 
 // Tiles held per wave (one computed, the rest in flight): what the registers
-// left by the query digits take (rings of eight at four chunks were no faster).  Signs are small (256 bytes per tile), so
-// only many of them in flight cover the memory latency.
+// left by the query digits take (rings of eight at four chunks were no faster).
+// Signs are small (256 bytes per tile), so only many of them in flight cover the
+// memory latency.
 constexpr int ring_size(int doc, bool res, int nt, int kc, bool unit) {
   if (doc == kDocSign && !res && kc == 1) return unit ? 8 : nt == 4 ? 4 : 8;
   if (kc == 4) return res && nt == 2 ? 2 : 4;
@@ -372,7 +377,10 @@ __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void 
     const int64_t b0 = grow0 / p.query_tokens;
     if (sum_regs) {
       // 32-token queries: a batch row's token l and l + 16 are 32 lanes apart
-      // (lane groups g and g + 2), summed in token_sum16's order.
+      // (lane groups g and g + 2), summed in token_sum16's order.  Of no other
+      // length do two whole 16-row blocks make a batch row; those go through LDS,
+      // at most 3 % slower (16,384 documents, 31 / 32 tokens, the call: 1 query
+      // 38.7 / 38.3 us, 2 49.1 / 47.7, 4 85.1 / 83.5).
       float w = v, o = 0.0f;
       const auto r = sw32(__float_as_uint(w), __float_as_uint(o));  // upper half of w over the lower of o
       w = row_butterfly16(__uint_as_float(r[0]) + __uint_as_float(r[1]));

@@ -22,10 +22,11 @@
 //
 // Measured, 10,240 documents of 256..1,024 tokens, queries of 32 tokens (before:
 // passes of always 256 rows, a tile's maxima behind a fence, tables of one
-// list per wave): 1 query 115 -> 33 us, 4 queries 115 -> 55, 8: 115 -> 91 (kernel);
-// 256: 3,380 -> 2,154 (call; 10.1 ns per block and SIMD, the MFMAs alone 8.1 to
-// 8.6).  One workgroup per CU instead of two: 15 % slower; units followed by
-// position instead of TileStream's running pointer: another 8 %.
+// list per wave): 1 query 115 -> 33 us, 4 queries 115 -> 54, 8: 115 -> 84 (kernel);
+// 256: 3,380 -> 2,137 (10.3 ns per block and SIMD; MFMAs alone 8.7 at two waves per
+// SIMD, with two maxima after each 10.9: microbench/rates.hip).  One workgroup
+// per CU instead of two: 15 % slower; units followed by position instead of
+// TileStream's running pointer: another 8 %.
 #include <algorithm>
 
 #include "common.hpp"
@@ -134,7 +135,9 @@ __global__ __launch_bounds__(kGroupThreads, 4) void hamming_kernel(ScoreArgs p) 
     if (sum_regs) {
       // 32-token queries: tokens l and l + 16 of a batch row are 32 lanes
       // apart; two quads' sums (batch rows 4 i .. 4 i + 3) in one register,
-      // one batch row per lane group.
+      // one batch row per lane group.  Of no other length do two whole 16-row
+      // blocks make a batch row; those go through LDS, about 1 % slower (31 / 32
+      // tokens, the call: 4 queries 52.8 / 52.5 us, 8 84.3 / 83.5, 32 288 / 285).
 #pragma unroll
       for (int i = 0; i < kQuads; i += 2) {
         const auto r = __builtin_amdgcn_permlane32_swap(
