@@ -555,6 +555,11 @@ def bench_config2(args):
 FP32_PEAK_TFLOPS = 157.3
 
 
+# Calls after which an fp32-query handle is in steady use: its 33rd search makes
+# the fp6 copy of its codes, once.
+STEADY_CALLS = 40
+
+
 def _timed(step, steps, warmup, stream):
     """Wall ms per step over `steps` back-to-back steps, and per-step event ms."""
     import torch
@@ -611,6 +616,8 @@ def bench_config3(args):
     scores = torch.empty((b, n), dtype=torch.float32, device="cuda")
     ts = torch.empty((b, args.k), dtype=torch.float32, device="cuda")
     ti = torch.empty((b, args.k), dtype=torch.int64, device="cuda")
+    for _ in range(STEADY_CALLS):
+        check(lib.msim_int4_score_async(h._h, ptr(dq), b, q, b"maxsim", None, 0, 0, 0, 1.0, 0, ptr(scores), sptr))
     per = {}
     for red in ("maxsim", "weighted_maxsim", "topk2", "topk4", "smoothsim"):
         w = weights if red == "weighted_maxsim" else None
@@ -821,6 +828,8 @@ def bench_config5(args):
     # The same cascade with the rescoring pass on the fp32 query,
     # against the fused scan of every document on the fp32 query.
     h.set_rescore_limbs(3)
+    for _ in range(STEADY_CALLS):
+        step()
     fp32_wall, _ = _timed(step, args.steps, args.warmup, stream)
     fp32_full_wall, _ = _timed(full, args.steps, args.warmup, stream)
     h.set_rescore_limbs(1)

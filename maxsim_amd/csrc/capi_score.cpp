@@ -564,11 +564,11 @@ void copy_scores_out(ScoreWorkspace& ws, void* out, const void* d, size_t bytes)
 // beyond the first search, or 32 searches.  A handle that serves one search, or
 // short candidate lists, keeps to the memory of its corpus.  From nibbles / from
 // the copy, calls of 4 queries of 32 tokens: 4,096 documents 64 / 53 us, 16,384
-// 157 / 115; a first call with the copy / without, 512 documents 450 / 189 us, of
-// 100 candidates 354 / 94.  The copy takes at most half of the free device
-// memory, or is tried again much later; it is waited for, so that a later call
-// may come on any stream; and a captured call makes none.  Rows the kernel cannot
-// load (dims that are no multiple of 8) are copied at once.
+// 157 / 115; a first call that made the copy took 260 us longer (512 documents or
+// 100 candidates).  The copy takes at most half of the free device memory, or is
+// tried again much later; it is waited for, so that a later call may come on any
+// stream; and a captured call makes none.  Rows the kernel cannot load (dims that
+// are no multiple of 8) are copied at once.
 const uint8_t* fp6_rows(Fp6Copy& copy, const uint8_t* codes, int64_t num_tokens, int64_t dim, int64_t tokens,
                         hipStream_t stream) {
   if (copy.rows.ptr != nullptr || num_tokens == 0) return copy.rows.as<uint8_t>();
