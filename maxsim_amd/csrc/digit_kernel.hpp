@@ -14,7 +14,7 @@
 // Documents.  int4 codes are integers up to 8, exact in e2m3 too.  A handle in
 // steady use keeps a copy of its codes as fp6 rows (96 bytes per token and 128
 // dims, encode_fp6_kernel), because decoding nibbles to 6-bit fields in registers
-// takes 82 VALU instructions per tile and chunk (decode_fp6: first calls,
+// takes 37 VALU instructions per tile and chunk (decode_fp6: first calls,
 // candidates, no memory for the copy).  Sign documents become
 // fp4 +-1 with two instructions per dword (fp4_signs).  The MFMA's E8M0 scales
 // hold the digits' weights 32^-i, so one v_mfma_scale_f32_16x16x128_f8f6f4
@@ -103,8 +103,46 @@ __device__ __forceinline__ v8i operand(const Six& x) {
 __device__ __forceinline__ v8i operand(const v4i& x) { return (v8i){x[0], x[1], x[2], x[3], 0, 0, 0, 0}; }
 
 // One lane's 32 nibbles of int4 codes as the fp6 fields the copy of the corpus
-// holds (encode_fp6_kernel): 82 VALU instructions.
+// holds (encode_fp6_kernel): 37 VALU instructions.  Nibbles q and q + 4 of a dword
+// lie 16 bits apart and are elements 8 q + 2 d and the next one of the operand:
+// with bit 3 flipped under the exponent of 1024 they are the halves 1024 + v + 8 (or,
+// in bits 4..7, 1024 + 16 (v + 8)), one fma makes them v / 8, exactly, and one
+// conversion packs all 32.  Against decode_fp6_lean, calls over 3,000 documents, 4
+// queries of 32 tokens / one of 8: 128 dims 62.6 -> 59.6 / 35.1 -> 33.7 us, residual
+// 82.8 -> 75.9 / 43.1 -> 40.1, 256 dims 97 -> 91 / 42.9 -> 40.2, residual 151 -> 125 /
+// 58.0 -> 51.8, 512 dims 173 -> 149 / 71.5 -> 55.1 (and a kernel of 16 rows), residual
+// 280 -> 231 / 103 -> 77.
 __device__ __forceinline__ Six decode_fp6(const v4i& nibbles) {
+  typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+  typedef _Float16 v32h __attribute__((ext_vector_type(32)));
+  union {
+    v2h pair[16];
+    v32h all;
+  } h;
+  uint32_t flip_lo = 0x64086408u, flip_hi = 0x64806480u;
+  asm("" : "+v"(flip_lo), "+v"(flip_hi));  // in VGPRs: and + xor is one v_bitop3_b32
+  auto eighths = [&](uint32_t w, bool hi) __attribute__((always_inline)) -> v2h {
+    const _Float16 unit = hi ? (_Float16)0.0078125f : (_Float16)0.125f, bias = hi ? (_Float16)-9.0f : (_Float16)-129.0f;
+    const uint32_t x = hi ? (w & 0x00F000F0u) ^ flip_hi : (w & 0x000F000Fu) ^ flip_lo;
+    return __builtin_elementwise_fma(__builtin_bit_cast(v2h, x), (v2h){unit, unit}, (v2h){bias, bias});
+  };
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const uint32_t w = (uint32_t)nibbles[d], w8 = w >> 8;
+    h.pair[d] = eighths(w, false);
+    h.pair[4 + d] = eighths(w, true);
+    h.pair[8 + d] = eighths(w8, false);
+    h.pair[12 + d] = eighths(w8, true);
+  }
+  const auto f = __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(h.all, 1.0f);
+  return {{(int)f[0], (int)f[1], (int)f[2], (int)f[3], (int)f[4], (int)f[5]}};
+}
+
+// The same in 82 instructions, sign and magnitude by bit operations, fields joined
+// by dot products, without the 16 registers of halves: for the kernels that would
+// spill 30 registers for them (residual, two chunks, TopK4 and SmoothSim: 60 us
+// where those take 74, of 4 queries 158 against 186).
+__device__ __forceinline__ Six decode_fp6_lean(const v4i& nibbles) {
   uint32_t pair[4][4];  // [8 fields][field 2 d and 2 d + 1 as 12 bits]
 #pragma unroll
   for (int d = 0; d < 4; ++d) {
@@ -440,8 +478,9 @@ __global__ __launch_bounds__(kWave * group_waves(KC), group_waves(KC) / 4) void 
     if constexpr (RAW) {
 #pragma unroll
       for (int kc = 0; kc < KC; ++kc) {
-        if constexpr (DOC == kDocInt4) f.code[kc] = decode_fp6(t.code[kc]);
-        if constexpr (RES) f.res[kc] = decode_fp6(t.res[kc]);
+        constexpr bool kLean = RES && KC == 2 && (RED == kRedTop4 || RED == kRedLse);
+        if constexpr (DOC == kDocInt4) f.code[kc] = kLean ? decode_fp6_lean(t.code[kc]) : decode_fp6(t.code[kc]);
+        if constexpr (RES) f.res[kc] = kLean ? decode_fp6_lean(t.res[kc]) : decode_fp6(t.res[kc]);
       }
     }
   };
@@ -622,7 +661,7 @@ hipError_t launch_wide4(const ScoreArgs& a, int doc, bool residual, int nt, int 
 hipError_t launch_wide4_residual(const ScoreArgs& a, int nt, int reducer, dim3 grid, hipStream_t s);
 // ScoreArgs::code_bytes set.
 hipError_t launch_raw(const ScoreArgs& a, int doc, bool residual, int nt, int reducer, dim3 grid, hipStream_t s);
-hipError_t launch_raw_wide(const ScoreArgs& a, bool residual, int reducer, dim3 grid, hipStream_t s);
+hipError_t launch_raw_wide(const ScoreArgs& a, bool residual, int nt, int reducer, dim3 grid, hipStream_t s);
 
 }  // namespace digit
 }  // namespace msim
