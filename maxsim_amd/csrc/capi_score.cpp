@@ -562,10 +562,10 @@ void copy_scores_out(ScoreWorkspace& ws, void* out, const void* d, size_t bytes)
 // the corpus, takes about 300 us (an allocation; encoding half a million tokens
 // 30 us), so it is made once decoding may have cost as much: after 2^24 tokens
 // beyond the first search, or 32 searches.  A handle that serves one search, or
-// short candidate lists, keeps to the memory of its corpus.  From nibbles / from
-// the copy, calls of 4 queries of 32 tokens: 4,096 documents 64 / 53 us, 16,384
-// 157 / 115; a first call that made the copy took 260 us longer (512 documents or
-// 100 candidates).  The copy takes at most half of the free device memory, or is
+// short candidate lists, keeps to the memory of its corpus.  Kernel from nibbles /
+// from the copy, 32-token queries: 4 over 4,096 documents 35.8 / 27.2 us, one over
+// 16,384 46.1 / 35.8; a first call that made the copy took 260 us longer (512
+// documents or 100 candidates).  The copy takes at most half of the free device memory, or is
 // tried again much later; it is waited for, so that a later call may come on any
 // stream; and a captured call makes none.  Rows the kernel cannot load (dims that
 // are no multiple of 8) are copied at once.

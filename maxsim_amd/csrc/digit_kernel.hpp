@@ -35,11 +35,11 @@
 // (microbench/rates.hip): i8 16x16x64 9.1 ns, fp6 x fp6 16x16x128 10.0, fp4 x fp6
 // 9.4; with two fmas after each 10.0, 12.4 and 11.7.  MaxSim launches with three
 // limbs and now, 32 query tokens:
-//   int4, 16,384 documents of 64..192 tokens, 4 queries   117.6 -> 79.7 us
-//   int4,  4,096 of the same, 2 queries                    20.8 -> 17.6 us
+//   int4, 16,384 documents of 64..192 tokens, 4 queries   117.6 -> 79.3 us
+//   int4,  4,096 of the same, 2 queries                    20.8 -> 17.4 us
 //   signs, 10,240 documents of 256..1,024 tokens, 1 / 2    125 / 206 -> 62 / 96 us
-// (74 ns per 16 x 16 block of int4 at four blocks, 59 of signs, against 50 and 47
-// of the MFMAs alone; one int4 query, 35.7 us, is bound by memory.)
+// (73 ns per 16 x 16 block of int4 at four blocks, 59 of signs, against 50 and 47
+// of the MFMAs alone; one int4 query, 35.8 us, is bound by memory.)
 //
 // Work split: the waves of a workgroup (group_waves) share one pass of
 // query rows; its digits are staged once in LDS and held in registers (NT
